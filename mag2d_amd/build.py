@@ -147,7 +147,7 @@ def build_oracle(verbose: bool = False) -> None:
     reference sources exist in this container."""
     _run(["make", "-B", "-C", str(ROOT / "oracle"), "-s", "all"])
     _write_stamp("oracle")
-    if REFERENCE.exists():
+    if (REFERENCE / "src" / "Field2D.hpp").exists():
         _run(["make", "-C", str(ROOT / "oracle"), "-s", "ref", f"REF={REFERENCE}"])
     if verbose:
         print("built oracle")
