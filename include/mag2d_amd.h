@@ -190,7 +190,9 @@ typedef struct {
 enum { M2D_FIELD_U = 0, M2D_FIELD_URF = 1, M2D_FIELD_RHO = 2, M2D_FIELD_VOLTAGE = 3 };
 
 /* Fields::Fields (fields.cpp:115-276): uploads mask and voltage, builds the
- * multigrid hierarchy that replaces the UMFPACK factorisation.  Grids need
+ * multigrid hierarchy that replaces the UMFPACK factorisation (or, when the
+ * free nodes fill one rectangle of at most 1024 a side, the sine matrices of
+ * a direct solve).  Grids need
  * nx, nz >= 3 and (nx+1) (nz+1) < 2^30 (M2D_ERR_BAD_ARG otherwise). */
 int m2d_fields2d_create(m2d_ctx *ctx, const m2d_fields2d_params *p, const uint8_t *mask,
                         const double *voltage, m2d_fields2d **out);
@@ -217,7 +219,7 @@ int m2d_fields2d_reset(m2d_fields2d *f);
 enum { M2D_SOLVE_STATIC = 0, M2D_SOLVE_RF = 1, M2D_SOLVE_RAW = 2 };
 typedef struct {
     int32_t outer_iters;      /* FP64 refinement steps */
-    int32_t inner_iters;      /* FP32 MG-PCG iterations in total */
+    int32_t inner_iters;      /* FP32 MG-PCG iterations in total (a direct solve: one per step) */
     double rel_residual;      /* ||b - A u||_2 / ||b_eff||_2 in FP64 over free nodes */
 } m2d_solve_info;
 /* Fields::boundary_solve (STATIC -> u, fields.cpp:278-312), boundary_solve_rf

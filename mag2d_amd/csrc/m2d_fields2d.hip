@@ -21,41 +21,37 @@ namespace m2d {
 // ------------------------------------------------------------------ tables
 // Edge gradients of u and uRF, padded so Field2D::grad's first/last-row
 // fallbacks (Field2D.hpp:106-124,148-166) are the bilinear formula itself.
-__global__ void k_build_gx(const double *u, const double *urf, int nx, int nz, double idx,
-                           float2 *gx)
+// Both tables in one launch (one dispatch fewer a solve, about 2.5 us):
+// thread (j, i) of the (nx+1) x (nz+1) edges writes gx's row i and gz's
+// column j.
+__global__ void k_build_tables(const double *u, const double *urf, int nx, int nz, double idx, double idz,
+                               float2 *gx, float2 *gz)
 {
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    int e = blockIdx.y;  // 0..nx
-    if (j >= nz || e > nx) return;
-    int ee = e < 1 ? 1 : (e > nx - 1 ? nx - 1 : e);
-    size_t k1 = (size_t)ee * nz + j, k0 = k1 - nz;
-    float2 v;
-    v.x = (float)((u[k1] - u[k0]) * idx);
-    v.y = (float)((urf[k1] - urf[k0]) * idx);
-    gx[(size_t)e * nz + j] = v;
-}
-
-__global__ void k_build_gz(const double *u, const double *urf, int nx, int nz, double idz,
-                           float2 *gz)
-{
-    int e = blockIdx.x * blockDim.x + threadIdx.x;  // 0..nz
-    int i = blockIdx.y;
-    if (e > nz || i >= nx) return;
-    int ee = e < 1 ? 1 : (e > nz - 1 ? nz - 1 : e);
-    size_t k1 = (size_t)i * nz + ee, k0 = k1 - 1;
-    float2 v;
-    v.x = (float)((u[k1] - u[k0]) * idz);
-    v.y = (float)((urf[k1] - urf[k0]) * idz);
-    gz[(size_t)i * (nz + 1) + e] = v;
+    const int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
+    if (j < nz) {
+        const int e = i < 1 ? 1 : (i > nx - 1 ? nx - 1 : i);
+        const size_t k1 = (size_t)e * nz + j, k0 = k1 - nz;
+        float2 v;
+        v.x = (float)((u[k1] - u[k0]) * idx);
+        v.y = (float)((urf[k1] - urf[k0]) * idx);
+        gx[(size_t)i * nz + j] = v;
+    }
+    if (j <= nz && i < nx) {
+        const int e = j < 1 ? 1 : (j > nz - 1 ? nz - 1 : j);
+        const size_t k1 = (size_t)i * nz + e, k0 = k1 - 1;
+        float2 v;
+        v.x = (float)((u[k1] - u[k0]) * idz);
+        v.y = (float)((urf[k1] - urf[k0]) * idz);
+        gz[(size_t)i * (nz + 1) + j] = v;
+    }
 }
 
 int fields_build_tables(m2d_fields2d *f)
 {
     hipStream_t s = f->ctx->stream;
-    dim3 b(256);
     f->ph_valid = false;
-    k_build_gx<<<dim3((f->nz + 255) / 256, f->nx + 1), b, 0, s>>>(f->u, f->urf, f->nx, f->nz, f->idx, f->gx);
-    k_build_gz<<<dim3((f->nz + 1 + 255) / 256, f->nx), b, 0, s>>>(f->u, f->urf, f->nx, f->nz, f->idz, f->gz);
+    k_build_tables<<<dim3((f->nz + 1 + 255) / 256, f->nx + 1), 256, 0, s>>>(f->u, f->urf, f->nx, f->nz, f->idx,
+                                                                           f->idz, f->gx, f->gz);
     M2D_HIP(hipGetLastError());
     return M2D_OK;
 }
@@ -63,50 +59,31 @@ int fields_build_tables(m2d_fields2d *f)
 // ------------------------------------------------------------------ FP64 kernels
 __device__ __forceinline__ bool is_dir(uint8_t m) { return m == M2D_FIXED || m == M2D_FIXED_RF; }
 
-// rhs in place (fields.cpp:297-310, 333-346), Dirichlet values into u.
-// The node bodies below are shared by the grid kernels and the
-// single-workgroup solve, so both paths compute each node the same way.
-__device__ __forceinline__ void node_rhs(const uint8_t *mask, const double *voltage, double *rho, double *u,
-                                         size_t k, int mode, double scale)
+// rhs (fields.cpp:297-310, 333-346) of node k: the voltage on Dirichlet
+// nodes, which is also u there
+__device__ __forceinline__ double rhs_at(uint8_t m, const double *voltage, const double *rho, size_t k, int mode,
+                                         double scale)
 {
-    uint8_t m = mask[k];
-    double b;
-    if (mode == M2D_SOLVE_RAW) b = rho[k];
-    else if (m == M2D_FIXED) b = mode == M2D_SOLVE_STATIC ? voltage[k] : 0.0;
-    else if (m == M2D_FIXED_RF) b = mode == M2D_SOLVE_RF ? voltage[k] : 0.0;
-    else b = rho[k] * scale;
-    rho[k] = b;
-    if (is_dir(m)) u[k] = b;
+    if (mode == M2D_SOLVE_RAW) return rho[k];
+    if (m == M2D_FIXED) return mode == M2D_SOLVE_STATIC ? voltage[k] : 0.0;
+    if (m == M2D_FIXED_RF) return mode == M2D_SOLVE_RF ? voltage[k] : 0.0;
+    return rho[k] * scale;
 }
 
-__global__ void k_rhs(const uint8_t *mask, const double *voltage, double *rho, double *u, size_t n,
-                      int mode, double scale)
+// r = b - A u at a free node from u there and at its neighbours (m: their
+// masks, order -x, -z, +z, +x), rr = r^2 and bb = b_eff^2 (b with the
+// Dirichlet neighbours moved to the right-hand side)
+__device__ __forceinline__ double resid_row(double b, double uc, const double (&un)[4], const uint8_t (&m)[4],
+                                            double &bb)
 {
-    size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) node_rhs(mask, voltage, rho, u, k, mode, scale);
-}
-
-// r = b - A u at node k (0 on Dirichlet nodes), d = -r in FP32; rr = r^2 and
-// bb = b_eff^2 (b with the Dirichlet neighbours moved to the right-hand side)
-__device__ __forceinline__ void node_residual64(const uint8_t *mask, const double *b, const double *u, int nz,
-                                                double *r, float *d, size_t k, double &rr, double &bb)
-{
-    double rv = 0;
-    bb = 0;
-    if (!is_dir(mask[k])) {
-        // free rows never sit on the frame (checked at creation)
-        double au = u[k - nz] + u[k - 1] - 4.0 * u[k] + u[k + 1] + u[k + nz];
-        rv = b[k] - au;
-        double be = b[k];
-        if (is_dir(mask[k - nz])) be -= u[k - nz];
-        if (is_dir(mask[k - 1])) be -= u[k - 1];
-        if (is_dir(mask[k + 1])) be -= u[k + 1];
-        if (is_dir(mask[k + nz])) be -= u[k + nz];
-        bb = be * be;
-    }
-    r[k] = rv;
-    d[k] = (float)(-rv);
-    rr = rv * rv;
+    const double au = un[0] + un[1] - 4.0 * uc + un[2] + un[3];
+    double be = b;
+    if (is_dir(m[0])) be -= un[0];
+    if (is_dir(m[1])) be -= un[1];
+    if (is_dir(m[2])) be -= un[2];
+    if (is_dir(m[3])) be -= un[3];
+    bb = be * be;
+    return b - au;
 }
 
 // u += e on free nodes
@@ -378,19 +355,51 @@ __global__ void __launch_bounds__(kRedBlock) k_cg_update_dot(float *e, float *r,
     finish_sums<1>(v, partial, ticket, out, fin, post);
 }
 
-// the FP64 residual with its norms finished in the same launch: out[0] =
-// |r|^2, out[1] = |b_eff|^2, out[2] = |d|^2 of the FP32 copy d = -r
-__global__ void __launch_bounds__(kRedBlock) k_residual64_fin(const uint8_t *mask, const double *b, const double *u,
-                                                             size_t n, int nz, double *r, float *d, double *partial,
+// The FP64 residual r = b - A u (0 on Dirichlet nodes) and its FP32 copy
+// d = -r, with the norms finished in the same launch: out[0] = |r|^2, out[1]
+// = |b_eff|^2, out[2] = |d|^2.  FIRST: the solve's first residual, which
+// forms the right-hand side in place on rho and sets u on the Dirichlet
+// nodes on the way (a neighbour's Dirichlet value is formed again rather
+// than read, since its own thread may not have written it yet): the
+// right-hand side needs no launch of its own.
+template <bool FIRST, class Post>
+__global__ void __launch_bounds__(kRedBlock) k_residual64_fin(const uint8_t *mask, const double *voltage, double *rho,
+                                                             double *u, int mode, double scale, size_t n, int nz,
+                                                             double *r, float *d, double *partial,
                                                              unsigned int *ticket, double *out, int fin,
-                                                             const int *stop, CtlEval post)
+                                                             const int *stop, Post post)
 {
-    if (stopped(stop)) return;
+    if (!FIRST && stopped(stop)) return;
     double v[3] = {0, 0, 0};
     const size_t k = (size_t)blockIdx.x * kRedBlock + threadIdx.x;
     if (k < n) {
-        node_residual64(mask, b, u, nz, r, d, k, v[0], v[1]);
-        v[2] = (double)d[k] * d[k];
+        const uint8_t mk = mask[k];
+        double b;
+        if constexpr (FIRST) {
+            b = rhs_at(mk, voltage, rho, k, mode, scale);
+            rho[k] = b;
+            if (is_dir(mk)) u[k] = b;
+        } else {
+            b = rho[k];
+        }
+        double rv = 0;
+        if (!is_dir(mk)) {
+            // free rows never sit on the frame (checked at creation)
+            const size_t at[4] = {k - nz, k - 1, k + 1, k + nz};
+            uint8_t m[4];
+            double un[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                m[q] = mask[at[q]];
+                un[q] = FIRST && is_dir(m[q]) ? rhs_at(m[q], voltage, rho, at[q], mode, scale) : u[at[q]];
+            }
+            rv = resid_row(b, u[k], un, m, v[1]);
+        }
+        r[k] = rv;
+        const float dk = (float)(-rv);
+        d[k] = dk;
+        v[0] = rv * rv;
+        v[2] = (double)dk * dk;
     }
     finish_sums<3>(v, partial, ticket, out, fin, post);
 }
@@ -1056,6 +1065,24 @@ static int dmalloc(void **p, size_t bytes)
     return M2D_OK;
 }
 
+// what every solve keeps: the residual, the dot products and the control block
+static int solve_setup(m2d_fields2d *f)
+{
+    Mg &mg = f->mg;
+    const size_t n = f->n;
+    M2D_TRY(dmalloc((void **)&mg.pr, sizeof(float) * n));
+    M2D_TRY(dmalloc((void **)&mg.r64, sizeof(double) * n));
+    // 16 device scalars, then the solve's control block (SolveCtl)
+    M2D_TRY(dmalloc((void **)&mg.dots, sizeof(double) * 32));
+    M2D_TRY(dmalloc((void **)&mg.ticket, sizeof(unsigned int)));
+    M2D_HIP(hipMemset(mg.ticket, 0, sizeof(unsigned int)));
+    M2D_HIP(hipHostMalloc((void **)&mg.h_dots, sizeof(double) * 32));
+    mg.npartial = (int)std::min<size_t>((n + 255) / 256, 65536);
+    // up to three sums per block of the fused reductions
+    M2D_TRY(dmalloc((void **)&mg.partial, sizeof(double) * 3 * std::max<size_t>(mg.npartial, (n + 255) / 256)));
+    return M2D_OK;
+}
+
 static int mg_setup(m2d_fields2d *f)
 {
     Mg &mg = f->mg;
@@ -1128,17 +1155,11 @@ static int mg_setup(m2d_fields2d *f)
         M2D_HIP(hipMemcpy(mg.coarse_invT, invT.data(), sizeof(float) * invT.size(), hipMemcpyHostToDevice));
     }
     const size_t n = f->n;
-    M2D_TRY(dmalloc((void **)&mg.pr, sizeof(float) * n));
     M2D_TRY(dmalloc((void **)&mg.pz, sizeof(float) * n));
     M2D_TRY(dmalloc((void **)&mg.pp, sizeof(float) * n));
     M2D_TRY(dmalloc((void **)&mg.pp2, sizeof(float) * n));
     M2D_TRY(dmalloc((void **)&mg.pq, sizeof(float) * n));
     M2D_TRY(dmalloc((void **)&mg.pe, sizeof(float) * n));
-    M2D_TRY(dmalloc((void **)&mg.r64, sizeof(double) * n));
-    // 16 device scalars, then the solve's control block (SolveCtl)
-    M2D_TRY(dmalloc((void **)&mg.dots, sizeof(double) * 32));
-    M2D_TRY(dmalloc((void **)&mg.ticket, sizeof(unsigned int)));
-    M2D_HIP(hipMemset(mg.ticket, 0, sizeof(unsigned int)));
     // the coarse part of the V-cycle runs in one workgroup from the first
     // level of at most kBlockLevelNodes nodes (the dense level at the latest)
     mg.lc = (int)mg.lv.size() - 1;
@@ -1146,10 +1167,6 @@ static int mg_setup(m2d_fields2d *f)
         if (mg.lv[l].n <= kBlockLevelNodes) { mg.lc = l; break; }
     M2D_CHECK(mg.lv.size() <= (size_t)kMaxLevels && mg.coarse_n <= 3200, M2D_ERR_BAD_ARG,
               "Fields: multigrid hierarchy of %d levels, coarsest %d nodes", (int)mg.lv.size(), mg.coarse_n);
-    M2D_HIP(hipHostMalloc((void **)&mg.h_dots, sizeof(double) * 32));
-    mg.npartial = (int)std::min<size_t>((n + 255) / 256, 65536);
-    // up to three sums per block of the fused reductions
-    M2D_TRY(dmalloc((void **)&mg.partial, sizeof(double) * 3 * std::max<size_t>(mg.npartial, (n + 255) / 256)));
     return M2D_OK;
 }
 
@@ -1265,11 +1282,7 @@ static unsigned red_blocks(size_t n) { return (unsigned)((n + kRedBlock - 1) / k
 __global__ void k_ctl_init(SolveCtl *c)
 {
     if (threadIdx.x) return;
-    SolveCtl z{};
-    z.stop_pcg = 1;
-    z.no_add = 1;
-    z.rel = INFINITY;
-    *c = z;
+    ctl_reset(c);
 }
 
 // opens a CG pass on the FP32 residual d (|d|^2 = dots[10])
@@ -1382,9 +1395,48 @@ static void queue_residual(m2d_fields2d *f, double *u, double tol, int max_outer
     const int *stop = &ctl->stop_outer;
     const CtlEval post{ctl, tol, max_outer};
     reduce_launch<3>(rb, mg.partial, mg.dots + 8, s, [&](int fin) {
-        k_residual64_fin<<<rb, kRedBlock, 0, s>>>(f->mask, f->rho, u, n, f->nz, mg.r64, mg.pr, mg.partial, mg.ticket,
-                                                  mg.dots + 8, fin, stop, post);
+        k_residual64_fin<false><<<rb, kRedBlock, 0, s>>>(f->mask, f->voltage, f->rho, u, 0, 0.0, n, f->nz, mg.r64,
+                                                         mg.pr, mg.partial, mg.ticket, mg.dots + 8, fin, stop, post);
     }, stop, post);
+}
+
+// the solve's first residual: the right-hand side, the Dirichlet values of u
+// and a fresh control block with it
+static void queue_first_residual(m2d_fields2d *f, double *u, int mode, double scale, double tol, int max_outer)
+{
+    Mg &mg = f->mg;
+    hipStream_t s = f->ctx->stream;
+    const size_t n = f->n;
+    const unsigned rb = red_blocks(n);
+    const CtlFirst post{{solve_ctl(mg), tol, max_outer}};
+    reduce_launch<3>(rb, mg.partial, mg.dots + 8, s, [&](int fin) {
+        k_residual64_fin<true><<<rb, kRedBlock, 0, s>>>(f->mask, f->voltage, f->rho, u, mode, scale, n, f->nz, mg.r64,
+                                                        mg.pr, mg.partial, mg.ticket, mg.dots + 8, fin, nullptr,
+                                                        post);
+    }, nullptr, post);
+}
+
+// FP64 refinement whose every pass is the direct solve of its residual: one
+// pass meets any tolerance FP64 can hold on most grids, and as many as the
+// last solve took are queued before the host reads the control block
+static int refine_direct(m2d_fields2d *f, double *u, double tol)
+{
+    Mg &mg = f->mg;
+    hipStream_t s = f->ctx->stream;
+    SolveCtl *ctl = solve_ctl(mg), *h = (SolveCtl *)(mg.h_dots + 16);
+    int J = mg.est.passes < 1 ? 1 : (mg.est.passes > kMaxOuter ? kMaxOuter : mg.est.passes);
+    for (int round = 0; round <= kMaxOuter; round++, J = 1) {
+        for (int j = 0; j < J; j++) {
+            M2D_TRY(direct2d_pass(f, u, ctl));
+            queue_residual(f, u, tol, kMaxOuter);
+        }
+        M2D_HIP(hipGetLastError());
+        M2D_HIP(hipMemcpyAsync(h, ctl, sizeof(SolveCtl), hipMemcpyDeviceToHost, s));
+        M2D_HIP(hipStreamSynchronize(s));
+        if (h->nan || h->stop_outer) break;
+    }
+    mg.est.passes = h->outer > 1 ? h->outer : 1;
+    return M2D_OK;
 }
 
 // FP64 iterative refinement of u over FP32 multigrid-preconditioned CG
@@ -1400,13 +1452,15 @@ static int solve(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info)
     if (tol <= 0) tol = 1e-10;
     SolveCtl *ctl = solve_ctl(mg);
     SolveCtl *h = (SolveCtl *)(mg.h_dots + 16);
-    k_rhs<<<gb, 256, 0, s>>>(f->mask, f->voltage, f->rho, u, n, mode, scale);
-    k_ctl_init<<<1, 64, 0, s>>>(ctl);
-    queue_residual(f, u, tol, kMaxOuter);
-    M2D_TRY(queue_refinement(
-        s, ctl, h, mg.dots, mg.est, tol, 60, [&](int from, int to, int &cur) { return queue_pcg(f, from, to, cur); },
-        [&] { k_add_correction<<<gb, 256, 0, s>>>(f->mask, u, mg.pe, n, &ctl->no_add); },
-        [&] { queue_residual(f, u, tol, kMaxOuter); }));
+    queue_first_residual(f, u, mode, scale, tol, kMaxOuter);
+    if (f->direct.on)
+        M2D_TRY(refine_direct(f, u, tol));
+    else
+        M2D_TRY(queue_refinement(
+            s, ctl, h, mg.dots, mg.est, tol, 60,
+            [&](int from, int to, int &cur) { return queue_pcg(f, from, to, cur); },
+            [&] { k_add_correction<<<gb, 256, 0, s>>>(f->mask, u, mg.pe, n, &ctl->no_add); },
+            [&] { queue_residual(f, u, tol, kMaxOuter); }));
     if (info) { info->outer_iters = h->outer; info->inner_iters = h->iters; info->rel_residual = h->rel; }
     if (h->nan) return set_error(M2D_ERR_NAN, "Fields solve: residual is not finite");
     M2D_TRY(fields_build_tables(f));
@@ -1496,7 +1550,9 @@ int m2d_fields2d_create(m2d_ctx *ctx, const m2d_fields2d_params *p, const uint8_
     if ((r = fill_bytes(ctx, f->u, 0, 8 * n)) || (r = fill_bytes(ctx, f->urf, 0, 8 * n)) ||
         (r = fill_bytes(ctx, f->rho, 0, 8 * n)))
         return fail(r);
-    if ((r = mg_setup(f))) return fail(r);
+    // a rectangle of free nodes is solved directly, anything else by multigrid-PCG
+    f->direct.on = direct2d_fits(f->h_mask, f->nx, f->nz, f->direct);
+    if ((r = solve_setup(f)) || (r = f->direct.on ? direct2d_setup(f) : mg_setup(f))) return fail(r);
     if ((r = fields_build_tables(f))) return fail(r);
     if (hipStreamSynchronize(ctx->stream) != hipSuccess)
         return fail(set_error(M2D_ERR_HIP, "m2d_fields2d_create: synchronise failed"));
@@ -1510,7 +1566,7 @@ int m2d_fields2d_destroy(m2d_fields2d *f)
     if (f->ctx) (void)hipStreamSynchronize(f->ctx->stream);
     for (void *p : {(void *)f->mask, (void *)f->cellfree, (void *)f->winfree, (void *)f->voltage, (void *)f->u,
                     (void *)f->urf, (void *)f->rho, (void *)f->gx, (void *)f->gz, (void *)f->phx, (void *)f->phz, (void *)f->bt,
-                    (void *)f->smooth_tmp})
+                    (void *)f->smooth_tmp, (void *)f->direct.buf})
         if (p) (void)hipFree(p);
     mg_free(f->mg);
     if (f->ctx) ctx_release(f->ctx);

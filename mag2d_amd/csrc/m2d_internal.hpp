@@ -271,6 +271,24 @@ struct CtlEval {
         }
     }
 };
+// a fresh control block: no pass open, nothing to add
+__device__ __forceinline__ void ctl_reset(SolveCtl *c)
+{
+    SolveCtl z{};
+    z.stop_pcg = 1;
+    z.no_add = 1;
+    z.rel = INFINITY;
+    *c = z;
+}
+// CtlEval of a solve's first residual, which no launch of the solve precedes
+struct CtlFirst {
+    CtlEval eval;
+    __device__ void operator()(const double *out) const
+    {
+        ctl_reset(eval.c);
+        eval(out);
+    }
+};
 struct CtlCheck {
     SolveCtl *c;
     __device__ void operator()(const double *out) const

@@ -73,6 +73,17 @@ struct Mg {
     SolveEst est;  // the last solve's passes and iterations: what the next queues
 };
 
+// ------------------------------------------------------------------ direct solve
+// The sine-basis solve of fields whose free nodes fill the rectangle
+// [i0, i0 + m) x [j0, j0 + n) (m2d_direct2d.hip); M, N: m, n padded
+constexpr int kDstPad = 32;
+struct Direct2 {
+    bool on = false;
+    int i0 = 0, j0 = 0, m = 0, n = 0, M = 0, N = 0;
+    double *buf = nullptr;        // one allocation behind the pointers below
+    double *sm = nullptr, *sn = nullptr, *lm = nullptr, *ln = nullptr, *t0 = nullptr, *t1 = nullptr;
+};
+
 }  // namespace m2d
 
 struct m2d_fields2d {
@@ -101,6 +112,7 @@ struct m2d_fields2d {
     m2d_grid2d bgrid{};
     double *smooth_tmp = nullptr;  // nx*nz copy of the field u_smooth filters
     m2d::Mg mg;
+    m2d::Direct2 direct;          // on: the solve is direct, and mg holds no levels
     std::vector<uint8_t> h_mask;
 };
 
@@ -114,6 +126,9 @@ struct m2d_mcc {
 
 namespace m2d {
 int fields_build_tables(m2d_fields2d *f);
+bool direct2d_fits(const std::vector<uint8_t> &mask, int nx, int nz, Direct2 &d);
+int direct2d_setup(m2d_fields2d *f);
+int direct2d_pass(m2d_fields2d *f, double *u, SolveCtl *ctl);
 int mcc_sync(m2d_mcc *m);
 // some target draws its partners from the store whose first position array
 // is x (the colliding species itself)
