@@ -5,9 +5,10 @@
 // Solver: FP64 iterative refinement around FP32 conjugate gradients on the
 // Dirichlet-eliminated SPD system 6u - sum_free u_nb = ..., preconditioned by
 // one symmetric geometric multigrid V-cycle: coarse node I sits on fine node
-// 2I, every level carries the 7-point operator of its own mask, restriction
-// is P^T / 2 (full weighting with the h^2 of the coarser spacing), red-black
-// Gauss-Seidel smooths, and the coarsest level is solved by a dense inverse.
+// 2I, every level carries a 7-point operator of its own (mg3_setup),
+// restriction is P^T / 2 (full weighting with the h^2 of the coarser
+// spacing), one red-black Gauss-Seidel sweep smooths on either side, and the
+// coarsest level is solved by a dense inverse.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -21,9 +22,10 @@ namespace m2d {
 struct Mg3Level {
     int nx = 0, ny = 0, nz = 0;
     size_t n = 0;
-    uint8_t *dir = nullptr;   // 1 on Dirichlet nodes (and the coarse faces)
-    uint8_t *nbm = nullptr;   // per node: bits 0-5 set for free neighbours -x,-y,-z,+z,+y,+x; 0x80 if pinned
-    float *x = nullptr, *b = nullptr, *r = nullptr;
+    uint8_t *nbm = nullptr;   // per node: bits 0-5 set for links to free neighbours -x,-y,-z,+z,+y,+x;
+                              // 0x40: colour (i+j+k) & 1; 0x80: pinned
+    float *di = nullptr;      // inverse diagonal (level 0: 1/6, no array)
+    float *x = nullptr, *b = nullptr;  // not on level 0
 };
 
 }  // namespace m2d
@@ -39,14 +41,11 @@ struct m2d_fields3d {
     double *voltage = nullptr, *u = nullptr, *rho = nullptr;
     float *tx = nullptr, *ty = nullptr, *tz = nullptr;  // (u_m - u_{m-e}) * 1/h per axis, FP32
     std::vector<m2d::Mg3Level> lv;
-    float *coarse_inv = nullptr;
-    float *coarse_invT = nullptr;  // the same, transposed (read by k_dense_solve)
-    unsigned int *ticket = nullptr;  // block counter of the fused reductions
-    int coarse_n = 0;
+    float *coarse_inv = nullptr;   // inverse of the coarsest operator over all its nodes (symmetric)
     bool coarse_dense = true;
-    int lc3 = 1;                   // first level of the one-workgroup coarse V-cycle
+    unsigned int *ticket = nullptr;  // block counter of the fused reductions
     float *pr = nullptr, *pz = nullptr, *pp = nullptr, *pp2 = nullptr, *pq = nullptr, *pe = nullptr;
-    double *r64 = nullptr, *dots = nullptr, *h_dots = nullptr, *partial = nullptr;
+    double *dots = nullptr, *h_dots = nullptr, *partial = nullptr;
     int npartial = 0;
     m2d::SolveEst est;  // the last solve's passes and iterations: what the next queues
 };
@@ -64,33 +63,20 @@ __device__ __forceinline__ void node3(size_t m, int ny, int nz, int &i, int &j, 
 }
 
 // ------------------------------------------------------------------ tables and solve kernels
-__global__ void k3_tables(const double *u, int nx, int ny, int nz, double idx, double idy, double idz,
-                          float *tx, float *ty, float *tz)
+// blocks of 64 x 4 nodes (k, j) and a grid of (nz / 64, ny / 4, nx)
+__global__ void __launch_bounds__(256) k3_tables(const double *u, int nx, int ny, int nz, double idx, double idy,
+                                                 double idz, float *tx, float *ty, float *tz)
 {
-    const size_t n = (size_t)nx * ny * nz;
-    size_t m = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= n) return;
-    int i, j, k;
-    node3(m, ny, nz, i, j, k);
-    const size_t sx = (size_t)ny * nz;
-    tx[m] = i >= 1 ? (float)((u[m] - u[m - sx]) * idx) : 0.f;
-    ty[m] = j >= 1 ? (float)((u[m] - u[m - nz]) * idy) : 0.f;
-    tz[m] = k >= 1 ? (float)((u[m] - u[m - 1]) * idz) : 0.f;
+    const int i = blockIdx.z, j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.x * 64 + threadIdx.x;
+    if (j >= ny || k >= nz) return;
+    const size_t m = ((size_t)i * ny + j) * nz + k, sx = (size_t)ny * nz;
+    const double c = u[m], ux = u[i >= 1 ? m - sx : m], uy = u[j >= 1 ? m - nz : m], uz = u[k >= 1 ? m - 1 : m];
+    tx[m] = (float)((c - ux) * idx);
+    ty[m] = (float)((c - uy) * idy);
+    tz[m] = (float)((c - uz) * idz);
 }
 
-// Solver::solve rows (fields3d.cpp:86-93); Dirichlet values into u
-__global__ void k3_rhs(const uint8_t *mask, const double *voltage, double *rho, double *u, size_t n,
-                       double scale)
-{
-    size_t m = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= n) return;
-    const bool d = dir3(mask[m]);
-    const double b = d ? voltage[m] : rho[m] * -scale;
-    rho[m] = b;
-    if (d) u[m] = b;
-}
-
-// r = b - A u on free rows (matrix_init, fields3d.cpp:35-76); d = -r in FP32;
+// u += e on free nodes
 __global__ void k3_add_correction(const uint8_t *mask, double *u, const float *e, size_t n, const int *stop)
 {
     if (stopped(stop)) return;
@@ -98,525 +84,506 @@ __global__ void k3_add_correction(const uint8_t *mask, double *u, const float *e
     if (m < n && !dir3(mask[m])) u[m] += (double)e[m];
 }
 
-// r = b - A u on free nodes (0 on Dirichlet nodes) with its norms finished in
-// the same launch: out[0] = |r|^2, out[1] = |b_eff|^2, out[2] = |d|^2, d = -r in FP32
-__global__ void __launch_bounds__(kRedBlock) k3_residual64_fin(const uint8_t *mask, const double *b, const double *u,
-                                                              int nx, int ny, int nz, double *r, float *d,
-                                                              double *partial, unsigned int *ticket, double *out,
-                                                              int fin, const int *stop, CtlEval post)
-{
-    if (stopped(stop)) return;
-    const size_t n = (size_t)nx * ny * nz, sx = (size_t)ny * nz;
-    double v[3] = {0, 0, 0};
-    for (size_t m = (size_t)blockIdx.x * kRedBlock + threadIdx.x; m < n; m += (size_t)gridDim.x * kRedBlock) {
-        double rv = 0;
-        if (!dir3(mask[m])) {
-            // free rows never touch the grid faces (checked at creation)
-            const size_t nb[6] = {m - sx, m - nz, m - 1, m + 1, m + nz, m + sx};
-            double au = -6.0 * u[m], be = b[m];
+// ---- the finest level's stencils outside the V-cycle.  A block of 64 x 4
+// threads (k, j) takes DI planes of i: a thread reads its column of nodes and
+// the two columns beside it along j whole, before it stores anything (the
+// arrays do not alias), and gets the neighbours along k from the lanes beside
+// it.  A node then costs 3 reads and a bit instead of 7, all in flight
+// together.  DI is 8 where that fills the GPU, 4 on smaller grids.
+constexpr int kMarchK = 64, kMarchJ = 4;
+struct Cols3 {
+    int nx, ny, nz;
+    int di() const { return (size_t)nx * ny * nz >= (1 << 20) ? 8 : 4; }
+    dim3 grid() const
+    {
+        return dim3((unsigned)((nz + kMarchK - 1) / kMarchK), (unsigned)((ny + kMarchJ - 1) / kMarchJ),
+                    (unsigned)((nx + di() - 1) / di()));
+    }
+    unsigned blocks() const
+    {
+        const dim3 g = grid();
+        return g.x * g.y * g.z;
+    }
+};
+
+// the thread's column: j, k (clamped onto the grid), whether it is inside
+struct Column3 {
+    bool in;
+    int lane, k;
+    size_t col, up, dn;  // offsets in a plane: its node, j - 1, j + 1 (clamped: never a free node's)
+    __device__ explicit Column3(const Cols3 &g)
+    {
+        lane = threadIdx.x & 63;
+        const int jj = blockIdx.y * kMarchJ + (threadIdx.x >> 6), kk = blockIdx.x * kMarchK + lane;
+        in = jj < g.ny && kk < g.nz;
+        const int j = min(jj, g.ny - 1);
+        k = min(kk, g.nz - 1);
+        col = (size_t)j * g.nz + k;
+        up = col - (j > 0 ? g.nz : 0);
+        dn = col + (j < g.ny - 1 ? g.nz : 0);
+    }
+};
+
+// DI + 2 planes of the column from plane i0 - 1 on and DI of each column
+// beside it (planes clamped onto the grid, as no free node lies on a face),
+// and what the first and the last lane have beside them along k
+template <class T, int DI>
+struct Reach3 {
+    T c[DI + 2], up[DI], dn[DI], edge[DI];
+    template <class F>
+    __device__ __forceinline__ void read(const Column3 &C, const Cols3 &g, int i0, F at)
+    {
+        const size_t sx = (size_t)g.ny * g.nz;
+        const size_t e = C.lane == 0 ? (C.k > 0 ? C.col - 1 : C.col) : (C.k < g.nz - 1 ? C.col + 1 : C.col);
 #pragma unroll
-            for (int q = 0; q < 6; q++) {
-                au += u[nb[q]];
-                if (dir3(mask[nb[q]])) be -= u[nb[q]];
-            }
-            rv = b[m] - au;
-            v[1] += be * be;
+        for (int t = 0; t < DI + 2; t++) c[t] = at((size_t)min(max(i0 - 1 + t, 0), g.nx - 1) * sx + C.col);
+#pragma unroll
+        for (int t = 0; t < DI; t++) {
+            const size_t base = (size_t)min(i0 + t, g.nx - 1) * sx;
+            up[t] = at(base + C.up);
+            dn[t] = at(base + C.dn);
+            if (C.lane == 0 || C.lane == 63) edge[t] = at(base + e);
         }
-        r[m] = rv;
-        const float dm = (float)(-rv);
-        d[m] = dm;
-        v[0] += rv * rv;
-        v[2] += (double)dm * dm;
+    }
+    __device__ __forceinline__ T left(const Column3 &C, int t) const
+    {
+        const T v = __shfl_up(c[t + 1], 1);
+        return C.lane == 0 ? edge[t] : v;
+    }
+    __device__ __forceinline__ T right(const Column3 &C, int t) const
+    {
+        const T v = __shfl_down(c[t + 1], 1);
+        return C.lane == 63 ? edge[t] : v;
+    }
+};
+
+// The FP64 residual b - A u of the free rows (matrix_init, fields3d.cpp:35-76),
+// its negative d in FP32 (0 on Dirichlet nodes), and its norms finished in the
+// same launch: out[0] = |r|^2, out[1] = |b_eff|^2 (b with the Dirichlet
+// neighbours moved to the right-hand side), out[2] = |d|^2.
+template <int DI, class Post>
+__global__ void __launch_bounds__(kRedBlock) k3_residual64_fin(Cols3 g, const uint8_t *__restrict__ mask,
+                                                              const double *__restrict__ b,
+                                                              const double *__restrict__ u, float *__restrict__ d,
+                                                              double *partial, unsigned int *ticket, double *out,
+                                                              int fin, const int *stop, Post post)
+{
+    const int stopped_ = stop ? *stop : 0;  // read beside the operands
+    const Column3 C(g);
+    const int i0 = blockIdx.z * DI;
+    const size_t sx = (size_t)g.ny * g.nz;
+    Reach3<double, DI> U;
+    Reach3<int, DI> P;
+    double bv[DI];
+    P.read(C, g, i0, [&](size_t m) { return (int)dir3(mask[m]); });
+    U.read(C, g, i0, [&](size_t m) { return u[m]; });
+#pragma unroll
+    for (int t = 0; t < DI; t++) bv[t] = b[(size_t)min(i0 + t, g.nx - 1) * sx + C.col];
+    if (stopped_) return;
+    double v[3] = {0, 0, 0};
+#pragma unroll
+    for (int t = 0; t < DI; t++) {
+        const double ul = U.left(C, t), ur = U.right(C, t);
+        const int pl = P.left(C, t), pr = P.right(C, t);
+        if (!C.in || i0 + t >= g.nx) continue;
+        float dm = 0.f;
+        if (!P.c[t + 1]) {
+            double au = -6.0 * U.c[t + 1];
+            au += U.c[t]; au += U.up[t]; au += ul; au += ur; au += U.dn[t]; au += U.c[t + 2];
+            double be = bv[t];
+            if (P.c[t]) be -= U.c[t];
+            if (P.up[t]) be -= U.up[t];
+            if (pl) be -= ul;
+            if (pr) be -= ur;
+            if (P.dn[t]) be -= U.dn[t];
+            if (P.c[t + 2]) be -= U.c[t + 2];
+            const double r = bv[t] - au;
+            dm = (float)(-r);
+            v[0] += r * r;
+            v[1] += be * be;
+            v[2] += (double)dm * dm;
+        }
+        d[(size_t)(i0 + t) * sx + C.col] = dm;
     }
     finish_sums<3>(v, partial, ticket, out, fin, post);
 }
 
-// Neighbour masks of the 7-point levels: one byte per node replaces the
-// seven Dirichlet flags a stencil update reads.  Bits 0-5: neighbours
-// -x, -y, -z, +z, +y, +x free; kNbSelf: the node itself is pinned.
-constexpr uint8_t kNbSelf = 0x80;
-
-// A' x = 6 x - sum over free neighbours (Dirichlet rows: 0)
-__device__ __forceinline__ float apply7(uint8_t nb, const float *x, size_t m, size_t sx, int nz)
+// Solver::solve rows (fields3d.cpp:86-93); Dirichlet values into u
+__global__ void k3_rhs(const uint8_t *__restrict__ mask, const double *__restrict__ voltage, double *rho, double *u,
+                       size_t n, double scale)
 {
-    float s = 6.f * x[m];
-    if (nb & 1) s -= x[m - sx];
-    if (nb & 2) s -= x[m - nz];
-    if (nb & 4) s -= x[m - 1];
-    if (nb & 8) s -= x[m + 1];
-    if (nb & 16) s -= x[m + nz];
-    if (nb & 32) s -= x[m + sx];
-    return s;
+    size_t m = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (m >= n) return;
+    const double r = rho[m];
+    const bool d = dir3(mask[m]);
+    const double b = d ? voltage[m] : r * -scale;
+    rho[m] = b;
+    if (d) u[m] = b;
 }
 
+// Neighbour masks of the 7-point levels: one byte per node replaces the
+// seven Dirichlet flags a stencil update reads.  Bits 0-5: linked to the
+// free neighbour -x, -y, -z, +z, +y, +x; kNbBlack: colour 1 of the
+// red-black order; kNbSelf: the node itself is pinned.
+constexpr uint8_t kNbSelf = 0x80, kNbBlack = 0x40;
+
 // The CG direction and the operator in one launch: p' = z + beta p (first:
-// p' = z), q = A' p' and out = p'.q.  Each node's p' is recomputed at its
-// stencil neighbours from z and p (the same operations, so the same bits) and
+// p' = z), q = A' p' = 6 p' - sum over the neighbours (p' is 0 on Dirichlet
+// nodes, as z is; q too) and out = p'.q.  Each node's p' is formed again at
+// its neighbours from z and p (the same operations, so the same bits) and
 // written to pn, not p, which other blocks are still reading.
-__global__ void __launch_bounds__(kRedBlock) k3_dir_apply_dot(const uint8_t *nbm, const float *z, const float *p,
-                                                             float *pn, float *q, const double *rz_new,
-                                                             const double *rz_old, int first, int nx, int ny, int nz,
-                                                             double *partial, unsigned int *ticket, double *out,
-                                                             int fin, const int *stop)
+template <int DI>
+__global__ void __launch_bounds__(kRedBlock) k3_dir_apply_dot(Cols3 g, const uint8_t *__restrict__ nbm,
+                                                             const float *__restrict__ z,
+                                                             const float *__restrict__ p, float *__restrict__ pn,
+                                                             float *__restrict__ q, const double *rz_new,
+                                                             const double *rz_old, int first, double *partial,
+                                                             unsigned int *ticket, double *out, int fin,
+                                                             const int *stop)
 {
-    if (stopped(stop)) return;
-    const size_t n = (size_t)nx * ny * nz, sx = (size_t)ny * nz;
+    const int stopped_ = stop ? *stop : 0;  // read beside the operands
     const float beta = first ? 0.f : cg_beta(rz_new, rz_old);
+    const Column3 C(g);
+    const int i0 = blockIdx.z * DI;
+    const size_t sx = (size_t)g.ny * g.nz;
+    Reach3<float, DI> D;
+    uint8_t nb[DI];
+    if (first) D.read(C, g, i0, [&](size_t m) { return z[m]; });
+    else D.read(C, g, i0, [&](size_t m) { return fmaf(beta, p[m], z[m]); });
+#pragma unroll
+    for (int t = 0; t < DI; t++) nb[t] = nbm[(size_t)min(i0 + t, g.nx - 1) * sx + C.col];
+    if (stopped_) return;
     double v[1] = {0};
-    for (size_t m = (size_t)blockIdx.x * kRedBlock + threadIdx.x; m < n; m += (size_t)gridDim.x * kRedBlock) {
-        const uint8_t nb = nbm[m];
-        const float pk = cg_dir_at(z, p, m, beta, first);
-        pn[m] = pk;
-        float ym = 0.f;
-        if (!(nb & kNbSelf)) {
-            // apply7's order
-            float t = 6.f * pk;
-            if (nb & 1) t -= cg_dir_at(z, p, m - sx, beta, first);
-            if (nb & 2) t -= cg_dir_at(z, p, m - nz, beta, first);
-            if (nb & 4) t -= cg_dir_at(z, p, m - 1, beta, first);
-            if (nb & 8) t -= cg_dir_at(z, p, m + 1, beta, first);
-            if (nb & 16) t -= cg_dir_at(z, p, m + nz, beta, first);
-            if (nb & 32) t -= cg_dir_at(z, p, m + sx, beta, first);
-            ym = t;
-        }
-        q[m] = ym;
-        v[0] += (double)pk * ym;
+#pragma unroll
+    for (int t = 0; t < DI; t++) {
+        const float l = D.left(C, t), r = D.right(C, t), c = D.c[t + 1];
+        if (!C.in || i0 + t >= g.nx) continue;
+        const float y = nb[t] & kNbSelf ? 0.f : 6.f * c - D.c[t] - D.up[t] - l - r - D.dn[t] - D.c[t + 2];
+        const size_t m = (size_t)(i0 + t) * sx + C.col;
+        pn[m] = c;
+        q[m] = y;
+        v[0] += (double)c * y;
     }
     finish_sums<1>(v, partial, ticket, out, fin);
 }
 
-// Gauss-Seidel update of node m (the node bodies here are shared by the grid
-// kernels and the one-workgroup coarse V-cycle)
-__device__ __forceinline__ void node3_rbgs(const uint8_t *nbm, float *x, const float *b, size_t m, size_t sx, int nz)
+// ------------------------------------------------------------------ the V-cycle
+// sum of the free neighbours' values at node m of an array with strides si,
+// sj, 1 (in LDS tiles and in the coarse cycle's arrays)
+template <class T>
+__device__ __forceinline__ float links7(uint8_t nb, const T *x, int m, int si, int sj)
 {
-    const uint8_t nb = nbm[m];
-    if (nb & kNbSelf) return;
-    float s = b[m];
-    if (nb & 1) s += x[m - sx];
-    if (nb & 2) s += x[m - nz];
+    float s = 0.f;
+    if (nb & 1) s += x[m - si];
+    if (nb & 2) s += x[m - sj];
     if (nb & 4) s += x[m - 1];
     if (nb & 8) s += x[m + 1];
-    if (nb & 16) s += x[m + nz];
-    if (nb & 32) s += x[m + sx];
-    x[m] = s * (1.f / 6.f);
+    if (nb & 16) s += x[m + sj];
+    if (nb & 32) s += x[m + si];
+    return s;
 }
 
-// The six neighbours of node (i, j, k) = m, read beside its mask byte: the
-// indices come from the coordinates, not from the mask (a face's missing
-// neighbour reads the node itself, which the mask never selects), so the
-// loads do not wait for the mask.  Order: -x, -y, -z, +z, +y, +x (mask bits
-// 1, 2, 4, 8, 16, 32).
-struct Nb7 {
-    float v[6];
+// Smoothing is one red-black sweep down and one (in reverse) up, which lets
+// each side of a level be one launch over LDS tiles:
+//   down, from x = 0:  red x = b / d;  black x = (b + sum red) / d;
+//     the residual is then 0 on the black nodes and sum of the black
+//     neighbours on the red ones; restrict it
+//   up:  red x = b / d + P x_c  (the descent's red values are formed again,
+//     so the descent stores nothing but the coarse right-hand side, and its
+//     black values are not needed);  black x = (b + sum red) / d;
+//     red x = (b + sum black) / d
+// Two sweeps a side converge in 0.7 times the iterations but take 11
+// launches a level instead of 2; the half sweeps ran at about 7.7 us each on
+// 128^3 (every one reads and writes the level) and at the 2.5 us of an empty
+// launch on small grids.
+//
+// A block holds a tile of TI x TJ x TK fine nodes with its halo in LDS, red
+// and black nodes in arrays of their own (a half sweep then reads
+// consecutive words): 3 nodes below and 2 above going down (black needs red
+// one ring out, the residual black, the restriction the residual), 2 on both
+// sides going up.  A thread keeps its place (j, k) in the tile's plane and
+// steps through the planes, so that the index arithmetic is done once (it
+// bound a version that divided a linear index at every node: 38 us a side
+// at 128^3).  Tiles of 8 x 8 x 64 with 512 threads reload 2.9 times their
+// nodes through L2 and fill the GPU from 2^20 nodes on; smaller levels are
+// bound by latency and take 4 x 8 x 32 with 256 threads, several times the
+// blocks.
+//
+// FINEST: the links of the finest level are those to free neighbours, so
+// its sums need no masks where pinned nodes hold 0; the diagonal is 6.
+template <int TI, int TJ, int TK, int LO, int HI>
+struct Tile3 {
+    static constexpr int SI = TI + LO + HI, SJ = TJ + LO + HI, SK = TK + LO + HI;
+    static constexpr int HK = (SK + 1) / 2;  // nodes of a colour in a row
+    static constexpr int PH = SJ * HK;       // and in a plane
+    static constexpr int N = SI * PH;
 };
-__device__ __forceinline__ Nb7 neighbours7(const float *x, size_t m, int i, int j, int k, int nx, int ny, int nz)
+
+// the sum over the links of the node at half-row index h of the other
+// colour's array x; s = e & 1 of its position e = 2 (h % HK) + s.  All six
+// are read and the unlinked ones dropped: no branch waits for the mask.
+template <int HK, int PH, bool FINEST>
+__device__ __forceinline__ float links_half(const float *x, int h, int s, uint8_t nb)
 {
-    const size_t sx = (size_t)ny * nz;
-    Nb7 q;
-    q.v[0] = x[i > 0 ? m - sx : m];
-    q.v[1] = x[j > 0 ? m - nz : m];
-    q.v[2] = x[k > 0 ? m - 1 : m];
-    q.v[3] = x[k < nz - 1 ? m + 1 : m];
-    q.v[4] = x[j < ny - 1 ? m + nz : m];
-    q.v[5] = x[i < nx - 1 ? m + sx : m];
-    return q;
+    const float q[6] = {x[h - PH], x[h - HK], x[h - 1 + s], x[h + s], x[h + HK], x[h + PH]};
+    if (FINEST) return ((q[0] + q[5]) + (q[1] + q[4])) + (q[2] + q[3]);
+    float v = 0.f;
+#pragma unroll
+    for (int l = 0; l < 6; l++) v += nb >> l & 1 ? q[l] : 0.f;
+    return v;
 }
 
-// red-black Gauss-Seidel half sweep, colour = (i+j+k) & 1.  Threads cover
-// only the nodes of the colour: thread (kk, j, i) updates k = 2 kk + parity,
-// blocks of 64 x 4 (kk, j) and a grid of (nz/2 / 64, ny / 4, nx).  The node
-// body is node3_rbgs's, in the same order, on neighbours read early.
+// The tile's masks and right-hand sides from memory: red nodes get b / d,
+// black ones b, pinned ones and those outside the grid 0.  A thread's
+// column of nodes is read whole before any is stored (clamped addresses,
+// so that no load waits behind a branch).
+template <class G, int THREADS, bool FINEST>
+__device__ __forceinline__ void tile3_load(const uint8_t *nbm, const float *di, const float *b, int nx, int ny, int nz,
+                                           int i0, int j0, int k0, float *sr, float *sk, float *sdr, float *sdk,
+                                           uint8_t *nr, uint8_t *nk)
+{
+    const int par0 = (i0 + j0 + k0) & 1;  // colour of the held corner
+#pragma unroll
+    for (int r = 0; r < (G::SJ * G::SK + THREADS - 1) / THREADS; r++) {
+        const int p = threadIdx.x + r * THREADS, c = p / G::SK, e = p % G::SK;
+        if (p >= G::SJ * G::SK) break;
+        const int j = j0 + c, k = k0 + e;
+        const bool in = (unsigned)j < (unsigned)ny && (unsigned)k < (unsigned)nz;
+        const int m0 = min(max(j, 0), ny - 1) * nz + min(max(k, 0), nz - 1), h0 = c * G::HK + (e >> 1);
+        uint8_t nb[G::SI];
+        float v[G::SI], d[FINEST ? 1 : G::SI];
+#pragma unroll
+        for (int a = 0; a < G::SI; a++) {
+            const size_t m = (size_t)min(max(i0 + a, 0), nx - 1) * ny * nz + m0;
+            nb[a] = nbm[m];
+            v[a] = b[m];
+            if (!FINEST) d[a] = di[m];
+        }
+#pragma unroll
+        for (int a = 0; a < G::SI; a++) {
+            const uint8_t q = in && (unsigned)(i0 + a) < (unsigned)nx ? nb[a] : kNbSelf;
+            const int h = a * G::PH + h0;
+            const bool black = (par0 + a + c + e) & 1;
+            float w = v[a];
+            if (!black) w *= FINEST ? 1.f / 6.f : d[a];
+            if (q & kNbSelf) w = 0.f;
+            (black ? sk : sr)[h] = w;
+            (black ? nk : nr)[h] = q;
+            if (!FINEST) (black ? sdk : sdr)[h] = d[a];
+        }
+    }
+}
+
+// black = (b + sum red) / d one ring inside the tile.  The rows' ends (e
+// outside the ring) are computed from whatever lies beside them and not used.
+template <class G, int THREADS, bool FINEST>
+__device__ __forceinline__ void tile3_black(int par0, const float *sr, float *sk, const float *sdk, const uint8_t *nk)
+{
+#pragma unroll
+    for (int r = 0; r < (G::PH + THREADS - 1) / THREADS; r++) {
+        const int p = threadIdx.x + r * THREADS, c = p / G::HK;
+        if (c < 1 || c > G::SJ - 2) continue;
+#pragma unroll
+        for (int a = 1; a < G::SI - 1; a++) {
+            const int h = a * G::PH + p;
+            const uint8_t nb = nk[h];
+            const float v = sk[h] + links_half<G::HK, G::PH, FINEST>(sr, h, (par0 + a + c + 1) & 1, nb);
+            sk[h] = nb & kNbSelf ? 0.f : v * (FINEST ? 1.f / 6.f : sdk[h]);
+        }
+    }
+}
+
+template <int TI, int TJ, int TK, int THREADS, bool FINEST>
+__global__ void __launch_bounds__(THREADS) k3_down(const uint8_t *nbm, const float *di, const float *b, int nx, int ny,
+                                                   int nz, float *bc, const uint8_t *nbmc, int cx, int cy, int cz,
+                                                   const int *stop)
+{
+    using G = Tile3<TI, TJ, TK, 3, 2>;
+    constexpr int HK = G::HK, PH = G::PH;
+    __shared__ float sr[G::N], sk[G::N], sdr[FINEST ? 1 : G::N], sdk[FINEST ? 1 : G::N];
+    __shared__ uint8_t nr[G::N], nk[G::N];
+    const int stopped_ = stop ? *stop : 0;  // read beside the operands
+    const int i0 = (int)blockIdx.z * TI - 3, j0 = (int)blockIdx.y * TJ - 3, k0 = (int)blockIdx.x * TK - 3;
+    const int par0 = (i0 + j0 + k0) & 1;
+    tile3_load<G, THREADS, FINEST>(nbm, di, b, nx, ny, nz, i0, j0, k0, sr, sk, sdr, sdk, nr, nk);
+    if (stopped_) return;  // uniform
+    __syncthreads();
+    tile3_black<G, THREADS, FINEST>(par0, sr, sk, sdk, nk);
+    __syncthreads();
+    // the residual on the red nodes two rings inside, in their place
+#pragma unroll
+    for (int r = 0; r < (PH + THREADS - 1) / THREADS; r++) {
+        const int p = threadIdx.x + r * THREADS, c = p / HK;
+        if (c < 2 || c > G::SJ - 3) continue;
+#pragma unroll
+        for (int a = 2; a < G::SI - 2; a++) {
+            const int h = a * PH + p;
+            const uint8_t nb = nr[h];
+            const float v = links_half<HK, PH, FINEST>(sk, h, (par0 + a + c) & 1, nb);
+            sr[h] = nb & kNbSelf ? 0.f : v;
+        }
+    }
+    __syncthreads();
+    // P^T r / 2: of the 27 fine nodes around a coarse one 13 are red, the
+    // node itself (weight 1) and the twelve two steps away (1/4 each);
+    // pinned ones hold 0
+    constexpr int CI = TI / 2, CJ = TJ / 2, CK = TK / 2;
+#pragma unroll
+    for (int t0 = 0; t0 < CI * CJ * CK; t0 += THREADS) {
+        const int t = t0 + threadIdx.x, a = t / (CJ * CK), c = t / CK % CJ, e = t % CK;
+        const int I = blockIdx.z * CI + a, J = blockIdx.y * CJ + c, K = blockIdx.x * CK + e;
+        if (t >= CI * CJ * CK || I >= cx || J >= cy || K >= cz) continue;
+        const size_t M = ((size_t)I * cy + J) * cz + K;
+        const uint8_t nb = nbmc[M];
+        // its fine node is at (3 + 2 a, 3 + 2 c, 3 + 2 e): half-row index
+        // e + 1, odd; the red nodes beside it at +-1 are even: e + 1, e + 2
+        const float *q = sr + ((3 + 2 * a) * G::SJ + 3 + 2 * c) * HK + 1 + e;
+        const float v = (q[-PH - HK] + q[-PH + HK] + q[PH - HK] + q[PH + HK]) +
+                        (q[-PH] + q[-PH + 1] + q[PH] + q[PH + 1]) + (q[-HK] + q[-HK + 1] + q[HK] + q[HK + 1]);
+        bc[M] = nb & kNbSelf ? 0.f : 0.5f * fmaf(0.25f, v, q[0]);
+    }
+}
+
+// DOT: out's product with b as well, dot = b.out (the CG's r.z)
+template <int TI, int TJ, int TK, int THREADS, bool FINEST, bool DOT>
+__global__ void __launch_bounds__(THREADS) k3_up(const uint8_t *nbm, const float *di, const float *b, int nx, int ny,
+                                                 int nz, const float *xc, int cx, int cy, int cz, float *out,
+                                                 double *partial, unsigned int *ticket, double *dot, int fin,
+                                                 const int *stop)
+{
+    using G = Tile3<TI, TJ, TK, 2, 2>;
+    constexpr int HK = G::HK, PH = G::PH;
+    constexpr int QI = TI / 2 + 3, QJ = TJ / 2 + 3, QK = TK / 2 + 3;
+    __shared__ float sr[G::N], sk[G::N], sdr[FINEST ? 1 : G::N], sdk[FINEST ? 1 : G::N], sc[QI * QJ * QK];
+    __shared__ uint8_t nr[G::N], nk[G::N];
+    const int stopped_ = stop ? *stop : 0;
+    const int i0 = (int)blockIdx.z * TI - 2, j0 = (int)blockIdx.y * TJ - 2, k0 = (int)blockIdx.x * TK - 2;  // even
+    // the coarse nodes the prolongation reads: from fine node i0 / 2 on
+    constexpr int NQ = (QI * QJ * QK + THREADS - 1) / THREADS;
+    float qv[NQ];
+#pragma unroll
+    for (int r = 0; r < NQ; r++) {
+        const int t = threadIdx.x + r * THREADS;
+        const int I = i0 / 2 + t / (QJ * QK), J = j0 / 2 + t / QK % QJ, K = k0 / 2 + t % QK;
+        const bool in = (unsigned)I < (unsigned)cx && (unsigned)J < (unsigned)cy && (unsigned)K < (unsigned)cz;
+        const float v = xc[((size_t)min(max(I, 0), cx - 1) * cy + min(max(J, 0), cy - 1)) * cz + min(max(K, 0), cz - 1)];
+        qv[r] = in ? v : 0.f;
+    }
+    tile3_load<G, THREADS, FINEST>(nbm, di, b, nx, ny, nz, i0, j0, k0, sr, sk, sdr, sdk, nr, nk);
+#pragma unroll
+    for (int r = 0; r < NQ; r++)
+        if (threadIdx.x + r * THREADS < QI * QJ * QK) sc[threadIdx.x + r * THREADS] = qv[r];
+    if (stopped_) return;  // uniform
+    __syncthreads();
+    // red += P x_c: a red node has no odd coordinate or two, and takes one
+    // coarse node or the mean of four
+#pragma unroll
+    for (int r = 0; r < (PH + THREADS - 1) / THREADS; r++) {
+        const int p = threadIdx.x + r * THREADS, c = p / HK, kk = p % HK;
+        if (p >= PH) break;
+        const float *qc = sc + (c >> 1) * QK + kk;
+        const int oj = c & 1;
+#pragma unroll
+        for (int a = 0; a < G::SI; a++) {
+            const int h = a * PH + p, s = (a + c) & 1, oi = a & 1;
+            const float *q = qc + (a >> 1) * (QJ * QK);
+            const int s1 = oi ? QJ * QK : oj ? QK : 0, s2 = s ? 1 : oj ? QK : 0;  // 0, 0: the node itself four times
+            const float v = 0.25f * ((q[0] + q[s1]) + (q[s2] + q[s1 + s2]));
+            sr[h] = nr[h] & kNbSelf ? 0.f : sr[h] + v;
+        }
+    }
+    __syncthreads();
+    tile3_black<G, THREADS, FINEST>(0, sr, sk, sdk, nk);
+    __syncthreads();
+    double acc[1] = {0};
+    static_assert(TJ * TK % THREADS == 0 || THREADS % (TJ * TK) == 0, "whole planes of threads");
+    constexpr int ROWS = THREADS > TJ * TK ? THREADS / (TJ * TK) : 1;  // planes at once
+    constexpr int REP = THREADS < TJ * TK ? TJ * TK / THREADS : 1;
+#pragma unroll
+    for (int r = 0; r < REP; r++) {
+        const int p = (threadIdx.x + r * THREADS) % (TJ * TK), c = 2 + p / TK, e = 2 + p % TK;
+        const int j = j0 + c, k = k0 + e;
+        if (j >= ny || k >= nz) continue;
+        const int m0 = j * nz + k, h0 = c * HK + (e >> 1), a0 = 2 + threadIdx.x / (TJ * TK);
+        float bm[TI / ROWS];
+#pragma unroll
+        for (int t = 0; t < TI / ROWS; t++) bm[t] = b[(size_t)min(i0 + a0 + t * ROWS, nx - 1) * ny * nz + m0];
+#pragma unroll
+        for (int t = 0; t < TI / ROWS; t++) {
+            const int a = a0 + t * ROWS, i = i0 + a, h = a * PH + h0;
+            const bool black = (a + c + e) & 1;
+            const uint8_t nb = (black ? nk : nr)[h];
+            const float w = bm[t] + links_half<HK, PH, FINEST>(sk, h, e & 1, nb);
+            float x = w * (FINEST ? 1.f / 6.f : sdr[h]);
+            if (black) x = sk[h];
+            if (nb & kNbSelf) x = 0.f;
+            if (i < nx) {
+                out[(size_t)i * ny * nz + m0] = x;
+                if (DOT) acc[0] += (double)bm[t] * x;
+            }
+        }
+    }
+    if constexpr (DOT) finish_sums<1, THREADS>(acc, partial, ticket, dot, fin);
+}
+
+// x = A^-1 b on the coarsest level, with the inverse held for all its nodes
+// (rows and columns of pinned ones 0): a wavefront a row.  On 9^3 nodes the
+// 2 MB are read once from L2 by 183 blocks; one workgroup running the levels
+// below 17^3 in its LDS took 15-17 us.
+__global__ void __launch_bounds__(256) k3_dense(const float *inv, const float *b, float *x, int n, const int *stop)
+{
+    const int stopped_ = stop ? *stop : 0;
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= n) return;
+    float s = 0.f;
+#pragma unroll 4
+    for (int c = lane; c < n; c += 64) s = fmaf(inv[(size_t)row * n + c], b[c], s);
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (lane == 0 && !stopped_) x[row] = s;
+}
+
+// Half sweep of colour on a grid that has one level only and is too large
+// for a dense solve (a side below 5 nodes): its preconditioner is symmetric
+// sweeps from zero.  Threads cover only the nodes of the colour: thread
+// (kk, j, i) updates k = 2 kk + parity, blocks of 64 x 4 (kk, j).
 constexpr int kRbgsX = 64, kRbgsY = 4;
 __global__ void __launch_bounds__(kRbgsX * kRbgsY) k3_rbgs(const uint8_t *nbm, float *x, const float *b, int nx,
                                                            int ny, int nz, int colour, const int *stop)
 {
     if (stopped(stop)) return;
-    const size_t sx = (size_t)ny * nz;
     const int i = blockIdx.z, j = blockIdx.y * kRbgsY + threadIdx.y;
     const int k = 2 * (blockIdx.x * kRbgsX + threadIdx.x) + ((i + j + colour) & 1);
-    if (j >= ny || k >= nz) return;
-    const size_t m = (size_t)i * sx + (size_t)j * nz + k;
+    if (i >= nx || j >= ny || k >= nz) return;
+    const int m = (i * ny + j) * nz + k;
     const uint8_t nb = nbm[m];
-    const float bm = b[m];
-    const Nb7 q = neighbours7(x, m, i, j, k, nx, ny, nz);
-    if (nb & kNbSelf) return;
-    float s = bm;
-    if (nb & 1) s += q.v[0];
-    if (nb & 2) s += q.v[1];
-    if (nb & 4) s += q.v[2];
-    if (nb & 8) s += q.v[3];
-    if (nb & 16) s += q.v[4];
-    if (nb & 32) s += q.v[5];
-    x[m] = s * (1.f / 6.f);
+    if (!(nb & kNbSelf)) x[m] = (b[m] + links7(nb, x, m, ny * nz, nz)) * (1.f / 6.f);
 }
 
-// x = 0, then the colour-0 half sweep, in one pass over every node: from
-// zero, every neighbour a colour-0 node reads is +0, so its update is
-// (b + 0) / 6 -- the +0 once, which turns a -0 right-hand side into +0 as
-// the sweep's sums do, and not at all for a node with no free neighbour.
-// Blocks of 64 x 4 nodes (k, j) and a grid of (nz / 64, ny / 4, nx).
-__global__ void __launch_bounds__(256) k3_rbgs_from_zero(const uint8_t *nbm, float *x, const float *b, int nx,
-                                                         int ny, int nz, const int *stop)
+__global__ void k3_zero(float *x, size_t n, const int *stop)
 {
     if (stopped(stop)) return;
-    const int i = blockIdx.z, j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.x * 64 + threadIdx.x;
-    if (j >= ny || k >= nz) return;
-    const size_t m = ((size_t)i * ny + j) * nz + k;
-    const uint8_t nb = nbm[m];
-    float v = 0.f;
-    if (((i + j + k) & 1) == 0 && !(nb & kNbSelf)) {
-        float t = b[m];
-        if (nb & 63) t += 0.f;
-        v = t * (1.f / 6.f);
-    }
-    x[m] = v;
+    size_t m = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (m < n) x[m] = 0.f;
 }
 
-// r = b - A' x; blocks of 64 x 4 nodes (k, j) and a grid of (nz / 64, ny / 4, nx)
-__global__ void __launch_bounds__(256) k3_resid(const uint8_t *nbm, const float *x, const float *b, float *r, int nx,
-                                                int ny, int nz, const int *stop)
-{
-    if (stopped(stop)) return;
-    const int i = blockIdx.z, j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.x * 64 + threadIdx.x;
-    if (j >= ny || k >= nz) return;
-    const size_t m = ((size_t)i * ny + j) * nz + k;
-    const uint8_t nb = nbm[m];
-    const float bm = b[m], xm = x[m];
-    const Nb7 q = neighbours7(x, m, i, j, k, nx, ny, nz);
-    // apply7's body, in its order, on the neighbours read early
-    float s = 6.f * xm;
-    if (nb & 1) s -= q.v[0];
-    if (nb & 2) s -= q.v[1];
-    if (nb & 4) s -= q.v[2];
-    if (nb & 8) s -= q.v[3];
-    if (nb & 16) s -= q.v[4];
-    if (nb & 32) s -= q.v[5];
-    r[m] = (nb & kNbSelf) ? 0.f : bm - s;
-}
-
-
-// 1D weights of the trilinear prolongation: fine i from coarse I
-__device__ __forceinline__ float w1(int i, int I) { int d = i - 2 * I; return d == 0 ? 1.f : (d == 1 || d == -1 ? 0.5f : 0.f); }
-
-// b_c = P^T r_f / 2 at free coarse node M = (I, J, K).  The 27 fine nodes
-// are summed in (i, j, k) order; one outside the grid reads a node inside
-// with weight 0, which adds +0 to a sum that never holds -0: the same bits
-// as skipping it, with every load issued at once.
-__device__ __forceinline__ float node3_restrict_at(const float *rf, int fx, int fy, int fz, int I, int J, int K)
-{
-    float w[3][3];
-    int ix[3][3];
-    const int c[3] = {I, J, K}, nf[3] = {fx, fy, fz};
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-#pragma unroll
-        for (int t = 0; t < 3; t++) {
-            const int f = 2 * c[d] - 1 + t;
-            const bool in = f >= 0 && f < nf[d];
-            ix[d][t] = in ? f : 2 * c[d];
-            w[d][t] = in ? w1(f, c[d]) : 0.f;
-        }
-    }
-    float v[27];
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-        for (int b = 0; b < 3; b++)
-#pragma unroll
-            for (int e = 0; e < 3; e++)
-                v[(a * 3 + b) * 3 + e] = rf[((size_t)ix[0][a] * fy + ix[1][b]) * fz + ix[2][e]];
-    float s = 0.f;
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-        for (int b = 0; b < 3; b++) {
-            const float wij = w[0][a] * w[1][b];
-#pragma unroll
-            for (int e = 0; e < 3; e++) s = fmaf(wij * w[2][e], v[(a * 3 + b) * 3 + e], s);  // r is 0 on Dirichlet nodes
-        }
-    return 0.5f * s;
-}
-
-__device__ __forceinline__ float node3_restrict(const float *rf, int fx, int fy, int fz, const uint8_t *dirc, int cy,
-                                                int cz, size_t M)
-{
-    if (dirc[M]) return 0.f;
-    int I, J, K;
-    node3(M, cy, cz, I, J, K);
-    return node3_restrict_at(rf, fx, fy, fz, I, J, K);
-}
-
-// blocks of 64 x 4 coarse nodes (K, J) and a grid of (cz / 64, cy / 4, cx):
-// the coordinates come from the launch, not from divisions
-__global__ void __launch_bounds__(256) k3_restrict(const float *rf, int fx, int fy, int fz, float *bc,
-                                                   const uint8_t *dirc, int cx, int cy, int cz, const int *stop)
-{
-    if (stopped(stop)) return;
-    const int I = blockIdx.z, J = blockIdx.y * 4 + threadIdx.y, K = blockIdx.x * 64 + threadIdx.x;
-    if (J >= cy || K >= cz) return;
-    const size_t M = ((size_t)I * cy + J) * cz + K;
-    bc[M] = dirc[M] ? 0.f : node3_restrict_at(rf, fx, fy, fz, I, J, K);
-}
-
-// x_f += P x_c at free fine node m = (i, j, k)
-__device__ __forceinline__ void node3_prolong_at(float *xf, int i, int j, int k, const float *xc, int cx, int cy,
-                                                 int cz, size_t m)
-{
-    // per axis the coarse nodes of fine index f: f / 2 (weight 1) when f is
-    // even, else (f - 1) / 2 and (f + 1) / 2 (0.5 each; the second can lie
-    // past the coarse grid).  All 8 combinations are summed in (a, b, c)
-    // order; an absent node is read at the first with weight 0, which adds
-    // +0 to a sum that never holds -0 -- the same bits as skipping it, with
-    // the loads issued together.
-    int Ia[2], Ja[2], Ka[2];
-    float wa[2], wb[2], wc[2];
-    auto split = [](int f, int nc, int *I, float *w) {
-        const bool odd = f & 1, second = odd && (f + 1) / 2 < nc;
-        I[0] = f >> 1;
-        w[0] = odd ? 0.5f : 1.f;
-        I[1] = second ? (f + 1) / 2 : I[0];
-        w[1] = second ? 0.5f : 0.f;
-    };
-    split(i, cx, Ia, wa);
-    split(j, cy, Ja, wb);
-    split(k, cz, Ka, wc);
-    float v[8];
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int c = 0; c < 2; c++) v[(a * 2 + b) * 2 + c] = xc[((size_t)Ia[a] * cy + Ja[b]) * cz + Ka[c]];
-    float s = 0.f;
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int c = 0; c < 2; c++) s = fmaf(wa[a] * wb[b] * wc[c], v[(a * 2 + b) * 2 + c], s);
-    xf[m] += s;
-}
-
-// x_f += P x_c at fine node m (a free node)
-__device__ __forceinline__ void node3_prolong_free(float *xf, int fy, int fz, const float *xc, int cx, int cy, int cz,
-                                                   size_t m)
-{
-    int i, j, k;
-    node3(m, fy, fz, i, j, k);
-    node3_prolong_at(xf, i, j, k, xc, cx, cy, cz, m);
-}
-
-// x_f += P x_c at fine node m when it is free
-__device__ __forceinline__ void node3_prolong(float *xf, const uint8_t *dirf, int fy, int fz, const float *xc, int cx,
-                                              int cy, int cz, size_t m)
-{
-    if (!dirf[m]) node3_prolong_free(xf, fy, fz, xc, cx, cy, cz, m);
-}
-
-// x_f += P x_c on free fine nodes; blocks of 64 x 4 nodes (k, j) and a grid
-// of (fz / 64, fy / 4, fx)
-__global__ void __launch_bounds__(256) k3_prolong(float *xf, const uint8_t *dirf, int fx, int fy, int fz,
-                                                  const float *xc, int cx, int cy, int cz, const int *stop)
-{
-    if (stopped(stop)) return;
-    const int i = blockIdx.z, j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.x * 64 + threadIdx.x;
-    if (j >= fy || k >= fz) return;
-    const size_t m = ((size_t)i * fy + j) * fz + k;
-    if (!dirf[m]) node3_prolong_at(xf, i, j, k, xc, cx, cy, cz, m);
-}
-
-// ---- the coarse levels [lc, L) of the V-cycle in one workgroup: the same
-// node bodies and sweep order as the grid kernels, a workgroup barrier
-// between sweeps instead of a launch
+// A coarsest level too large for a dense solve (a thin grid's): kCoarseSweeps
+// symmetric red-black sweeps from zero, half of them in reverse order, by one
+// workgroup with barriers between the half sweeps
 constexpr int kMaxLevels3 = 16;
-constexpr size_t kBlockLevelNodes3 = 4096;  // levels this small run inside the workgroup
-
-struct BLevel3 {
-    int nx, ny, nz, n;
-    const uint8_t *dir, *nbm;
-    float *x, *b, *r;
-};
-
-struct Coarse3Args {
-    int lc, L;
-    BLevel3 lv[kMaxLevels3];
-    int dense;          // dense coarsest solve (else sweeps symmetric RB-GS sweeps)
-    const float *invT;  // the dense inverse, transposed
-    int coarse_n, sweeps, pre, post;
-    const int *stop;    // the solve's stop flag (see stopped())
-};
-
-__device__ void c3_smooth(const BLevel3 &V, float *x, const float *b, int sweeps, bool forward)
+__global__ void __launch_bounds__(kCoarseThreads) k3_sweeps(const uint8_t *nbm, const float *di, const float *b,
+                                                            float *x, int ny, int nz, int n, int sweeps,
+                                                            const int *stop)
 {
-    const size_t sx = (size_t)V.ny * V.nz;
-    for (int it = 0; it < sweeps; it++) {
-        for (int h = 0; h < 2; h++) {
-            const int colour = forward ? h : 1 - h;
-            for (int m = threadIdx.x; m < V.n; m += kCoarseThreads) {
-                int i, j, k;
-                node3((size_t)m, V.ny, V.nz, i, j, k);
-                if (((i + j + k) & 1) == colour) node3_rbgs(V.nbm, x, b, (size_t)m, sx, V.nz);
-            }
-            __syncthreads();
-        }
-    }
-}
-
-__global__ void __launch_bounds__(kCoarseThreads) k3_vcycle_coarse(Coarse3Args C)
-{
-    if (stopped(C.stop)) return;
-    extern __shared__ float sb[];  // dense solve: coarse_n words, then kDenseParts partial rows
-    for (int l = C.lc; l < C.L - 1; l++) {
-        const BLevel3 &V = C.lv[l];
-        for (int m = threadIdx.x; m < V.n; m += kCoarseThreads) V.x[m] = 0.f;
-        __syncthreads();
-        c3_smooth(V, V.x, V.b, C.pre, true);
-        const size_t sx = (size_t)V.ny * V.nz;
-        for (int m = threadIdx.x; m < V.n; m += kCoarseThreads) {
-            const uint8_t nb = V.nbm[m];
-            V.r[m] = (nb & kNbSelf) ? 0.f : V.b[m] - apply7(nb, V.x, (size_t)m, sx, V.nz);
-        }
-        __syncthreads();
-        const BLevel3 &W = C.lv[l + 1];
-        for (int M = threadIdx.x; M < W.n; M += kCoarseThreads)
-            W.b[M] = node3_restrict(V.r, V.nx, V.ny, V.nz, W.dir, W.ny, W.nz, (size_t)M);
-        __syncthreads();
-    }
-    {
-        const BLevel3 &Z = C.lv[C.L - 1];
-        if (C.dense) {
-            const int n = C.coarse_n;
-            float *part = sb + n;
-            for (int k = threadIdx.x; k < n; k += kCoarseThreads) sb[k] = Z.b[k];
-            __syncthreads();
-            const int len = (n + kDenseParts - 1) / kDenseParts;
-            for (int t = threadIdx.x; t < n * kDenseParts; t += kCoarseThreads) {
-                const int row = t % n, p = t / n;
-                const int c0 = p * len, c1 = min(n, c0 + len);
-                float s = 0.f;
-                int c = c0;
-                for (; c + 8 <= c1; c += 8) {
-                    float a[8];
-#pragma unroll
-                    for (int q = 0; q < 8; q++) a[q] = C.invT[(size_t)(c + q) * n + row];
-#pragma unroll
-                    for (int q = 0; q < 8; q++) s = fmaf(a[q], sb[c + q], s);
-                }
-                for (; c < c1; c++) s = fmaf(C.invT[(size_t)c * n + row], sb[c], s);
-                part[p * n + row] = s;
-            }
-            __syncthreads();
-            for (int row = threadIdx.x; row < n; row += kCoarseThreads) {
-                float s = part[row];
-                for (int p = 1; p < kDenseParts; p++) s += part[p * n + row];
-                Z.x[row] = s;
-            }
-            __syncthreads();
-        } else {
-            for (int m = threadIdx.x; m < Z.n; m += kCoarseThreads) Z.x[m] = 0.f;
-            __syncthreads();
-            c3_smooth(Z, Z.x, Z.b, C.sweeps / 2, true);
-            c3_smooth(Z, Z.x, Z.b, C.sweeps / 2, false);
-        }
-    }
-    for (int l = C.L - 2; l >= C.lc; l--) {
-        const BLevel3 &V = C.lv[l];
-        const BLevel3 &W = C.lv[l + 1];
-        for (int m = threadIdx.x; m < V.n; m += kCoarseThreads)
-            node3_prolong(V.x, V.dir, V.ny, V.nz, W.x, W.nx, W.ny, W.nz, (size_t)m);
-        __syncthreads();
-        c3_smooth(V, V.x, V.b, C.post, false);
-    }
-}
-
-// The common case -- one red-black level of at most 4096 nodes above a dense
-// level of at most 512 -- with both levels in LDS and each thread's nodes and
-// their colours computed once.  Same node updates and order, same bits.
-constexpr int kLds3Nodes = 4096, kLds3Dense = 512, kLds3PerThread = kLds3Nodes / kCoarseThreads;
-
-__global__ void __launch_bounds__(kCoarseThreads) k3_vcycle_coarse_lds(Coarse3Args C)
-{
-    if (stopped(C.stop)) return;
-    __shared__ float s_x[kLds3Nodes], s_b[kLds3Nodes], s_r[kLds3Nodes];
-    __shared__ uint8_t s_nb[kLds3Nodes];
-    __shared__ float s_zb[kLds3Dense], s_zx[kLds3Dense];
-    const BLevel3 &V = C.lv[C.lc];
-    const BLevel3 &Z = C.lv[C.lc + 1];
-    const int n = V.n, ny = V.ny, nz = V.nz, cn = C.coarse_n;
-    const size_t sx = (size_t)ny * nz;
-    int par[kLds3PerThread];
-#pragma unroll
-    for (int q = 0; q < kLds3PerThread; q++) {
-        const int m = threadIdx.x + q * kCoarseThreads;
-        par[q] = 2;
-        if (m < n) {
-            int i, j, k;
-            node3((size_t)m, ny, nz, i, j, k);
-            par[q] = (i + j + k) & 1;
-            s_nb[m] = V.nbm[m];
-            s_b[m] = V.b[m];
-            s_x[m] = 0.f;
-        }
-    }
+    if (stopped(stop)) return;
+    for (int m = threadIdx.x; m < n; m += kCoarseThreads) x[m] = 0.f;
     __syncthreads();
-    auto sweep = [&](int colour) {
-#pragma unroll
-        for (int q = 0; q < kLds3PerThread; q++)
-            if (par[q] == colour) node3_rbgs(s_nb, s_x, s_b, (size_t)(threadIdx.x + q * kCoarseThreads), sx, nz);
-        __syncthreads();
-    };
-    for (int it = 0; it < C.pre; it++) { sweep(0); sweep(1); }
-#pragma unroll
-    for (int q = 0; q < kLds3PerThread; q++) {
-        const int m = threadIdx.x + q * kCoarseThreads;
-        if (m < n) {
-            const uint8_t nb = s_nb[m];
-            s_r[m] = (nb & kNbSelf) ? 0.f : s_b[m] - apply7(nb, s_x, (size_t)m, sx, nz);
-        }
-    }
-    __syncthreads();
-    for (int M = threadIdx.x; M < cn; M += kCoarseThreads)
-        s_zb[M] = node3_restrict(s_r, V.nx, ny, nz, Z.dir, Z.ny, Z.nz, (size_t)M);
-    __syncthreads();
-    {
-        // the dense solve of k3_vcycle_coarse; its partial rows reuse s_r
-        float *part = s_r;
-        const int len = (cn + kDenseParts - 1) / kDenseParts;
-        for (int t = threadIdx.x; t < cn * kDenseParts; t += kCoarseThreads) {
-            const int row = t % cn, p = t / cn;
-            const int c0 = p * len, c1 = min(cn, c0 + len);
-            float s = 0.f;
-            int c = c0;
-            for (; c + 32 <= c1; c += 32) {  // 32 loads in flight: the loop waits on L2
-                float a[32];
-#pragma unroll
-                for (int q = 0; q < 32; q++) a[q] = C.invT[(size_t)(c + q) * cn + row];
-#pragma unroll
-                for (int q = 0; q < 32; q++) s = fmaf(a[q], s_zb[c + q], s);
-            }
-            for (; c < c1; c++) s = fmaf(C.invT[(size_t)c * cn + row], s_zb[c], s);
-            part[p * cn + row] = s;
+    for (int h = 0; h < 2 * sweeps; h++) {
+        const uint8_t colour = (h & 1) == (h < sweeps ? 0 : 1) ? 0 : kNbBlack;
+        for (int m = threadIdx.x; m < n; m += kCoarseThreads) {
+            const uint8_t nb = nbm[m];
+            if ((nb & (kNbSelf | kNbBlack)) == colour) x[m] = (b[m] + links7(nb, x, m, ny * nz, nz)) * di[m];
         }
         __syncthreads();
-        for (int row = threadIdx.x; row < cn; row += kCoarseThreads) {
-            float s = part[row];
-            for (int p = 1; p < kDenseParts; p++) s += part[p * cn + row];
-            s_zx[row] = s;
-        }
-        __syncthreads();
-    }
-    // node3_prolong with the pinned flag from the neighbour mask
-#pragma unroll
-    for (int q = 0; q < kLds3PerThread; q++) {
-        const int m = threadIdx.x + q * kCoarseThreads;
-        if (m < n && !(s_nb[m] & kNbSelf)) node3_prolong_free(s_x, ny, nz, s_zx, Z.nx, Z.ny, Z.nz, (size_t)m);
-    }
-    __syncthreads();
-    for (int it = 0; it < C.post; it++) { sweep(1); sweep(0); }
-#pragma unroll
-    for (int q = 0; q < kLds3PerThread; q++) {
-        const int m = threadIdx.x + q * kCoarseThreads;
-        if (m < n) V.x[m] = s_x[m];
     }
 }
 
@@ -1146,233 +1113,6 @@ static int check_parts3(const m2d_particles3d *p)
     return M2D_OK;
 }
 
-// Gauss-Jordan inverse of the coarsest 7-point operator on its free nodes
-static bool dense_inverse7(const std::vector<uint8_t> &dir, int nx, int ny, int nz, std::vector<float> &inv)
-{
-    const int n = nx * ny * nz;
-    std::vector<int> id, pos(n, -1);
-    for (int m = 0; m < n; m++)
-        if (!dir[m]) { pos[m] = (int)id.size(); id.push_back(m); }
-    const int q = (int)id.size();
-    std::vector<double> a((size_t)q * 2 * q, 0.0);
-    const int sx = ny * nz;
-    for (int r = 0; r < q; r++) {
-        const int m = id[r];
-        a[(size_t)r * 2 * q + r] = 6.0;
-        for (int nb : {m - sx, m - nz, m - 1, m + 1, m + nz, m + sx}) {
-            if (nb < 0 || nb >= n || pos[nb] < 0) continue;
-            a[(size_t)r * 2 * q + pos[nb]] = -1.0;
-        }
-        a[(size_t)r * 2 * q + q + r] = 1.0;
-    }
-    for (int c = 0; c < q; c++) {
-        int piv = c;
-        for (int r = c + 1; r < q; r++)
-            if (fabs(a[(size_t)r * 2 * q + c]) > fabs(a[(size_t)piv * 2 * q + c])) piv = r;
-        if (fabs(a[(size_t)piv * 2 * q + c]) < 1e-300) return false;
-        if (piv != c)
-            for (int t = 0; t < 2 * q; t++) std::swap(a[(size_t)c * 2 * q + t], a[(size_t)piv * 2 * q + t]);
-        const double d = 1.0 / a[(size_t)c * 2 * q + c];
-        for (int t = 0; t < 2 * q; t++) a[(size_t)c * 2 * q + t] *= d;
-        for (int r = 0; r < q; r++) {
-            if (r == c) continue;
-            const double f = a[(size_t)r * 2 * q + c];
-            if (f == 0.0) continue;
-            for (int t = 0; t < 2 * q; t++) a[(size_t)r * 2 * q + t] -= f * a[(size_t)c * 2 * q + t];
-        }
-    }
-    inv.assign((size_t)n * n, 0.f);
-    for (int r = 0; r < q; r++)
-        for (int c = 0; c < q; c++) inv[(size_t)id[r] * n + id[c]] = (float)a[(size_t)r * 2 * q + q + c];
-    return true;
-}
-
-constexpr int kCoarseDenseMax = 1024;   // free nodes for the dense coarsest solve
-constexpr int kCoarseSweeps = 40;       // symmetric RB-GS sweeps otherwise
-
-static int mg3_setup(m2d_fields3d *f, const std::vector<uint8_t> &mask)
-{
-    std::vector<std::vector<uint8_t>> dirs;
-    std::vector<int> dims;  // nx, ny, nz per level
-    std::vector<uint8_t> d0(f->n);
-    for (size_t m = 0; m < f->n; m++) d0[m] = mask[m] == M2D_FIXED || mask[m] == M2D_FIXED_RF;
-    dirs.push_back(std::move(d0));
-    dims.insert(dims.end(), {f->nx, f->ny, f->nz});
-    for (;;) {
-        const int fx = dims[dims.size() - 3], fy = dims[dims.size() - 2], fz = dims[dims.size() - 1];
-        if ((size_t)fx * fy * fz <= 512 || fx < 5 || fy < 5 || fz < 5) break;
-        const int cx = (fx - 1) / 2 + 1, cy = (fy - 1) / 2 + 1, cz = (fz - 1) / 2 + 1;
-        const std::vector<uint8_t> &df = dirs.back();
-        std::vector<uint8_t> dc((size_t)cx * cy * cz);
-        for (int I = 0; I < cx; I++)
-            for (int J = 0; J < cy; J++)
-                for (int K = 0; K < cz; K++) {
-                    const bool face = I == 0 || J == 0 || K == 0 || I == cx - 1 || J == cy - 1 || K == cz - 1;
-                    dc[((size_t)I * cy + J) * cz + K] =
-                        face || df[((size_t)(2 * I) * fy + 2 * J) * fz + 2 * K];
-                }
-        dirs.push_back(std::move(dc));
-        dims.insert(dims.end(), {cx, cy, cz});
-    }
-    const size_t L = dirs.size();
-    f->lv.resize(L);
-    for (size_t l = 0; l < L; l++) {
-        Mg3Level &V = f->lv[l];
-        V.nx = dims[3 * l]; V.ny = dims[3 * l + 1]; V.nz = dims[3 * l + 2];
-        V.n = (size_t)V.nx * V.ny * V.nz;
-        M2D_TRY(dmalloc3((void **)&V.dir, V.n));
-        M2D_TRY(dmalloc3((void **)&V.nbm, V.n));
-        M2D_TRY(dmalloc3((void **)&V.x, sizeof(float) * V.n));
-        M2D_TRY(dmalloc3((void **)&V.b, sizeof(float) * V.n));
-        M2D_TRY(dmalloc3((void **)&V.r, sizeof(float) * V.n));
-        M2D_HIP(hipMemcpy(V.dir, dirs[l].data(), V.n, hipMemcpyHostToDevice));
-        // neighbour masks (a free node never sits on a face)
-        const std::vector<uint8_t> &d = dirs[l];
-        std::vector<uint8_t> nbm(V.n);
-        const size_t sx = (size_t)V.ny * V.nz;
-        for (int i = 0; i < V.nx; i++)
-            for (int j = 0; j < V.ny; j++)
-                for (int k = 0; k < V.nz; k++) {
-                    const size_t m = (size_t)i * sx + (size_t)j * V.nz + k;
-                    if (d[m]) { nbm[m] = kNbSelf; continue; }
-                    const bool inside = i > 0 && i < V.nx - 1 && j > 0 && j < V.ny - 1 && k > 0 && k < V.nz - 1;
-                    M2D_CHECK(inside, M2D_ERR_BAD_ARG, "Fields3D: free node on a face of level %d", (int)l);
-                    const size_t nb[6] = {m - sx, m - (size_t)V.nz, m - 1, m + 1, m + (size_t)V.nz, m + sx};
-                    uint8_t bits = 0;
-                    for (int q = 0; q < 6; q++)
-                        if (!d[nb[q]]) bits |= (uint8_t)(1u << q);
-                    nbm[m] = bits;
-                }
-        M2D_HIP(hipMemcpy(V.nbm, nbm.data(), V.n, hipMemcpyHostToDevice));
-    }
-    M2D_CHECK(L <= (size_t)kMaxLevels3, M2D_ERR_BAD_ARG, "Fields3D: %d multigrid levels", (int)L);
-    f->lc3 = (int)L - 1;
-    for (size_t l = 1; l < L; l++)
-        if (f->lv[l].n <= kBlockLevelNodes3) { f->lc3 = (int)l; break; }
-    const Mg3Level &C = f->lv.back();
-    size_t nfree = 0;
-    for (uint8_t d : dirs.back()) nfree += !d;
-    f->coarse_dense = nfree <= (size_t)kCoarseDenseMax && C.n <= 1024;
-    if (f->coarse_dense) {
-        std::vector<float> inv;
-        M2D_CHECK(dense_inverse7(dirs.back(), C.nx, C.ny, C.nz, inv), M2D_ERR_BAD_ARG,
-                  "Fields3D: coarsest multigrid operator is singular");
-        f->coarse_n = (int)C.n;
-        M2D_TRY(dmalloc3((void **)&f->coarse_inv, sizeof(float) * inv.size()));
-        M2D_HIP(hipMemcpy(f->coarse_inv, inv.data(), sizeof(float) * inv.size(), hipMemcpyHostToDevice));
-        const size_t cn = (size_t)f->coarse_n;
-        std::vector<float> invT(cn * cn);
-        for (size_t r = 0; r < cn; r++)
-            for (size_t c = 0; c < cn; c++) invT[c * cn + r] = inv[r * cn + c];
-        M2D_TRY(dmalloc3((void **)&f->coarse_invT, sizeof(float) * invT.size()));
-        M2D_HIP(hipMemcpy(f->coarse_invT, invT.data(), sizeof(float) * invT.size(), hipMemcpyHostToDevice));
-    }
-    const size_t n = f->n;
-    for (float **q : {&f->pr, &f->pz, &f->pp, &f->pp2, &f->pq, &f->pe}) M2D_TRY(dmalloc3((void **)q, sizeof(float) * n));
-    M2D_TRY(dmalloc3((void **)&f->r64, sizeof(double) * n));
-    // 16 scalars, then the solve's control block
-    M2D_TRY(dmalloc3((void **)&f->dots, sizeof(double) * 32));
-    M2D_HIP(hipHostMalloc((void **)&f->h_dots, sizeof(double) * 32));
-    f->npartial = (int)std::min<size_t>((n + 255) / 256, 65536);
-    // up to three sums per block of the fused reductions
-    M2D_TRY(dmalloc3((void **)&f->partial, sizeof(double) * 3 * std::max<size_t>(f->npartial, (n + 255) / 256)));
-    M2D_TRY(dmalloc3((void **)&f->ticket, sizeof(unsigned int)));
-    M2D_HIP(hipMemset(f->ticket, 0, sizeof(unsigned int)));
-    return M2D_OK;
-}
-
-constexpr int kPre3 = 2, kPost3 = 2;
-
-__global__ void k3_zero(float *x, size_t n, const int *stop)
-{
-    if (stopped(stop)) return;
-    size_t m = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (m < n) x[m] = 0.f;
-}
-
-static unsigned blocks_for(size_t n) { return (unsigned)((n + 255) / 256); }
-
-static int vcycle3(m2d_fields3d *f, const float *rhs, float *out, const int *stop)
-{
-    hipStream_t s = f->ctx->stream;
-    const int L = (int)f->lv.size();
-    // from_zero: x starts at 0 (the first half sweep also clears x)
-    auto smooth = [&](Mg3Level &V, float *x, const float *b, int sweeps, bool forward, bool from_zero = false) {
-        const dim3 g((unsigned)(((V.nz + 1) / 2 + kRbgsX - 1) / kRbgsX), (unsigned)((V.ny + kRbgsY - 1) / kRbgsY),
-                     (unsigned)V.nx);
-        const dim3 blk(kRbgsX, kRbgsY);
-        for (int it = 0; it < sweeps; it++) {
-            if (it == 0 && from_zero && forward) {
-                k3_rbgs_from_zero<<<dim3((unsigned)((V.nz + 63) / 64), (unsigned)((V.ny + 3) / 4), (unsigned)V.nx),
-                                    dim3(64, 4), 0, s>>>(V.nbm, x, b, V.nx, V.ny, V.nz, stop);
-            } else {
-                k3_rbgs<<<g, blk, 0, s>>>(V.nbm, x, b, V.nx, V.ny, V.nz, forward ? 0 : 1, stop);
-            }
-            k3_rbgs<<<g, blk, 0, s>>>(V.nbm, x, b, V.nx, V.ny, V.nz, forward ? 1 : 0, stop);
-        }
-    };
-    // levels [lc, L) run in one workgroup (k3_vcycle_coarse) when lc > 0
-    const int lc = L > 1 ? f->lc3 : L;
-    for (int l = 0; l < std::min(lc, L - 1); l++) {
-        Mg3Level &V = f->lv[l];
-        float *x = l == 0 ? out : V.x;
-        const float *b = l == 0 ? rhs : V.b;
-        smooth(V, x, b, kPre3, true, true);
-        k3_resid<<<dim3((unsigned)((V.nz + 63) / 64), (unsigned)((V.ny + 3) / 4), (unsigned)V.nx), dim3(64, 4), 0,
-                   s>>>(V.nbm, x, b, V.r, V.nx, V.ny, V.nz, stop);
-        Mg3Level &C = f->lv[l + 1];
-        k3_restrict<<<dim3((unsigned)((C.nz + 63) / 64), (unsigned)((C.ny + 3) / 4), (unsigned)C.nx), dim3(64, 4), 0,
-                      s>>>(V.r, V.nx, V.ny, V.nz, C.b, C.dir, C.nx, C.ny, C.nz, stop);
-    }
-    if (lc < L) {
-        Coarse3Args C;
-        C.lc = lc;
-        C.L = L;
-        for (int l = 0; l < L; l++) {
-            const Mg3Level &V = f->lv[l];
-            C.lv[l] = BLevel3{V.nx, V.ny, V.nz, (int)V.n, V.dir, V.nbm, V.x, V.b, V.r};
-        }
-        C.dense = f->coarse_dense;
-        C.invT = f->coarse_invT;
-        C.coarse_n = f->coarse_n;
-        C.sweeps = kCoarseSweeps;
-        C.pre = kPre3;
-        C.post = kPost3;
-        C.stop = stop;
-        if (L - 1 - lc == 1 && f->lv[lc].n <= (size_t)kLds3Nodes && C.dense && f->coarse_n <= kLds3Dense) {
-            k3_vcycle_coarse_lds<<<1, kCoarseThreads, 0, s>>>(C);
-        } else {
-            const size_t shm = C.dense ? sizeof(float) * f->coarse_n * (1 + kDenseParts) : 0;
-            k3_vcycle_coarse<<<1, kCoarseThreads, shm, s>>>(C);
-        }
-    } else {
-        Mg3Level &C = f->lv[L - 1];
-        float *x = L == 1 ? out : C.x;
-        const float *b = L == 1 ? rhs : C.b;
-        if (f->coarse_dense) {
-            k_dense_solve<<<1, kCoarseThreads, sizeof(float) * f->coarse_n * (1 + kDenseParts), s>>>(
-                f->coarse_invT, b, x, f->coarse_n, stop);
-        } else {
-            k3_zero<<<blocks_for(C.n), 256, 0, s>>>(x, C.n, stop);
-            smooth(C, x, b, kCoarseSweeps / 2, true);
-            smooth(C, x, b, kCoarseSweeps / 2, false);
-        }
-    }
-    for (int l = std::min(lc, L - 1) - 1; l >= 0; l--) {
-        Mg3Level &V = f->lv[l];
-        Mg3Level &C = f->lv[l + 1];
-        float *x = l == 0 ? out : V.x;
-        const float *b = l == 0 ? rhs : V.b;
-        k3_prolong<<<dim3((unsigned)((V.nz + 63) / 64), (unsigned)((V.ny + 3) / 4), (unsigned)V.nx), dim3(64, 4), 0,
-                     s>>>(x, V.dir, V.nx, V.ny, V.nz, C.x, C.nx, C.ny, C.nz, stop);
-        smooth(V, x, b, kPost3, false);
-    }
-    M2D_HIP(hipGetLastError());
-    return M2D_OK;
-}
-
-static SolveCtl *solve_ctl3(m2d_fields3d *f) { return (SolveCtl *)(f->dots + 16); }
-
 // blocks of the fused reductions over the finest level: one node a thread up
 // to kRed3Blocks blocks (524288 nodes), then that many, whose threads stride
 // over several nodes (each block's reduction and partial sum then serve more
@@ -1380,11 +1120,267 @@ static SolveCtl *solve_ctl3(m2d_fields3d *f) { return (SolveCtl *)(f->dots + 16)
 // bits, which the FP32 CG coefficients round away in practice).  At 128^3,
 // 2048 blocks made the step 3% faster than one node a thread, 1024 and 4096
 // less so.
-constexpr size_t kRed3Blocks = 2048;
+constexpr size_t kRed3Blocks = 1024;
 static unsigned red_blocks3(size_t n)
 {
     return (unsigned)std::min<size_t>((n + kRedBlock - 1) / kRedBlock, kRed3Blocks);
 }
+
+static unsigned up_blocks3(const m2d_fields3d *f);
+
+// a level on the host while the hierarchy is built
+struct Host3 {
+    int n[3];
+    std::vector<uint8_t> nbm;      // as Mg3Level::nbm
+    std::vector<float> cond[6];    // conductance of each link, to a free neighbour (1) or to a Dirichlet value
+    size_t size() const { return (size_t)n[0] * n[1] * n[2]; }
+    int stride(int q) const  // of link q: -x, -y, -z, +z, +y, +x
+    {
+        const int s[6] = {-n[1] * n[2], -n[2], -1, 1, n[2], n[1] * n[2]};
+        return s[q];
+    }
+    float diag(size_t m) const
+    {
+        float d = 0.f;
+        for (int q = 0; q < 6; q++) d += cond[q].empty() ? 1.f : cond[q][m];
+        return d;
+    }
+};
+
+// Inverse of the coarsest 7-point operator on its free nodes (in place,
+// without pivoting: it is symmetric and positive definite), as a matrix over
+// all its nodes with zeros for the pinned ones
+static bool dense_inverse7(const Host3 &V, std::vector<float> &inv)
+{
+    const size_t n = V.size();
+    std::vector<int> pos(n, -1), id;
+    for (size_t m = 0; m < n; m++)
+        if (!(V.nbm[m] & kNbSelf)) { pos[m] = (int)id.size(); id.push_back((int)m); }
+    const int q = (int)id.size();
+    std::vector<double> a((size_t)q * q, 0.0);
+    for (int r = 0; r < q; r++) {
+        const int m = id[r];
+        a[(size_t)r * q + r] = V.diag(m);
+        for (int l = 0; l < 6; l++)
+            if (V.nbm[m] >> l & 1) a[(size_t)r * q + pos[m + V.stride(l)]] = -1.0;
+    }
+    for (int c = 0; c < q; c++) {
+        double *rc = &a[(size_t)c * q];
+        if (!(rc[c] > 1e-300)) return false;
+        const double d = 1.0 / rc[c];
+        rc[c] = 1.0;
+        for (int t = 0; t < q; t++) rc[t] *= d;
+        for (int r = 0; r < q; r++) {
+            if (r == c) continue;
+            double *rr = &a[(size_t)r * q];
+            const double f = rr[c];
+            if (f == 0.0) continue;
+            rr[c] = 0.0;
+            for (int t = 0; t < q; t++) rr[t] -= f * rc[t];
+        }
+    }
+    inv.assign(n * n, 0.f);
+    for (int r = 0; r < q; r++)
+        for (int c = 0; c < q; c++) inv[(size_t)id[r] * n + id[c]] = (float)a[(size_t)r * q + c];
+    return true;
+}
+
+// Coarse level of F: node I is free where fine node 2I is, faces are pinned.
+// An even side of f nodes gets f / 2 + 1 coarse ones, the last of them one
+// fine node past the grid: its neighbours then lie one node too far from the
+// wall on every level, where f / 2 nodes would bring the wall 2^l - 1 nodes
+// closer on level l.  A link that meets a Dirichlet node halfway (the fine
+// node between two coarse ones, or a shorter distance taken over from the
+// finer level) ends there, with the conductance 1 / (distance in coarse
+// spacings) to its value, so electrodes keep their size on coarse levels.
+// On a quadrupole trap of 64^3 the two bring the CG's residual per iteration
+// down by 9 instead of 4 (with the one sweep of this V-cycle), and by 20 with
+// two sweeps.
+static Host3 coarsen3(const Host3 &F)
+{
+    Host3 C;
+    for (int d = 0; d < 3; d++) C.n[d] = F.n[d] / 2 + 1;
+    C.nbm.assign(C.size(), kNbSelf);
+    for (auto &c : C.cond) c.assign(C.size(), 1.f);
+    for (int I = 0; I < C.n[0]; I++)
+        for (int J = 0; J < C.n[1]; J++)
+            for (int K = 0; K < C.n[2]; K++) {
+                const size_t M = ((size_t)I * C.n[1] + J) * C.n[2] + K;
+                uint8_t bits = (I + J + K) & 1 ? kNbBlack : 0;
+                const bool face = I == 0 || J == 0 || K == 0 || I == C.n[0] - 1 || J == C.n[1] - 1 || K == C.n[2] - 1;
+                const size_t m = ((size_t)(2 * I) * F.n[1] + 2 * J) * F.n[2] + 2 * K;
+                if (face || (F.nbm[m] & kNbSelf)) {
+                    C.nbm[M] = bits | kNbSelf;
+                    continue;
+                }
+                for (int q = 0; q < 6; q++) {
+                    auto cond = [&](size_t at) { return F.cond[q].empty() ? 1.f : F.cond[q][at]; };
+                    if (!(F.nbm[m] >> q & 1)) {
+                        C.cond[q][M] = 2.f * cond(m);
+                    } else {
+                        const size_t mid = m + F.stride(q);
+                        if (F.nbm[mid] >> q & 1) bits |= (uint8_t)(1u << q);
+                        else C.cond[q][M] = 2.f * cond(mid) / (1.f + cond(mid));
+                    }
+                }
+                C.nbm[M] = bits;
+            }
+    return C;
+}
+
+constexpr size_t kCoarsest3 = 800;      // coarsening stops at this many nodes (9^3 = 729 and fewer)
+constexpr int kCoarseDenseMax = 1024;   // nodes for the dense coarsest solve
+constexpr int kCoarseSweeps = 40;       // symmetric RB-GS sweeps otherwise
+
+// tiles of the finest and of the other levels (see k3_down)
+constexpr size_t kLargeTiles3 = 1 << 20;
+
+static int mg3_setup(m2d_fields3d *f, const std::vector<uint8_t> &mask)
+{
+    std::vector<Host3> lv(1);
+    {
+        Host3 &V = lv[0];
+        V.n[0] = f->nx; V.n[1] = f->ny; V.n[2] = f->nz;
+        V.nbm.resize(f->n);
+        auto pinned = [&](size_t m) { return mask[m] == M2D_FIXED || mask[m] == M2D_FIXED_RF; };
+        size_t m = 0;
+        for (int i = 0; i < f->nx; i++)
+            for (int j = 0; j < f->ny; j++)
+                for (int k = 0; k < f->nz; k++, m++) {
+                    uint8_t bits = (i + j + k) & 1 ? kNbBlack : 0;
+                    if (pinned(m)) bits |= kNbSelf;
+                    else  // a free node never sits on a face (checked at creation)
+                        for (int q = 0; q < 6; q++)
+                            if (!pinned(m + V.stride(q))) bits |= (uint8_t)(1u << q);
+                    V.nbm[m] = bits;
+                }
+    }
+    // down to kCoarsest3 nodes, or to a side that cannot be halved
+    while (lv.back().size() > kCoarsest3 && lv.back().n[0] >= 5 && lv.back().n[1] >= 5 && lv.back().n[2] >= 5)
+        lv.push_back(coarsen3(lv.back()));
+    const size_t L = lv.size();
+    M2D_CHECK(L <= (size_t)kMaxLevels3, M2D_ERR_BAD_ARG, "Fields3D: %d multigrid levels", (int)L);
+    f->lv.resize(L);
+    std::vector<float> di;
+    for (size_t l = 0; l < L; l++) {
+        Mg3Level &V = f->lv[l];
+        const Host3 &H = lv[l];
+        V.nx = H.n[0]; V.ny = H.n[1]; V.nz = H.n[2];
+        V.n = H.size();
+        M2D_TRY(dmalloc3((void **)&V.nbm, V.n));
+        M2D_HIP(hipMemcpy(V.nbm, H.nbm.data(), V.n, hipMemcpyHostToDevice));
+        if (l == 0) continue;
+        di.resize(V.n);
+        for (size_t m = 0; m < V.n; m++) di[m] = 1.f / H.diag(m);
+        M2D_TRY(dmalloc3((void **)&V.di, sizeof(float) * V.n));
+        M2D_TRY(dmalloc3((void **)&V.x, sizeof(float) * V.n));
+        M2D_TRY(dmalloc3((void **)&V.b, sizeof(float) * V.n));
+        M2D_HIP(hipMemcpy(V.di, di.data(), sizeof(float) * V.n, hipMemcpyHostToDevice));
+        // the descent's tiles need not cover the last, pinned nodes
+        M2D_HIP(hipMemset(V.b, 0, sizeof(float) * V.n));
+    }
+    f->coarse_dense = lv.back().size() <= (size_t)kCoarseDenseMax;
+    if (f->coarse_dense) {
+        std::vector<float> inv;
+        M2D_CHECK(dense_inverse7(lv.back(), inv), M2D_ERR_BAD_ARG, "Fields3D: coarsest multigrid operator is singular");
+        M2D_TRY(dmalloc3((void **)&f->coarse_inv, sizeof(float) * inv.size()));
+        M2D_HIP(hipMemcpy(f->coarse_inv, inv.data(), sizeof(float) * inv.size(), hipMemcpyHostToDevice));
+    }
+    const size_t n = f->n;
+    for (float **q : {&f->pr, &f->pz, &f->pp, &f->pp2, &f->pq, &f->pe}) M2D_TRY(dmalloc3((void **)q, sizeof(float) * n));
+    // 16 scalars, then the solve's control block
+    M2D_TRY(dmalloc3((void **)&f->dots, sizeof(double) * 32));
+    M2D_HIP(hipHostMalloc((void **)&f->h_dots, sizeof(double) * 32));
+    // up to three sums per block of the fused reductions, one per tile of the ascent
+    f->npartial = (int)std::max({red_blocks3(n), up_blocks3(f), 3 * Cols3{f->nx, f->ny, f->nz}.blocks()});
+    M2D_TRY(dmalloc3((void **)&f->partial, sizeof(double) * f->npartial));
+    M2D_TRY(dmalloc3((void **)&f->ticket, sizeof(unsigned int) * kTicketWords));
+    M2D_HIP(hipMemset(f->ticket, 0, sizeof(unsigned int) * kTicketWords));
+    return M2D_OK;
+}
+
+static unsigned blocks_for(size_t n) { return (unsigned)((n + 255) / 256); }
+
+static dim3 tiles3(const Mg3Level &V, int ti, int tj, int tk)
+{
+    return dim3((unsigned)((V.nz + tk - 1) / tk), (unsigned)((V.ny + tj - 1) / tj), (unsigned)((V.nx + ti - 1) / ti));
+}
+
+// (the levels below the finest always take the small tiles)
+static dim3 tiles3(const Mg3Level &V)
+{
+    return !V.di && V.n >= kLargeTiles3 ? tiles3(V, 8, 8, 64) : tiles3(V, 4, 8, 32);
+}
+
+static unsigned up_blocks3(const m2d_fields3d *f)
+{
+    const dim3 g = tiles3(f->lv[0]);
+    return g.x * g.y * g.z;
+}
+
+template <bool FINEST>
+static void launch_down3(const Mg3Level &V, const Mg3Level &C, const float *b, hipStream_t s, const int *stop)
+{
+    auto go = [&](auto kern, int threads) {
+        kern<<<tiles3(V), threads, 0, s>>>(V.nbm, V.di, b, V.nx, V.ny, V.nz, C.b, C.nbm, C.nx, C.ny, C.nz, stop);
+    };
+    if (FINEST && V.n >= kLargeTiles3) go(k3_down<8, 8, 64, 512, true>, 512);
+    else go(k3_down<4, 8, 32, 256, FINEST>, 256);
+}
+
+template <bool FINEST>
+static void launch_up3(const Mg3Level &V, const Mg3Level &C, const float *b, float *out, hipStream_t s,
+                       const int *stop, double *partial = nullptr, unsigned int *ticket = nullptr,
+                       double *dot = nullptr, int fin = 0)
+{
+    auto go = [&](auto kern, int threads) {
+        kern<<<tiles3(V), threads, 0, s>>>(V.nbm, V.di, b, V.nx, V.ny, V.nz, C.x, C.nx, C.ny, C.nz, out, partial,
+                                           ticket, dot, fin, stop);
+    };
+    if (FINEST && V.n >= kLargeTiles3) go(k3_up<8, 8, 64, 512, true, true>, 512);
+    else go(k3_up<4, 8, 32, 256, FINEST, FINEST>, 256);
+}
+
+// out = V-cycle of rhs and dot = rhs.out
+static int vcycle3(m2d_fields3d *f, const float *rhs, float *out, double *dot, const int *stop)
+{
+    hipStream_t s = f->ctx->stream;
+    const int L = (int)f->lv.size();
+    Mg3Level &Z = f->lv[L - 1];
+    for (int l = 0; l < L - 1; l++) {
+        if (l == 0) launch_down3<true>(f->lv[0], f->lv[1], rhs, s, stop);
+        else launch_down3<false>(f->lv[l], f->lv[l + 1], f->lv[l].b, s, stop);
+    }
+    const float *zb = L == 1 ? rhs : Z.b;
+    float *zx = L == 1 ? out : Z.x;
+    if (f->coarse_dense) {
+        k3_dense<<<(unsigned)((Z.n + 3) / 4), 256, 0, s>>>(f->coarse_inv, zb, zx, (int)Z.n, stop);
+    } else if (L > 1) {
+        k3_sweeps<<<1, kCoarseThreads, 0, s>>>(Z.nbm, Z.di, zb, zx, Z.ny, Z.nz, (int)Z.n, kCoarseSweeps, stop);
+    } else {
+        const dim3 g((unsigned)(((Z.nz + 1) / 2 + kRbgsX - 1) / kRbgsX), (unsigned)((Z.ny + kRbgsY - 1) / kRbgsY),
+                     (unsigned)Z.nx);
+        k3_zero<<<blocks_for(Z.n), 256, 0, s>>>(out, Z.n, stop);
+        for (int h = 0; h < 2 * kCoarseSweeps; h++)
+            k3_rbgs<<<g, dim3(kRbgsX, kRbgsY), 0, s>>>(Z.nbm, out, rhs, Z.nx, Z.ny, Z.nz,
+                                                       h < kCoarseSweeps ? h & 1 : ~h & 1, stop);
+    }
+    for (int l = L - 2; l >= 1; l--) launch_up3<false>(f->lv[l], f->lv[l + 1], f->lv[l].b, f->lv[l].x, s, stop);
+    if (L > 1) {
+        reduce_launch<1>(up_blocks3(f), f->partial, dot, s, [&](int fin) {
+            launch_up3<true>(f->lv[0], f->lv[1], rhs, out, s, stop, f->partial, f->ticket, dot, fin);
+        }, stop);
+    } else {
+        const unsigned rb = red_blocks3(f->n);
+        reduce_launch<1>(rb, f->partial, dot, s, [&](int fin) {
+            k_dot_fin<<<rb, kRedBlock, 0, s>>>(rhs, out, f->n, f->partial, f->ticket, dot, fin, stop);
+        }, stop);
+    }
+    M2D_HIP(hipGetLastError());
+    return M2D_OK;
+}
+
+static SolveCtl *solve_ctl3(m2d_fields3d *f) { return (SolveCtl *)(f->dots + 16); }
 
 // Iterations from + 1 .. to of the open FP32 PCG pass on A' e = d (d in pr,
 // e in pe), from 0: the pass's start; every launch stops with the pass
@@ -1396,32 +1392,30 @@ static int queue_pcg3(m2d_fields3d *f, int from, int to, int &cur)
     const size_t n = f->n;
     const unsigned rb = red_blocks3(n);
     const Mg3Level &V = f->lv[0];
+    const Cols3 g{V.nx, V.ny, V.nz};
     SolveCtl *ctl = solve_ctl3(f);
     const int *stop = &ctl->stop_pcg;
     // iteration it's direction goes to P[it & 1], the previous one's is read from the other
     float *const P[2] = {f->pp, f->pp2};
     if (from == 0) {
-        M2D_TRY(vcycle3(f, f->pr, f->pz, stop));
-        reduce_launch<1>(rb, f->partial, f->dots, s, [&](int fin) {
-            k_dot_fin<<<rb, kRedBlock, 0, s>>>(f->pr, f->pz, n, f->partial, f->ticket, f->dots, fin, stop);
-        }, stop);
+        M2D_TRY(vcycle3(f, f->pr, f->pz, f->dots, stop));
         cur = 0;
     }
     for (int it = from + 1; it <= to; it++) {
         if (it > 1) {
-            M2D_TRY(vcycle3(f, f->pr, f->pz, stop));
-            reduce_launch<1>(rb, f->partial, f->dots + 4 * (cur ^ 1), s, [&](int fin) {
-                k_dot_fin<<<rb, kRedBlock, 0, s>>>(f->pr, f->pz, n, f->partial, f->ticket, f->dots + 4 * (cur ^ 1),
-                                                   fin, stop);
-            }, stop);
+            M2D_TRY(vcycle3(f, f->pr, f->pz, f->dots + 4 * (cur ^ 1), stop));
             cur ^= 1;
         }
         const float *pold = P[(it - 1) & 1];
         float *pnew = P[it & 1];
-        reduce_launch<1>(rb, f->partial, f->dots + 1, s, [&](int fin) {
-            k3_dir_apply_dot<<<rb, kRedBlock, 0, s>>>(V.nbm, f->pz, pold, pnew, f->pq, f->dots + 4 * cur,
-                                                      f->dots + 4 * (cur ^ 1), it == 1, V.nx, V.ny, V.nz, f->partial,
-                                                      f->ticket, f->dots + 1, fin, stop);
+        reduce_launch<1>(g.blocks(), f->partial, f->dots + 1, s, [&](int fin) {
+            auto go = [&](auto kern) {
+                kern<<<g.grid(), kRedBlock, 0, s>>>(g, V.nbm, f->pz, pold, pnew, f->pq, f->dots + 4 * cur,
+                                                    f->dots + 4 * (cur ^ 1), it == 1, f->partial, f->ticket,
+                                                    f->dots + 1, fin, stop);
+            };
+            if (g.di() == 8) go(k3_dir_apply_dot<8>);
+            else go(k3_dir_apply_dot<4>);
         }, stop);
         reduce_launch<1>(rb, f->partial, f->dots + 2, s, [&](int fin) {
             k_cg_update_dot<<<rb, kRedBlock, 0, s>>>(f->pe, f->pr, pnew, f->pq, f->dots + 4 * cur, f->dots + 1, n,
@@ -1433,24 +1427,34 @@ static int queue_pcg3(m2d_fields3d *f, int from, int to, int &cur)
     return M2D_OK;
 }
 
-// the FP64 residual of u, its norms, and the refinement's decision on them
-static void queue_residual3(m2d_fields3d *f, double tol)
+// the FP64 residual of u, its norms, and the refinement's decision on them;
+// first: the solve's first one, which starts a fresh control block
+static void queue_residual3(m2d_fields3d *f, double tol, bool first)
 {
     hipStream_t s = f->ctx->stream;
-    const unsigned rb = red_blocks3(f->n);
+    const Cols3 g{f->nx, f->ny, f->nz};
     SolveCtl *ctl = solve_ctl3(f);
-    const int *stop = &ctl->stop_outer;
-    const CtlEval post{ctl, tol, kMaxOuter};
-    reduce_launch<3>(rb, f->partial, f->dots + 8, s, [&](int fin) {
-        k3_residual64_fin<<<rb, kRedBlock, 0, s>>>(f->mask, f->rho, f->u, f->nx, f->ny, f->nz, f->r64, f->pr,
-                                                   f->partial, f->ticket, f->dots + 8, fin, stop, post);
-    }, stop, post);
+    const int *stop = first ? nullptr : &ctl->stop_outer;
+    const CtlEval eval{ctl, tol, kMaxOuter};
+    auto go = [&](auto kern, auto post) {
+        reduce_launch<3>(g.blocks(), f->partial, f->dots + 8, s, [&](int fin) {
+            kern<<<g.grid(), kRedBlock, 0, s>>>(g, f->mask, f->rho, f->u, f->pr, f->partial, f->ticket, f->dots + 8,
+                                                fin, stop, post);
+        }, stop, post);
+    };
+    if (g.di() == 8) {
+        if (first) go(k3_residual64_fin<8, CtlFirst>, CtlFirst{eval});
+        else go(k3_residual64_fin<8, CtlEval>, eval);
+    } else {
+        if (first) go(k3_residual64_fin<4, CtlFirst>, CtlFirst{eval});
+        else go(k3_residual64_fin<4, CtlEval>, eval);
+    }
 }
 
 static int build_tables3(m2d_fields3d *f)
 {
-    k3_tables<<<blocks_for(f->n), 256, 0, f->ctx->stream>>>(f->u, f->nx, f->ny, f->nz, f->idx, f->idy, f->idz,
-                                                            f->tx, f->ty, f->tz);
+    k3_tables<<<dim3((unsigned)((f->nz + 63) / 64), (unsigned)((f->ny + 3) / 4), (unsigned)f->nx), dim3(64, 4), 0,
+                f->ctx->stream>>>(f->u, f->nx, f->ny, f->nz, f->idx, f->idy, f->idz, f->tx, f->ty, f->tz);
     M2D_HIP(hipGetLastError());
     return M2D_OK;
 }
@@ -1512,11 +1516,11 @@ static void free3(m2d_fields3d *f)
 {
     for (void *q : {(void *)f->mask, (void *)f->cellfree, (void *)f->voltage, (void *)f->u, (void *)f->rho,
                     (void *)f->tx, (void *)f->ty, (void *)f->tz, (void *)f->coarse_inv, (void *)f->pr,
-                    (void *)f->pz, (void *)f->pp, (void *)f->pp2, (void *)f->pq, (void *)f->pe, (void *)f->r64,
-                    (void *)f->dots, (void *)f->partial, (void *)f->coarse_invT, (void *)f->ticket})
+                    (void *)f->pz, (void *)f->pp, (void *)f->pp2, (void *)f->pq, (void *)f->pe,
+                    (void *)f->dots, (void *)f->partial, (void *)f->ticket})
         if (q) (void)hipFree(q);
     for (Mg3Level &V : f->lv)
-        for (void *q : {(void *)V.dir, (void *)V.nbm, (void *)V.x, (void *)V.b, (void *)V.r})
+        for (void *q : {(void *)V.nbm, (void *)V.di, (void *)V.x, (void *)V.b})
             if (q) (void)hipFree(q);
     if (f->h_dots) (void)hipHostFree(f->h_dots);
 }
@@ -1634,13 +1638,12 @@ int m2d_fields3d_solve(m2d_fields3d *f, double tol, m2d_solve_info *info)
     if (tol <= 0) tol = 1e-10;
     SolveCtl *ctl = solve_ctl3(f);
     SolveCtl *h = (SolveCtl *)(f->h_dots + 16);
-    k_ctl_init<<<1, 64, 0, s>>>(ctl);
-    queue_residual3(f, tol);
+    queue_residual3(f, tol, true);
     M2D_TRY(queue_refinement(
         s, ctl, h, f->dots, f->est, tol, 80,
         [&](int from, int to, int &cur) { return queue_pcg3(f, from, to, cur); },
         [&] { k3_add_correction<<<gb, 256, 0, s>>>(f->mask, f->u, f->pe, n, &ctl->no_add); },
-        [&] { queue_residual3(f, tol); }));
+        [&] { queue_residual3(f, tol, false); }));
     const int outer = h->outer;
     const double rel = h->rel;
     if (info) { info->outer_iters = outer; info->inner_iters = h->iters; info->rel_residual = rel; }

@@ -346,11 +346,30 @@ __global__ void __launch_bounds__(kRedBlock) k_cg_update_dot(float *e, float *r,
     double v[1] = {0};
     const double den = *pq;
     const float alpha = den != 0.0 ? (float)(*rz / den) : 0.f;
-    for (size_t k = (size_t)blockIdx.x * kRedBlock + threadIdx.x; k < n; k += (size_t)gridDim.x * kRedBlock) {
-        e[k] = fmaf(alpha, p[k], first ? 0.f : e[k]);
-        const float rk = fmaf(-alpha, q[k], r[k]);
-        r[k] = rk;
+    // four nodes a thread as one 16-byte word of each array (hipMalloc's
+    // alignment), the last n % 4 one by one
+    const size_t n4 = n / 4, t0 = (size_t)blockIdx.x * kRedBlock + threadIdx.x;
+    auto one = [&](float &ek, float &rk, float pk, float qk) {
+        ek = fmaf(alpha, pk, first ? 0.f : ek);
+        rk = fmaf(-alpha, qk, rk);
         v[0] += (double)rk * rk;
+    };
+    for (size_t k = t0; k < n4; k += (size_t)gridDim.x * kRedBlock) {
+        const float4 p4 = ((const float4 *)p)[k], q4 = ((const float4 *)q)[k];
+        float4 r4 = ((float4 *)r)[k], e4 = first ? make_float4(0.f, 0.f, 0.f, 0.f) : ((float4 *)e)[k];
+        one(e4.x, r4.x, p4.x, q4.x);
+        one(e4.y, r4.y, p4.y, q4.y);
+        one(e4.z, r4.z, p4.z, q4.z);
+        one(e4.w, r4.w, p4.w, q4.w);
+        ((float4 *)e)[k] = e4;
+        ((float4 *)r)[k] = r4;
+    }
+    if (t0 < n % 4) {
+        const size_t k = 4 * n4 + t0;
+        float ek = first ? 0.f : e[k], rk = r[k];
+        one(ek, rk, p[k], q[k]);
+        e[k] = ek;
+        r[k] = rk;
     }
     finish_sums<1>(v, partial, ticket, out, fin, post);
 }
@@ -907,41 +926,6 @@ __global__ void __launch_bounds__(kCoarseThreads) k_vcycle_coarse_lds(CoarseArgs
     for (int k = threadIdx.x; k < n; k += kCoarseThreads) A.x[k] = xa[k];
 }
 
-// dense solve x = A^-1 b with the transposed inverse, one workgroup of
-// kCoarseThreads: kDenseParts threads per row (the same sums as the dense
-// step of k_vcycle_coarse); dynamic LDS of (1 + kDenseParts) n words
-__global__ void __launch_bounds__(kCoarseThreads) k_dense_solve(const float *invT, const float *b, float *x, int n,
-                                                                 const int *stop)
-{
-    if (stopped(stop)) return;
-    extern __shared__ float sb[];
-    float *part = sb + n;
-    for (int k = threadIdx.x; k < n; k += kCoarseThreads) sb[k] = b[k];
-    __syncthreads();
-    const int len = (n + kDenseParts - 1) / kDenseParts;
-    for (int t = threadIdx.x; t < n * kDenseParts; t += kCoarseThreads) {
-        const int row = t % n, p = t / n;
-        const int c0 = p * len, c1 = min(n, c0 + len);
-        float s = 0.f;
-        int c = c0;
-        for (; c + 8 <= c1; c += 8) {
-            float a[8];
-#pragma unroll
-            for (int q = 0; q < 8; q++) a[q] = invT[(size_t)(c + q) * n + row];
-#pragma unroll
-            for (int q = 0; q < 8; q++) s = fmaf(a[q], sb[c + q], s);
-        }
-        for (; c < c1; c++) s = fmaf(invT[(size_t)c * n + row], sb[c], s);
-        part[p * n + row] = s;
-    }
-    __syncthreads();
-    for (int row = threadIdx.x; row < n; row += kCoarseThreads) {
-        float s = part[row];
-        for (int p = 1; p < kDenseParts; p++) s += part[p * n + row];
-        x[row] = s;
-    }
-}
-
 // ------------------------------------------------------------------ host: hierarchy
 static void p1d(int i, int nc, int I[2], float w[2], int &cnt)
 {
@@ -1074,8 +1058,8 @@ static int solve_setup(m2d_fields2d *f)
     M2D_TRY(dmalloc((void **)&mg.r64, sizeof(double) * n));
     // 16 device scalars, then the solve's control block (SolveCtl)
     M2D_TRY(dmalloc((void **)&mg.dots, sizeof(double) * 32));
-    M2D_TRY(dmalloc((void **)&mg.ticket, sizeof(unsigned int)));
-    M2D_HIP(hipMemset(mg.ticket, 0, sizeof(unsigned int)));
+    M2D_TRY(dmalloc((void **)&mg.ticket, sizeof(unsigned int) * kTicketWords));
+    M2D_HIP(hipMemset(mg.ticket, 0, sizeof(unsigned int) * kTicketWords));
     M2D_HIP(hipHostMalloc((void **)&mg.h_dots, sizeof(double) * 32));
     mg.npartial = (int)std::min<size_t>((n + 255) / 256, 65536);
     // up to three sums per block of the fused reductions
@@ -1278,12 +1262,6 @@ static int vcycle(m2d_fields2d *f, const float *rhs, float *out, const int *stop
 
 // fused-reduction launch shape over the finest level
 static unsigned red_blocks(size_t n) { return (unsigned)((n + kRedBlock - 1) / kRedBlock); }
-
-__global__ void k_ctl_init(SolveCtl *c)
-{
-    if (threadIdx.x) return;
-    ctl_reset(c);
-}
 
 // opens a CG pass on the FP32 residual d (|d|^2 = dots[10])
 __global__ void k_ctl_open(SolveCtl *c, const double *dots, double tol)

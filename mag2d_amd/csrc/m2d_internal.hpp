@@ -205,7 +205,6 @@ __global__ void k_dot_fin(const float *a, const float *b, size_t n, double *part
                           double *out, int fin, const int *stop);
 constexpr int kCoarseThreads = 1024;
 constexpr int kDenseParts = 4;  // threads per row of the dense coarsest solves
-__global__ void k_dense_solve(const float *invT, const float *b, float *x, int n, const int *stop);
 int ensure_acc(m2d_ctx *ctx, size_t n);
 int fill_bytes(m2d_ctx *ctx, void *dst, int value, size_t bytes);
 int zero_words(m2d_ctx *ctx, unsigned long long *dst, size_t n);
@@ -317,15 +316,14 @@ struct SolveEst {
 };
 static_assert(kMaxPasses == 13, "SolveEst::iters initialiser");
 
-__global__ void k_ctl_init(SolveCtl *c);
 __global__ void k_ctl_open(SolveCtl *c, const double *dots, double tol);
 __global__ void k_ctl_end(SolveCtl *c, int max_iters);
 __global__ void k_ctl_resume(SolveCtl *c);
 __global__ void k_ctl_close(SolveCtl *c);
 
 // FP64 iterative refinement over FP32 CG passes, queued under SolveCtl.  The
-// caller has queued the right-hand side, k_ctl_init and resid() (the FP64
-// residual, its norms and CtlEval).  Passes are queued as many as the
+// caller has queued the first residual (with the right-hand side, its norms and
+// CtlFirst).  Passes are queued as many as the
 // last solve took, each with one CG iteration more than its counterpart
 // took then (the last pass of a refinement needs far fewer than the first);
 // the control block is read once after them.  A pass that needs more
@@ -549,26 +547,33 @@ inline int grid_for(int64_t n, int per_thread, int block = kBlock)
 // are then summed in block order, by sum_partials, either in a kernel of its
 // own (k_sum_partials) or, with fin set, by the block that takes the last
 // ticket, which writes out[] and resets the ticket: no extra launch, which
-// pays on small grids.  The last-ticket path costs each block a device-scope
-// fence, so it is for launches of at most kFinBlocks blocks.  Both paths add
-// in the same order and give the same bits on every run.  Blocks of
-// kRedBlock threads; every thread of every block must call finish_sums.
+// pays on small grids.  The partials cross the XCDs as device-scope atomic
+// stores and loads: a device-scope fence instead would write back the whole
+// L2, with everything the kernel just stored, once a block.  Tickets at one
+// address are served 8 ns apart (1024 blocks waited 8 us for theirs), so
+// blocks take one of kTicketWays counters, each on its own cache line, and the
+// last block of each takes one of the final counter.  kFinBlocks: past it a
+// launch of its own for the sums (about 3 us) is cheaper.  Both paths give the
+// same bits on every run.  ticket: kTicketWords words, 0 between launches.  Every thread of every block must call
+// finish_sums (blocks of BLOCK threads).
 constexpr int kRedBlock = 256;
-constexpr unsigned kFinBlocks = 256;
+constexpr unsigned kFinBlocks = 1024;
+constexpr unsigned kTicketWays = 16, kTicketStride = 32, kTicketWords = (1 + kTicketWays) * kTicketStride;
 
-template <int NV>
+template <int NV, int BLOCK = kRedBlock>
 __device__ __forceinline__ void sum_partials(const double *partial, unsigned nb, double *out)
 {
-    __shared__ double sh[NV][kRedBlock / 64];
+    __shared__ double sh[NV][BLOCK / 64];
     const int w = threadIdx.x >> 6;
     double t[NV];
 #pragma unroll
     for (int q = 0; q < NV; q++) t[q] = 0;
     // unrolled so that several loads are in flight; the adds keep block order
 #pragma unroll 8
-    for (unsigned b = threadIdx.x; b < nb; b += kRedBlock)
+    for (unsigned b = threadIdx.x; b < nb; b += BLOCK)
 #pragma unroll
-        for (int q = 0; q < NV; q++) t[q] += partial[NV * b + q];
+        for (int q = 0; q < NV; q++)
+            t[q] += __hip_atomic_load(partial + NV * b + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
     for (int q = 0; q < NV; q++) {
         for (int o = 32; o > 0; o >>= 1) t[q] += __shfl_down(t[q], o);
@@ -579,7 +584,7 @@ __device__ __forceinline__ void sum_partials(const double *partial, unsigned nb,
 #pragma unroll
         for (int q = 0; q < NV; q++) {
             double s = 0;
-            for (int k = 0; k < kRedBlock / 64; k++) s += sh[q][k];
+            for (int k = 0; k < BLOCK / 64; k++) s += sh[q][k];
             out[q] = s;
         }
     }
@@ -595,13 +600,16 @@ __global__ void __launch_bounds__(kRedBlock) k_sum_partials(const double *partia
     if (threadIdx.x == 0) post(out);
 }
 
-template <int NV, class Post = NoPost>
+template <int NV, int BLOCK = kRedBlock, class Post = NoPost>
 __device__ __forceinline__ void finish_sums(double (&v)[NV], double *partial, unsigned int *ticket, double *out,
                                             int fin, Post post = Post{})
 {
-    __shared__ double sh[NV][kRedBlock / 64];
+    __shared__ double sh[NV][BLOCK / 64];
     __shared__ bool last;
     const int w = threadIdx.x >> 6;
+    // blocks of a 3D launch in index order, x fastest
+    const unsigned bid = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    const unsigned nb = gridDim.x * gridDim.y * gridDim.z;
 #pragma unroll
     for (int q = 0; q < NV; q++) {
         for (int o = 32; o > 0; o >>= 1) v[q] += __shfl_down(v[q], o);
@@ -612,19 +620,26 @@ __device__ __forceinline__ void finish_sums(double (&v)[NV], double *partial, un
 #pragma unroll
         for (int q = 0; q < NV; q++) {
             double t = 0;
-            for (int k = 0; k < kRedBlock / 64; k++) t += sh[q][k];
-            partial[NV * blockIdx.x + q] = t;
+            for (int k = 0; k < BLOCK / 64; k++) t += sh[q][k];
+            __hip_atomic_store(partial + NV * bid + q, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (fin) {
-            __threadfence();
-            last = atomicAdd(ticket, 1u) == gridDim.x - 1;
+            // the partials are written through to where every XCD sees them
+            // and have arrived there before the ticket is taken
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            const unsigned way = bid % kTicketWays, ways = nb < kTicketWays ? nb : kTicketWays;
+            unsigned int *mine = ticket + (1 + way) * kTicketStride;
+            last = atomicAdd(mine, 1u) == (nb - way - 1) / kTicketWays;
+            if (last) {
+                *mine = 0u;
+                last = atomicAdd(ticket, 1u) == ways - 1;
+            }
         }
     }
     if (!fin) return;  // uniform: a kernel argument
     __syncthreads();
     if (!last) return;  // uniform over the block
-    __threadfence();
-    sum_partials<NV>(partial, gridDim.x, out);
+    sum_partials<NV, BLOCK>(partial, nb, out);
     if (threadIdx.x == 0) {
         *ticket = 0u;
         post(out);
