@@ -674,6 +674,7 @@ struct PushArgs3 {
     uint32_t *cq;
     unsigned long long *cq_len;
     unsigned long long *acc;
+    int rec;                       // acc holds cell records (untiled deposit, see deposit_buffer)
     unsigned long long *counters;
 };
 
@@ -729,39 +730,64 @@ __device__ __forceinline__ bool cic3(double X, double Y, double Z, const Grid3 &
     return true;
 }
 
-// Segmented sum across the wavefront of the lanes' weights keyed by their
-// cell (a sorted store puts a cell's particles on neighbouring lanes); the
-// last lane of each segment adds its sums to the 64-bit grid.  All 64
-// lanes must call it together.
-__device__ __forceinline__ void wave_deposit3(int cell, const uint32_t w8[8], const Grid3 &g,
-                                              unsigned long long *acc)
+// The deposits of a wavefront's lanes in memory: cell = its lower corner's
+// node (-1: none), w8 its corners' weights.  They pass through LDS (stage:
+// kStage3 words of the wavefront's own) so that round r serves lanes 8 r ..
+// 8 r + 7, eight lanes adding the corners of one particle: an instruction's
+// lanes then fall on 8 records of 64 bytes (or 8 x 4 node rows), not 64 x 8
+// nodes.  In cell order (many lanes of equal cells) the lanes' weights are
+// summed first.  All 64 lanes must call it together.
+constexpr int kStage3 = 64 * 9;
+__device__ __forceinline__ void wave_deposit3(int cell, const uint32_t w8[8], const Grid3 &g, unsigned long long *acc,
+                                              int rec, uint32_t *stage)
 {
     const int lane = __lane_id();
-    const bool valid = cell >= 0;
-    const int key = valid ? cell : -1 - lane;
-    const int prev = __shfl_up(key, 1);
-    const unsigned long long heads = __ballot(lane == 0 || prev != key);
-    const int seg = 63 - __clzll(heads & ((2ull << lane) - 1ull));
-    unsigned long long s[8];
+    const size_t sx = (size_t)g.ny * g.nz;
+    auto corner = [&](int q) { return ((q & 1) ? sx : 0) + (((q >> 1) & 1) ? (size_t)g.nz : 0) + (q >> 2); };
+    if (cells_repeat(cell)) {  // uniform
+        unsigned long long s[8];
 #pragma unroll
-    for (int q = 0; q < 8; q++) s[q] = valid ? w8[q] : 0ull;
+        for (int q = 0; q < 8; q++) s[q] = cell >= 0 ? w8[q] : 0ull;
+        if (segment_sums<8>(cell, s)) {
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-#pragma unroll
-        for (int q = 0; q < 8; q++) {
-            unsigned long long t = __shfl_up(s[q], off);
-            if (lane - off >= seg) s[q] += t;
+            for (int q = 0; q < 8; q++)
+                if (s[q]) atomicAdd(acc + (rec ? (size_t)cell * 8 + q : (size_t)cell + corner(q)), s[q]);
         }
+        return;
     }
-    const bool tail = lane == 63 || ((heads >> (lane + 1)) & 1ull);
-    if (valid && tail) {
-        const size_t sx = (size_t)g.ny * g.nz;
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const size_t m = (size_t)cell + ((q & 1) ? sx : 0) + (((q >> 1) & 1) ? (size_t)g.nz : 0) + (q >> 2);
-            if (s[q]) atomicAdd(acc + m, s[q]);
-        }
+    for (int q = 0; q < 8; q++) stage[lane * 9 + q] = cell >= 0 ? w8[q] : 0u;
+    stage[lane * 9 + 8] = (uint32_t)cell;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int q = lane & 7;
+    const size_t off = rec ? (size_t)q : corner(q);
+    const int mul = rec ? 8 : 1;
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
+        const int src = 8 * r + (lane >> 3);
+        const int c = (int)stage[src * 9 + 8];
+        const uint32_t v = stage[src * 9 + q];
+        if (c >= 0 && v) atomicAdd(acc + ((size_t)c * mul + off), (unsigned long long)v);
     }
+}
+
+// rho += charge * (sum of the records of the 8 cells around the node) *
+// 2^-31; blocks of 64 x 4 nodes (k, j) and a grid of (nz / 64, ny / 4, nx)
+__global__ void __launch_bounds__(256) k3_flush_rec(const unsigned long long *rec, double *rho, double charge, int nx,
+                                                    int ny, int nz)
+{
+    const int i = blockIdx.z, j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.x * 64 + threadIdx.x;
+    if (j >= ny || k >= nz) return;
+    const size_t sx = (size_t)ny * nz, m = (size_t)i * sx + (size_t)j * nz + k;
+    unsigned long long v = 0;
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+        const int a = q & 1, b = (q >> 1) & 1, c = q >> 2;
+        if (i >= a && j >= b && k >= c) v += rec[8 * (m - a * sx - (size_t)b * nz - c) + q];
+    }
+    if (v) rho[m] += charge * ((double)(long long)v * kInvFix);
 }
 
 // mod (mymath.cpp:62-67)
@@ -882,9 +908,10 @@ template <bool DEPOSIT, bool MCC>
 __global__ void __launch_bounds__(256) k_advance3d(PushArgs3 a)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ uint32_t stage[DEPOSIT ? 4 * kStage3 : 1];
     Step3 o;
     if (p < a.n) step3<DEPOSIT, MCC>(a, p, o);
-    if (DEPOSIT) wave_deposit3(o.cell, o.w8, a.g, a.acc);
+    if (DEPOSIT) wave_deposit3(o.cell, o.w8, a.g, a.acc, a.rec, stage + (threadIdx.x >> 6) * kStage3);
     wave_count(&a.counters[CNT_REMOVED], o.removed);
     if (MCC) wave_count(&a.counters[CNT_COLL], o.coll);
     if (__ballot(o.nan_pos) && __lane_id() == 0) raise_flag(a.counters, M2D_FLAG_NAN);
@@ -1010,9 +1037,10 @@ __global__ void __launch_bounds__(256) k_advance_init3d(PushArgs3 a)
 
 // Field3D::accumulate for every live particle
 __global__ void __launch_bounds__(256) k_accumulate3d(const float *xs, const float *ys, const float *zs,
-                                                      int64_t n, Grid3 g, unsigned long long *acc,
+                                                      int64_t n, Grid3 g, unsigned long long *acc, int rec,
                                                       unsigned long long *counters)
 {
+    __shared__ uint32_t stage[4 * kStage3];
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int cell = -1;
     uint32_t w8[8];
@@ -1025,7 +1053,7 @@ __global__ void __launch_bounds__(256) k_accumulate3d(const float *xs, const flo
             bad = true;
         }
     }
-    wave_deposit3(cell, w8, g, acc);
+    wave_deposit3(cell, w8, g, acc, rec, stage + (threadIdx.x >> 6) * kStage3);
     if (__ballot(bad) && __lane_id() == 0) raise_flag(counters, M2D_FLAG_OUT_OF_RANGE);
 }
 
@@ -1509,7 +1537,26 @@ static void fill_args3(PushArgs3 &a, m2d_fields3d *f, const m2d_species2d *s, co
     a.step = s->niter;
     a.mcc = nullptr; a.cq = nullptr; a.cq_len = nullptr;
     a.acc = nullptr;
+    a.rec = 0;
     a.counters = f->ctx->counters;
+}
+
+// Records pay from one particle per eight nodes on: 295k particles took 78 us
+// of atomics at the nodes against 15 us on 128^3, and 172 against 16 us on
+// 64^3; the records' flush and clearing, 64 bytes a node to read and to
+// write, take 33 and about 25 us on 96 x 112 x 128 (1.4M nodes).  On grids whose records stay within
+// 1 GiB.
+static bool use_rec3(int64_t particles, size_t nodes)
+{
+    return (size_t)particles >= nodes / 8 && particles >= 16384 && nodes <= (1u << 24);
+}
+
+static int flush_rec3(m2d_ctx *ctx, double *rho, double charge, int nx, int ny, int nz)
+{
+    k3_flush_rec<<<dim3((unsigned)((nz + 63) / 64), (unsigned)((ny + 3) / 4), (unsigned)nx), dim3(64, 4), 0,
+                   ctx->stream>>>((const unsigned long long *)ctx->rec.ptr, rho, charge, nx, ny, nz);
+    M2D_HIP(hipGetLastError());
+    return rec_done(ctx, (size_t)nx * ny * nz, 8);
 }
 
 static void free3(m2d_fields3d *f)
@@ -1661,12 +1708,15 @@ int m2d_accumulate_3d(m2d_ctx *ctx, const m2d_grid3d *g, const m2d_particles3d *
     M2D_TRY(check_grid3(g));
     M2D_TRY(check_parts3(p));
     const size_t n = (size_t)g->nx * g->ny * g->nz;
-    M2D_TRY(ensure_acc(ctx, n));
+    int rec = use_rec3(p->n, n);
+    unsigned long long *acc;
+    M2D_TRY(deposit_buffer(ctx, n, 8, rec, acc));
     if (p->n > 0) {
         k_accumulate3d<<<blocks_for((size_t)p->n), 256, 0, ctx->stream>>>(
-            p->x, p->y, p->z, p->n, grid3_of(*g), (unsigned long long *)ctx->acc.ptr, ctx->counters);
+            p->x, p->y, p->z, p->n, grid3_of(*g), acc, rec, ctx->counters);
         M2D_HIP(hipGetLastError());
     }
+    if (rec) return flush_rec3(ctx, rho, charge, g->nx, g->ny, g->nz);
     k_flush<<<blocks_for(n), 256, 0, ctx->stream>>>((unsigned long long *)ctx->acc.ptr, rho, charge, n);
     M2D_HIP(hipGetLastError());
     return M2D_OK;
@@ -1736,14 +1786,14 @@ int m2d_advance_3d(m2d_ctx *ctx, m2d_fields3d *f, const m2d_species2d *s, const 
         a.cq_len = ctx->counters + CNT_QLEN + slot;
         next_len = ctx->counters + CNT_QLEN + (slot ^ 1);
     }
-    if (deposit) {
-        M2D_TRY(ensure_acc(ctx, f->n));
-        a.acc = (unsigned long long *)ctx->acc.ptr;
-    }
     // a store sorted by m2d_sort_3d deposits through per-chunk LDS windows
     const int ntx3 = (f->nx - 2) / kTile3 + 1, nty3 = (f->ny - 2) / kTile3 + 1, ntz3 = (f->nz - 2) / kTile3 + 1;
     const m2d_tiling *T = deposit ? find_tiling(ctx, p->x, p->n) : nullptr;
     if (T && (T->ntx != ntx3 || T->nty != nty3 || T->ntz != ntz3)) T = nullptr;
+    if (deposit) {
+        a.rec = !T && use_rec3(p->n, f->n);
+        M2D_TRY(deposit_buffer(ctx, f->n, 8, a.rec, a.acc));
+    }
     if (p->n > 0) {
         if (T) {
             launch_timed(ctx, use_mcc ? k_advance3d_tiled<true> : k_advance3d_tiled<false>, dim3(T->max_chunks),
@@ -1760,7 +1810,9 @@ int m2d_advance_3d(m2d_ctx *ctx, m2d_fields3d *f, const m2d_species2d *s, const 
             ctx->cq_dirty = false;
         }
     }
-    if (deposit) {
+    if (a.rec) {
+        M2D_TRY(flush_rec3(ctx, rho, s->charge, f->nx, f->ny, f->nz));
+    } else if (deposit) {
         k_flush<<<blocks_for(f->n), 256, 0, ctx->stream>>>(a.acc, rho, s->charge, f->n);
         M2D_HIP(hipGetLastError());
     }

@@ -129,6 +129,8 @@ struct m2d_ctx {
     unsigned long long *counters = nullptr;  // CNT_N device words
     unsigned long long *h_counters = nullptr; // pinned mirror
     m2d::Scratch acc;       // int64 fixed-point deposit grid
+    m2d::Scratch rec;       // int64 cell records of unsorted deposits (see deposit_buffer)
+    bool rec_dirty = false; // a call failed between writing records and clearing them
     m2d::Scratch red;       // reduction partials
     m2d::Scratch tmp;       // general temporaries (compaction offsets)
     m2d::Scratch sortbuf;   // keys, slots and radix-sort temporaries
@@ -197,7 +199,8 @@ __global__ void k_flush(unsigned long long *acc, double *rho, double charge, siz
 __global__ void __launch_bounds__(kBlock) k_accumulate2d(const float *xs, const float *zs, const float *xls,
                                                          const float *zls, int64_t n, int nx, int nz, double idx,
                                                          double idz, double xmin, double zmin,
-                                                         unsigned long long *acc, unsigned long long *counters);
+                                                         unsigned long long *acc, int rec,
+                                                         unsigned long long *counters);
 // device address of the no-allocation entry point's static scratch on the
 // current device, resolved once per device (m2d_noalloc.hip)
 int noalloc_init_device(int device);
@@ -206,6 +209,22 @@ __global__ void k_dot_fin(const float *a, const float *b, size_t n, double *part
 constexpr int kCoarseThreads = 1024;
 constexpr int kDenseParts = 4;  // threads per row of the dense coarsest solves
 int ensure_acc(m2d_ctx *ctx, size_t n);
+// Cell records: an unsorted store's deposits go as 64-bit atomics to memory,
+// where each particle's corners cost a request per cache line they touch.  A
+// record holds the sums of one cell's 4 (3D: 8) corner weights side by side,
+// 32 (64) bytes, and the lanes of a wavefront are dealt so that one
+// instruction adds whole records: one request a particle instead of 4 (8).
+// The flush then gathers each node's sum from the cells around it (integers:
+// the same total as adding at the nodes).  Measured alone, 4.2M particles on
+// a blob of a third of the grid: 128^3 1886 -> 179 us, 512^2 734 -> 277 us.
+// deposit_buffer: with rec the all-zero records of `nodes` cells of `corners`
+// words, else the node grid.  It clears rec, and so chooses the node grid,
+// where the records' memory cannot be had, and in a call that is being
+// captured in a graph (whose replays would keep the address of a buffer that
+// later calls may grow; the node grid is there from the same call before).
+// rec_done: after the flush, clears the records again.
+int deposit_buffer(m2d_ctx *ctx, size_t nodes, int corners, int &rec, unsigned long long *&acc);
+int rec_done(m2d_ctx *ctx, size_t cells, int corners);
 int fill_bytes(m2d_ctx *ctx, void *dst, int value, size_t bytes);
 int zero_words(m2d_ctx *ctx, unsigned long long *dst, size_t n);
 int read_counters(m2d_ctx *ctx);
@@ -499,6 +518,40 @@ __device__ __forceinline__ void drift_pair(float &hi, float &lo, float v, float 
     const float l = lo + (e + dl);
     hi = s + l;
     lo = l - (hi - s);
+}
+
+// lane R of the lane's quad
+template <int R>
+__device__ __forceinline__ uint32_t quad_lane(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, R * 0x55, 0xf, 0xf, true);
+}
+// lanes whose cell is the lane before's: a wavefront of a store in cell order
+// has many, and sums them before the atomics
+__device__ __forceinline__ bool cells_repeat(int cell)
+{
+    const int prev = __shfl_up(cell, 1);
+    return __popcll(__ballot(__lane_id() > 0 && cell >= 0 && prev == cell)) >= 32;
+}
+// segmented inclusive sums over the lanes of equal cells (-1: none); true on
+// the last lane of a segment, whose s then holds its total
+template <int W>
+__device__ __forceinline__ bool segment_sums(int cell, unsigned long long (&s)[W])
+{
+    const int lane = __lane_id();
+    const int key = cell >= 0 ? cell : -1 - lane;
+    const int prev = __shfl_up(key, 1);
+    const unsigned long long heads = __ballot(lane == 0 || prev != key);
+    const int seg = 63 - __clzll(heads & ((2ull << lane) - 1ull));
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+#pragma unroll
+        for (int q = 0; q < W; q++) {
+            const unsigned long long t = __shfl_up(s[q], off);
+            if (lane - off >= seg) s[q] += t;
+        }
+    }
+    return cell >= 0 && (lane == 63 || ((heads >> (lane + 1)) & 1ull));
 }
 
 // wave-aggregated counter increment (one atomic per wavefront)

@@ -55,6 +55,7 @@ struct PushArgs {
     const int4 *sched;             // chunk -> (tile, first slot, end slot)
     const unsigned int *n_chunks;
     int ntz;                       // sort tiles along z
+    int rec;                       // acc holds cell records instead (untiled deposit, see deposit_buffer)
     // gridded B (Fields::B with magnetic_field_const = 0): {Br, Bz} per node
     // of its own grid, null for the constant rotation above
     const float2 *bt;
@@ -167,19 +168,19 @@ __device__ __forceinline__ void deposit_global(unsigned long long *acc, int nz, 
 // Deposits: the tiled pass adds every particle's four weights into its
 // block's LDS window (in a sorted store some lane of a wavefront changes cell
 // at almost every particle, so summing runs first would not save LDS
-// instructions, only add VALU work).  The untiled pass sums them twice before
-// they reach memory: in registers over a thread's run of equal cells, then
-// across the wavefront by a segmented scan over the lanes' last runs (lanes
-// hold consecutive slots, so a wavefront of a sorted store spans a few
-// cells); only the last lane of each segment issues the four 64-bit atomics.
+// instructions, only add VALU work).  The untiled pass adds them in memory
+// (wave_deposit).
 // Two-wavefront blocks with 5 KB of LDS (the deposit window): a launch of
 // a few thousand chunks is mostly resident at once.
 constexpr int kPass = 256;
 constexpr int kRound = kPass * 4;
 static_assert(kRound == kRound2, "the tile schedule orders chunks by rounds of the pass");
 constexpr int kGather = 2;                  // particles whose gathers are in flight together
-constexpr int kChunk = 2048;                // slots per block of the untiled pass
-constexpr int kPPT = kChunk / kBlock;       // slots per thread of the helper kernels
+constexpr int kPPT = 8;                     // slots per thread of the helper kernels
+// The untiled pass runs one round a block.  Up to kSmallStore slots its blocks
+// are single wavefronts (256 slots): with 2048 slots a block 12 000 ions
+// kept 6 CUs busy and took 9.1 us, and 300 000 147 CUs.
+constexpr int64_t kSmallStore = 1 << 20;
 
 // component c of the state (x, z, vx, vy, vz, and the position remainders
 // xl, zl of long-time positions); c is a constant after unrolling, so the
@@ -189,12 +190,6 @@ __device__ __forceinline__ float *comp(const PushArgs &a, int c)
 {
     return c == 0 ? a.x : c == 1 ? a.z : c == 2 ? a.vx : c == 3 ? a.vy : c == 4 ? a.vz : c == 5 ? a.xl : a.zl;
 }
-
-// running sum of one thread's deposits while consecutive particles share a cell
-struct DepRun {
-    int ci, cj;
-    long long w[4];
-};
 
 // one particle's weights into the block's LDS window (tile + halo), or
 // into the global grid when its cell lies outside the window
@@ -214,25 +209,46 @@ __device__ __forceinline__ void window_deposit(int ci, int cj, const uint32_t w[
     }
 }
 
-// segmented inclusive scan of the lanes' runs keyed by cell; segment tails
-// deposit.  All 64 lanes must call it together.
-__device__ __forceinline__ void wave_deposit(DepRun &d, unsigned long long *acc, int nz)
+// The deposits of a wavefront's lanes in memory: cell = i nz + j (-1: none),
+// w its corners' weights (i, j), (i+1, j), (i, j+1), (i+1, j+1).  Round r
+// serves lane r of every quad, each lane of the quad adding one corner, so an
+// instruction's lanes fall on 16 records (or 16 pairs of node rows), not 64.
+// All 64 lanes must call it together.
+__device__ __forceinline__ void wave_deposit(int cell, const uint32_t w[4], unsigned long long *acc, int rec, int nz)
 {
-    const int lane = __lane_id();
-    const bool valid = d.ci >= 0;
-    const int key = valid ? d.ci * nz + d.cj : -1 - lane;
-    const int prev = __shfl_up(key, 1);
-    const unsigned long long heads = __ballot(lane == 0 || prev != key);
-    const int seg = 63 - __clzll(heads & ((2ull << lane) - 1ull));
+    const int q = __lane_id() & 3;
+    const size_t off = rec ? (size_t)q : (size_t)(q & 1) * nz + (q >> 1);
+    const int mul = rec ? 4 : 1;
+    if (cells_repeat(cell)) {  // uniform
+        unsigned long long s[4] = {w[0], w[1], w[2], w[3]};
+        if (segment_sums<4>(cell, s)) {
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        long long u0 = __shfl_up(d.w[0], off), u1 = __shfl_up(d.w[1], off);
-        long long u2 = __shfl_up(d.w[2], off), u3 = __shfl_up(d.w[3], off);
-        if (lane - off >= seg) { d.w[0] += u0; d.w[1] += u1; d.w[2] += u2; d.w[3] += u3; }
+            for (int c = 0; c < 4; c++) {
+                const size_t at = rec ? (size_t)cell * 4 + c : (size_t)cell + (size_t)(c & 1) * nz + (c >> 1);
+                if (s[c]) atomicAdd(acc + at, s[c]);
+            }
+        }
+        return;
     }
-    const bool tail = lane == 63 || ((heads >> (lane + 1)) & 1ull);
-    if (valid && tail) deposit_global(acc, nz, d.ci, d.cj, d.w);
-    d.ci = -1;
+    auto round = [&](int c, uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3) {
+        const uint32_t v = q == 0 ? w0 : q == 1 ? w1 : q == 2 ? w2 : w3;
+        if (c >= 0 && v) atomicAdd(acc + ((size_t)c * mul + off), (unsigned long long)v);
+    };
+    round((int)quad_lane<0>(cell), quad_lane<0>(w[0]), quad_lane<0>(w[1]), quad_lane<0>(w[2]), quad_lane<0>(w[3]));
+    round((int)quad_lane<1>(cell), quad_lane<1>(w[0]), quad_lane<1>(w[1]), quad_lane<1>(w[2]), quad_lane<1>(w[3]));
+    round((int)quad_lane<2>(cell), quad_lane<2>(w[0]), quad_lane<2>(w[1]), quad_lane<2>(w[2]), quad_lane<2>(w[3]));
+    round((int)quad_lane<3>(cell), quad_lane<3>(w[0]), quad_lane<3>(w[1]), quad_lane<3>(w[2]), quad_lane<3>(w[3]));
+}
+
+// fixed-point sum of node k = (i, j) from the records of the cells around it
+__device__ __forceinline__ long long rec_node2(const unsigned long long *rec, size_t k, int nz)
+{
+    const size_t i = k / nz, j = k - i * nz;
+    unsigned long long v = rec[4 * k];
+    if (i > 0) v += rec[4 * (k - nz) + 1];
+    if (j > 0) v += rec[4 * (k - 1) + 2];
+    if (i > 0 && j > 0) v += rec[4 * (k - nz - 1) + 3];
+    return (long long)v;
 }
 
 // FAST: the common configuration fixed at compile time (B = 0, no periodic
@@ -244,17 +260,19 @@ __device__ __forceinline__ void wave_deposit(DepRun &d, unsigned long long *acc,
 // particles and two gathers in registers.  The specialised tiled pass's FP32
 // index arithmetic (gather, cell and CIC offsets) fits six wavefronts (80
 // VGPRs) when the gather reads the one-float phase-applied tables, five (96
-// VGPRs) with the two-component tables; the untiled forms carry the deposit
-// runs and the FP64 generic forms their wider arithmetic, and keep four (128
-// VGPRs), three for the untiled deposit with a gridded B; with long-time
-// positions (two more state components) the forms keep four, three for the
-// untiled generic deposit.  Each is the most that builds without spilling to
-// scratch memory, which costs far more than the occupancy gains.
+// VGPRs) with the two-component tables; the FP64 generic forms with their
+// wider arithmetic and those with long-time positions (two more state
+// components) keep four (128 VGPRs).  The untiled deposit, whose atomics hold
+// a wavefront's weights and addresses beside the state, keeps three, and two
+// in the generic forms with a gridded B or long-time positions.  Each is
+// the most that builds without spilling to scratch memory, which costs far
+// more than the occupancy gains.
 template <bool DEPOSIT, bool TILED, bool FAST, bool BGRID, bool PHT, bool HIPOS>
 constexpr int pass_waves()
 {
-    if (HIPOS) return !TILED && DEPOSIT && !FAST ? 3 : 4;  // two more state components
-    return TILED && FAST ? (PHT ? 6 : 5) : (BGRID && DEPOSIT && !TILED ? 3 : 4);
+    if (!TILED && DEPOSIT) return !FAST && (HIPOS || BGRID) ? 2 : 3;
+    if (HIPOS) return 4;  // two more state components
+    return TILED && FAST ? (PHT ? 6 : 5) : 4;
 }
 
 // HIPOS: long-time positions, the FP32 pairs (x, xl), (z, zl).
@@ -286,16 +304,14 @@ k_advance2d(PushArgs a)
         for (int k = tid; k < kWin * kWin; k += kPass) win[k] = 0ull;
         __syncthreads();
     } else {
-        lo = (int64_t)blockIdx.x * kChunk;
-        hi = min(lo + (int64_t)kChunk, a.n);
+        lo = (int64_t)blockIdx.x * (4 * blockDim.x);  // one round
+        hi = min(lo + (int64_t)(4 * blockDim.x), a.n);
         co0 = lo;
     }
     int n_removed = 0, n_coll = 0;
     bool nan_any = false, gbad = false;
-    DepRun run;
-    run.ci = -1;
 #pragma unroll 1
-    for (int64_t co = co0; co < hi; co += kRound) {  // uniform over the block
+    for (int64_t co = co0; co < hi; co += TILED ? kRound : 4 * kPass) {  // uniform over the block
         // ---- this thread's slots pb..pb+3; slots outside [lo, hi) belong to
         // other blocks: they are neither computed nor written
         const int64_t pb = co + 4 * tid;
@@ -351,6 +367,16 @@ k_advance2d(PushArgs a)
                                                          HIPOS ? pos64(v[1][h], v[6][h]) : (double)v[1][h], a.phase,
                                                          gex[h], gez[h]);
                     gbad |= b && !is_dead(v[0][h]);
+                }
+            }
+            // the untiled deposits, added by all lanes together after the group
+            int dcell[kGather];
+            uint32_t dw[kGather][4];
+            if constexpr (DEPOSIT && !TILED) {
+#pragma unroll
+                for (int q = 0; q < kGather; q++) {
+                    dcell[q] = -1;
+                    dw[q][0] = dw[q][1] = dw[q][2] = dw[q][3] = 0u;
                 }
             }
 #pragma unroll
@@ -466,7 +492,7 @@ k_advance2d(PushArgs a)
                     continue;
                 }
                 // ---- deposit (particles.hpp:408-409): tiled, straight into the
-                // LDS window; untiled, summed per run of equal cells
+                // LDS window; untiled, into memory (below)
                 if (DEPOSIT) {
                     int ci, cj;
                     uint32_t w[4];
@@ -484,12 +510,10 @@ k_advance2d(PushArgs a)
                     if (in_grid) {
                         if constexpr (TILED) {
                             window_deposit(ci, cj, w, win, wi0, wj0, a.acc, a.nz);
-                        } else if (ci == run.ci && cj == run.cj) {
-                            run.w[0] += w[0]; run.w[1] += w[1]; run.w[2] += w[2]; run.w[3] += w[3];
                         } else {
-                            if (run.ci >= 0) deposit_global(a.acc, a.nz, run.ci, run.cj, run.w);
-                            run.ci = ci; run.cj = cj;
-                            run.w[0] = w[0]; run.w[1] = w[1]; run.w[2] = w[2]; run.w[3] = w[3];
+                            dcell[q] = ci * a.nz + cj;
+#pragma unroll
+                            for (int c = 0; c < 4; c++) dw[q][c] = w[c];
                         }
                     } else {
                         raise_flag(a.counters, M2D_FLAG_OUT_OF_RANGE);
@@ -497,6 +521,10 @@ k_advance2d(PushArgs a)
                 }
                 v[0][q] = x; v[1][q] = z; v[2][q] = vx; v[3][q] = vy; v[4][q] = vz;
                 if constexpr (HIPOS) { v[5][q] = xl; v[6][q] = zl; }
+            }
+            if constexpr (DEPOSIT && !TILED) {
+#pragma unroll
+                for (int q = 0; q < kGather; q++) wave_deposit(dcell[q], dw[q], a.acc, a.rec, a.nz);
             }
 #pragma unroll
             for (int c = 0; c < NC; c++) {
@@ -512,7 +540,6 @@ k_advance2d(PushArgs a)
 #pragma unroll
             for (int q = 0; q < 4; q++) tw[q] = u[q];
         }
-        if constexpr (DEPOSIT && !TILED) wave_deposit(run, a.acc, a.nz);
         // ---- store
         if (full) {
 #pragma unroll
@@ -632,9 +659,10 @@ constexpr int kPhPerThread = 4;
 // After the pass, in dispatch order: with MCC, kScatterBlocks blocks apply
 // the collision queue (a long FP64 chain that sets the launch's length, so
 // it starts first); ntab blocks build the next step's phase-applied tables;
-// the rest add the deposit, rho += charge * acc * 2^-31, and clear acc.
+// the rest add the deposit, rho += charge * acc * 2^-31, and clear acc (REC:
+// from cell records, cleared by rec_done).
 constexpr unsigned kScatterBlocks = 64;
-template <bool MCC>
+template <bool MCC, bool REC>
 __global__ void __launch_bounds__(kBlock) k_flush_scatter(unsigned long long *acc, double *rho, double charge,
                                                          size_t n, PhBuild ph, unsigned ntab, PushArgs a,
                                                          unsigned long long *next_len)
@@ -662,10 +690,10 @@ __global__ void __launch_bounds__(kBlock) k_flush_scatter(unsigned long long *ac
     }
     const size_t k = (size_t)(blockIdx.x - ns - ntab) * kBlock + threadIdx.x;
     if (k >= n) return;
-    const long long v = (long long)acc[k];
+    const long long v = REC ? rec_node2(acc, k, a.nz) : (long long)acc[k];
     if (v) {
         rho[k] += charge * ((double)v * kInvFix);
-        acc[k] = 0ull;
+        if (!REC) acc[k] = 0ull;
     }
 }
 
@@ -730,44 +758,61 @@ __global__ void k_fields_E(PushArgs a, const double *xs, const double *zs, int64
     ez[k] = fz;
 }
 
-// Species::accumulate (particles.hpp:358-367) into the fixed-point grid
+// Species::accumulate (particles.hpp:358-367) into the fixed-point grid (or,
+// with rec, into cell records)
 __global__ void __launch_bounds__(kBlock) k_accumulate2d(const float *xs, const float *zs, const float *xls,
                                                          const float *zls, int64_t n, int nx, int nz, double idx,
                                                          double idz, double xmin, double zmin,
-                                                         unsigned long long *acc,
+                                                         unsigned long long *acc, int rec,
                                                          unsigned long long *counters)
 {
-    int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    float x = xs[p];
-    if (is_dead(x)) return;
-    const float xl = xls ? xls[p] : 0.f, zl = zls ? zls[p] : 0.f;
-    int i, j;
-    uint32_t w[4];
-    bool in_grid;
-    if (xmin == 0.0 && zmin == 0.0) {
-        // the FP32 pair arithmetic of the specialised pass, so a grid of
-        // origin 0 gets the bits of the fused deposit (a NaN fails x >= 0)
-        const float z = zs[p];
-        float sxh, sxl, szh, szl, u, ou, v, ov;
-        split_f32(idx, sxh, sxl);
-        split_f32(idz, szh, szl);
-        in_grid = pos64(x, xl) >= 0.0 && pos64(z, zl) >= 0.0;
-        if (in_grid) {
-            cell_f(x, xl, sxh, sxl, i, u, ou);
-            cell_f(z, zl, szh, szl, j, v, ov);
-            in_grid = (unsigned)i <= (unsigned)(nx - 2) && (unsigned)j <= (unsigned)(nz - 2);
-            if (in_grid) cic_from_offsets(u, ou, v, ov, w);
+    const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const float x = p < n ? xs[p] : dead_value();
+    int cell = -1;
+    uint32_t w[4] = {0u, 0u, 0u, 0u};
+    bool out = false;
+    if (!is_dead(x)) {
+        const float xl = xls ? xls[p] : 0.f, zl = zls ? zls[p] : 0.f;
+        int i, j;
+        bool in_grid;
+        if (xmin == 0.0 && zmin == 0.0) {
+            // the FP32 pair arithmetic of the specialised pass, so a grid of
+            // origin 0 gets the bits of the fused deposit (a NaN fails x >= 0)
+            const float z = zs[p];
+            float sxh, sxl, szh, szl, u, ou, v, ov;
+            split_f32(idx, sxh, sxl);
+            split_f32(idz, szh, szl);
+            in_grid = pos64(x, xl) >= 0.0 && pos64(z, zl) >= 0.0;
+            if (in_grid) {
+                cell_f(x, xl, sxh, sxl, i, u, ou);
+                cell_f(z, zl, szh, szl, j, v, ov);
+                in_grid = (unsigned)i <= (unsigned)(nx - 2) && (unsigned)j <= (unsigned)(nz - 2);
+                if (in_grid) cic_from_offsets(u, ou, v, ov, w);
+            }
+        } else {
+            in_grid = cic_weights((pos64(x, xl) - xmin) * idx, (pos64(zs[p], zl) - zmin) * idz, nx, nz, i, j, w);
         }
-    } else {
-        in_grid = cic_weights((pos64(x, xl) - xmin) * idx, (pos64(zs[p], zl) - zmin) * idz, nx, nz, i, j, w);
+        out = !in_grid;
+        if (in_grid) {
+            if (((size_t)nx * nz) >> 31) {  // uniform: no 32-bit cell index
+                const long long ww[4] = {w[0], w[1], w[2], w[3]};
+                deposit_global(acc, nz, i, j, ww);
+            } else {
+                cell = i * nz + j;
+            }
+        }
     }
-    if (in_grid) {
-        const long long ww[4] = {w[0], w[1], w[2], w[3]};
-        deposit_global(acc, nz, i, j, ww);
-    }
-    else
-        raise_flag(counters, M2D_FLAG_OUT_OF_RANGE);
+    wave_deposit(cell, w, acc, rec, nz);
+    if (__ballot(out) && __lane_id() == 0) raise_flag(counters, M2D_FLAG_OUT_OF_RANGE);
+}
+
+// rho += charge * (sum of the cell records) * 2^-31
+__global__ void k_flush_rec(const unsigned long long *rec, double *rho, double charge, size_t n, int nz)
+{
+    const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const long long v = rec_node2(rec, k, nz);
+    if (v) rho[k] += charge * ((double)v * kInvFix);
 }
 
 // rho += charge * acc * 2^-31; acc = 0
@@ -1124,6 +1169,53 @@ int ensure_acc(m2d_ctx *ctx, size_t n)
     return zero_words(ctx, (unsigned long long *)ctx->acc.ptr, ctx->acc.bytes / 8);
 }
 
+int deposit_buffer(m2d_ctx *ctx, size_t nodes, int corners, int &rec, unsigned long long *&acc)
+{
+    M2D_TRY(ensure_acc(ctx, nodes));
+    acc = (unsigned long long *)ctx->acc.ptr;
+    if (!rec) return M2D_OK;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        rec = 0;
+        return M2D_OK;
+    }
+    const size_t need = nodes * corners * sizeof(unsigned long long);
+    const bool grown = ctx->rec.bytes < need;
+    if (grown) {
+        const int r = ensure(ctx, ctx->rec, need);
+        if (r == M2D_ERR_NO_MEMORY) {  // the node grid does
+            (void)hipGetLastError();
+            rec = 0;
+            return M2D_OK;
+        }
+        M2D_TRY(r);
+    }
+    if (grown || ctx->rec_dirty) M2D_TRY(zero_words(ctx, (unsigned long long *)ctx->rec.ptr, ctx->rec.bytes / 8));
+    ctx->rec_dirty = true;  // until rec_done
+    acc = (unsigned long long *)ctx->rec.ptr;
+    return M2D_OK;
+}
+
+int rec_done(m2d_ctx *ctx, size_t cells, int corners)
+{
+    M2D_TRY(zero_words(ctx, (unsigned long long *)ctx->rec.ptr, cells * corners));
+    ctx->rec_dirty = false;
+    return M2D_OK;
+}
+
+// Records pay where the requests they save cover their clearing (a launch,
+// and 32 bytes a node to write and read instead of 8).  Atomics at the nodes
+// against records, alone: 33k particles 8.3 and 5.2 us (128^2 grid), 295k 61
+// and 35 us (128^2), 32 and 22 us (512^2); clearing takes a launch of 3-4 us
+// up to 200^2 and writes 8 MB at 512^2.  So: from kRecMin2 particles and one
+// a node on, and below 2^30 nodes (a cell's index is 32-bit).
+constexpr int64_t kRecMin2 = 49152;
+static bool use_rec2(int64_t particles, size_t nodes)
+{
+    return particles >= kRecMin2 && (size_t)particles >= nodes && nodes < (1u << 30);
+}
+
 static int flush(m2d_ctx *ctx, size_t n, double *rho, double charge)
 {
     k_flush<<<(unsigned)((n + 255) / 256), 256, 0, ctx->stream>>>((unsigned long long *)ctx->acc.ptr,
@@ -1193,6 +1285,7 @@ static void fill_push_args(PushArgs &a, m2d_fields2d *f, const m2d_species2d *s,
     a.n_chunks = nullptr;
     a.ntz = 0;
     a.acc = nullptr;
+    a.rec = 0;
     a.counters = f->ctx->counters;
     a.bt = f->bt;
     a.bnx = a.bnz = 0;
@@ -1306,8 +1399,8 @@ int m2d_advance_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s, const 
     const bool hipos = p->xl != nullptr;
     if (hipos && !fast) T = nullptr;
     if (deposit) {
-        M2D_TRY(ensure_acc(ctx, f->n));
-        a.acc = (unsigned long long *)ctx->acc.ptr;
+        a.rec = !T && use_rec2(p->n, f->n);
+        M2D_TRY(deposit_buffer(ctx, f->n, 4, a.rec, a.acc));
     }
     if (T) {
         a.sched = T->sched;
@@ -1322,9 +1415,10 @@ int m2d_advance_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s, const 
         void (*kern)(PushArgs) = hipos ? pick_pass<true>(T != nullptr, fast, pht, bgrid, deposit, use_mcc)
                                        : pick_pass<false>(T != nullptr, fast, pht, bgrid, deposit, use_mcc);
         M2D_CHECK(kern, M2D_ERR_UNSUPPORTED, "m2d_advance_2d: no compiled form of the pass for this configuration");
-        const int g = T ? (int)xcd_run_grid((unsigned)T->max_chunks) : (int)((p->n + kChunk - 1) / kChunk);
+        const int threads = T || p->n > kSmallStore ? kPass : 64;
+        const int g = T ? (int)xcd_run_grid((unsigned)T->max_chunks) : (int)((p->n + 4 * threads - 1) / (4 * threads));
         fast_tiled = T && fast;
-        launch_timed(ctx, kern, dim3(g), dim3(kPass), a);
+        launch_timed(ctx, kern, dim3(g), dim3(threads), a);
         M2D_HIP(hipGetLastError());
         ctx->last_pass = (deposit ? M2D_PASS_DEPOSIT : 0u) | (use_mcc ? M2D_PASS_MCC : 0u) |
                          (T ? M2D_PASS_TILED : 0u) | (fast ? M2D_PASS_FAST : bgrid ? M2D_PASS_BGRID : 0u) |
@@ -1363,12 +1457,11 @@ int m2d_advance_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s, const 
         const unsigned g = nfl + ntab + (use_mcc && !serial ? kScatterBlocks : 0u);
         // without a deposit no flush block runs: n = 0 ends them at once
         const size_t nodes = deposit ? f->n : 0;
-        if (use_mcc && !serial)
-            k_flush_scatter<true><<<g, kBlock, 0, ctx->stream>>>(a.acc, rho, s->charge, nodes, pb, ntab, a, next_len);
-        else if (g > 0)
-            k_flush_scatter<false><<<g, kBlock, 0, ctx->stream>>>(a.acc, rho, s->charge, nodes, pb, ntab, a,
-                                                                  next_len);
+        const auto flush_kernel = use_mcc && !serial ? (a.rec ? k_flush_scatter<true, true> : k_flush_scatter<true, false>)
+                                                     : (a.rec ? k_flush_scatter<false, true> : k_flush_scatter<false, false>);
+        if (g > 0) flush_kernel<<<g, kBlock, 0, ctx->stream>>>(a.acc, rho, s->charge, nodes, pb, ntab, a, next_len);
         M2D_HIP(hipGetLastError());
+        if (a.rec) M2D_TRY(rec_done(ctx, f->n, 4));
         if (a.cq_defer) {
             k_scatter_apply<<<kScatterBlocks, kBlock, 0, ctx->stream>>>(a);
             M2D_HIP(hipGetLastError());
@@ -1467,14 +1560,19 @@ int m2d_accumulate_2d(m2d_ctx *ctx, const m2d_grid2d *g, const m2d_particles2d *
               "m2d_accumulate_2d: bad grid");
     M2D_TRY(check_parts(p));
     size_t n = (size_t)g->nx * g->nz;
-    M2D_TRY(ensure_acc(ctx, n));
+    int rec = use_rec2(p->n, n);
+    unsigned long long *acc;
+    M2D_TRY(deposit_buffer(ctx, n, 4, rec, acc));
     if (p->n > 0) {
         k_accumulate2d<<<grid_for(p->n, 1), kBlock, 0, ctx->stream>>>(
             p->x, p->z, p->xl, p->zl, p->n, g->nx, g->nz, 1.0 / g->dx, 1.0 / g->dz, g->xmin, g->zmin,
-            (unsigned long long *)ctx->acc.ptr, ctx->counters);
+            acc, rec, ctx->counters);
         M2D_HIP(hipGetLastError());
     }
-    return flush(ctx, n, rho, charge);
+    if (!rec) return flush(ctx, n, rho, charge);
+    k_flush_rec<<<(unsigned)((n + 255) / 256), 256, 0, ctx->stream>>>(acc, rho, charge, n, g->nz);
+    M2D_HIP(hipGetLastError());
+    return rec_done(ctx, n, 4);
 }
 
 int m2d_interpolate_2d(m2d_ctx *ctx, const m2d_grid2d *g, const double *data, const double *x,
