@@ -142,7 +142,7 @@ def test_advance_3d(ctx):
 def test_captured_deposit_outlives_larger_records(ctx):
     """A captured deposit replays right after a call that outgrew the records
     (it runs on the node grid)."""
-    hip = C.CDLL("libamdhip64.so")
+    hip = C.CDLL(abi.lib()._name)  # the HIP runtime that the library itself is linked to
     g = abi.grid2d(64, 64, 1e-3, 1e-3)
     rng = np.random.default_rng(8)
     x, z = positions((64, 64), 1e-3, (0.0, 0.0), 50_000, rng, "random")
