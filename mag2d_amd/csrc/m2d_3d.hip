@@ -13,8 +13,8 @@
 #include <cmath>
 #include <cstring>
 #include <new>
-#include <rocprim/device/device_radix_sort.hpp>
 #include "m2d_objects.hpp"
+#include "m2d_sort.hpp"
 #include "m2d_scatter.hpp"
 
 namespace m2d {
@@ -1059,47 +1059,22 @@ __global__ void __launch_bounds__(256) k_accumulate3d(const float *xs, const flo
 
 // ------------------------------------------------------------------ sort
 // tile-major cell key: (tile << 6) | cell in its 4 x 4 x 4 tile
-__global__ void k_sort_keys3d(const float *xs, const float *ys, const float *zs, int64_t n, Grid3 g, int nty3,
-                              int ntz3, uint32_t dead_key, uint32_t *keys, uint32_t *vals)
-{
-    int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    const float x = xs[p];
-    uint32_t key = dead_key;
-    if (!is_dead(x)) {
+struct Key3 {
+    const float *x, *y, *z;
+    Grid3 g;
+    int nty3, ntz3;
+    uint32_t dead_key;
+    __device__ __forceinline__ uint32_t operator()(int64_t p) const
+    {
+        const float v = x[p];
+        if (is_dead(v)) return dead_key;
         auto idx = [](double X, int nmax) { return X >= 0.0 ? (int)fmin(X, (double)nmax) : 0; };
-        const int i = idx((double)x * g.idx, g.nx - 2), j = idx((double)ys[p] * g.idy, g.ny - 2),
-                  k = idx((double)zs[p] * g.idz, g.nz - 2);
+        const int i = idx((double)v * g.idx, g.nx - 2), j = idx((double)y[p] * g.idy, g.ny - 2),
+                  k = idx((double)z[p] * g.idz, g.nz - 2);
         const uint32_t tile = (uint32_t)(((i / kTile3) * nty3 + j / kTile3) * ntz3 + k / kTile3);
-        key = (tile << 6) | (uint32_t)((i % kTile3) * 16 + (j % kTile3) * 4 + k % kTile3);
+        return (tile << 6) | (uint32_t)((i % kTile3) * 16 + (j % kTile3) * 4 + k % kTile3);
     }
-    keys[p] = key;
-    vals[p] = (uint32_t)p;
-}
-
-__global__ void k_sort_gather3d(m2d_particles3d src, m2d_particles3d dst, const uint32_t *keys,
-                                const uint32_t *vals, uint32_t dead_key, unsigned long long *n_live)
-{
-    // destination ranges in XCD-contiguous order (as k_sort_gather)
-    const unsigned nb = (unsigned)((src.n + blockDim.x - 1) / blockDim.x);
-    const unsigned b = xcd_block(blockIdx.x, nb);
-    if (b >= nb) return;
-    int64_t i = (int64_t)b * blockDim.x + threadIdx.x;
-    if (i >= src.n) return;
-    const uint32_t k = keys[i];
-    if (k == dead_key) {
-        dst.x[i] = dead_value();
-        return;
-    }
-    if (i == src.n - 1 || keys[i + 1] == dead_key) *n_live = (unsigned long long)(i + 1);
-    const int64_t s = vals[i];
-    dst.x[i] = src.x[s];
-    dst.y[i] = src.y[s];
-    dst.z[i] = src.z[s];
-    dst.vx[i] = src.vx[s];
-    dst.vy[i] = src.vy[s];
-    dst.vz[i] = src.vz[s];
-}
+};
 
 // ------------------------------------------------------------------ host helpers
 static int dmalloc3(void **p, size_t bytes)
@@ -1857,41 +1832,17 @@ int m2d_sort_3d(m2d_ctx *ctx, m2d_fields3d *f, const m2d_particles3d *src, const
     }
     const Grid3 g = grid3_of(f->p.grid);
     const int ntx3 = (g.nx - 2) / kTile3 + 1, nty3 = (g.ny - 2) / kTile3 + 1, ntz3 = (g.nz - 2) / kTile3 + 1;
-    const uint64_t keyspace = ((uint64_t)ntx3 * nty3 * ntz3) << 6;
-    int bits = 0;
-    while ((1ull << bits) <= keyspace) bits++;
+    const int bits = sort_key_bits((uint64_t)ntx3 * nty3 * ntz3);
     M2D_CHECK(bits <= 32, M2D_ERR_BAD_ARG, "m2d_sort_3d: grid too large for 32-bit keys");
-    const uint32_t dead_key = bits == 32 ? 0xFFFFFFFFu : (uint32_t)((1ull << bits) - 1);
-    size_t temp = 0;
     // tile-major cell order.  Unlike the 2D store (ordered by tile only), a
     // 3D cell holds few particles (8 on average at the 16M-ion, 128^3
     // workload), so the lanes of a wave spread over several cells anyway, and
     // the cell order's gather locality wins: the tiled pass runs 419 us on a
     // cell-ordered store against 505 us on a tile-ordered one
-    hipError_t e = rocprim::radix_sort_pairs(nullptr, temp, (const uint32_t *)nullptr, (uint32_t *)nullptr,
-                                             (const uint32_t *)nullptr, (uint32_t *)nullptr, n, 0, bits,
-                                             ctx->stream);
-    M2D_CHECK(e == hipSuccess, M2D_ERR_HIP, "radix_sort_pairs size query: %s", hipGetErrorString(e));
-    const size_t arr = ((n * 4 + 255) / 256) * 256;
-    M2D_TRY(ensure(ctx, ctx->sortbuf, 4 * arr + temp + 256));
-    uint8_t *b = (uint8_t *)ctx->sortbuf.ptr;
-    uint32_t *k0 = (uint32_t *)b, *k1 = (uint32_t *)(b + arr), *v0 = (uint32_t *)(b + 2 * arr),
-             *v1 = (uint32_t *)(b + 3 * arr);
-    unsigned long long *live = ctx->counters + CNT_LIVE;
-    M2D_TRY(zero_words(ctx, live, 1));
-    k_sort_keys3d<<<blocks_for(n), 256, 0, ctx->stream>>>(src->x, src->y, src->z, src->n, g, nty3, ntz3, dead_key,
-                                                          k0, v0);
-    M2D_HIP(hipGetLastError());
-    e = rocprim::radix_sort_pairs(b + 4 * arr, temp, k0, k1, v0, v1, n, 0, bits, ctx->stream);
-    M2D_CHECK(e == hipSuccess, M2D_ERR_HIP, "radix_sort_pairs: %s", hipGetErrorString(e));
-    k_sort_gather3d<<<xcd_grid(blocks_for(n)), 256, 0, ctx->stream>>>(*src, *dst, k1, v1, dead_key, live);
-    M2D_HIP(hipGetLastError());
-    M2D_TRY(build_tiling(ctx, dst->x, dst->n, k1, dead_key, ntx3, nty3, ntz3, kChunkCap3, 256));
-    if (n_live) {
-        M2D_TRY(read_counters(ctx));
-        *n_live = (int64_t)ctx->h_counters[CNT_LIVE];
-    }
-    return M2D_OK;
+    const Key3 key{src->x, src->y, src->z, g, nty3, ntz3, sort_dead_key(bits)};
+    const Columns<6> from{{src->x, src->y, src->z, src->vx, src->vy, src->vz}},
+        to{{dst->x, dst->y, dst->z, dst->vx, dst->vy, dst->vz}};
+    return sort_store(ctx, key, from, to, n, 0, bits, ntx3, nty3, ntz3, kChunkCap3, 256, n_live);
 }
 
 int m2d_sort_forget_3d(m2d_ctx *ctx, const m2d_particles3d *p)

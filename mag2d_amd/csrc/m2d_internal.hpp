@@ -109,8 +109,8 @@ struct m2d_tiling {
     int64_t n = 0;
     int ntx = 0, nty = 1, ntz = 0;  // sort tiles along x, (y,) z
     int max_chunks = 0;        // launch bound
-    m2d::Scratch buf;          // device: sched, tile_start, tile_end, chunk_count, n_chunks
-    int *tile_start = nullptr, *tile_end = nullptr, *chunk_count = nullptr;
+    m2d::Scratch buf;          // device: sched, tile_start, tile_end, totals, n_chunks
+    int *tile_start = nullptr, *tile_end = nullptr, *totals = nullptr;
     int4 *sched = nullptr;
     unsigned int *n_chunks = nullptr;
 };
@@ -133,7 +133,7 @@ struct m2d_ctx {
     bool rec_dirty = false; // a call failed between writing records and clearing them
     m2d::Scratch red;       // reduction partials
     m2d::Scratch tmp;       // general temporaries (compaction offsets)
-    m2d::Scratch sortbuf;   // keys, slots and radix-sort temporaries
+    m2d::Scratch sortbuf;   // keys, slots, packed particles and radix-sort temporaries
     m2d::Scratch cq;        // MCC collision queue (slot indices)
     uint64_t launch_seq = 0;  // selects the collision-queue counter of a launch
     bool cq_dirty = false;    // a call failed between appending to a queue counter and its scatter
@@ -149,8 +149,6 @@ namespace m2d {
 // tile schedules of sorted stores (m2d_sort.hip)
 m2d_tiling *find_tiling(m2d_ctx *ctx, const float *x, int64_t n);
 int sort_keys_u32(m2d_ctx *ctx, const uint32_t *in, uint32_t *out, size_t n);
-int build_tiling(m2d_ctx *ctx, const float *x, int64_t n, const uint32_t *keys, uint32_t dead_key, int ntx,
-                 int nty, int ntz, int cap, int round);
 void forget_tiling(m2d_ctx *ctx, const float *x);
 void free_tilings(m2d_ctx *ctx);
 // objects that hold a context keep it alive until they are destroyed
