@@ -177,10 +177,11 @@ constexpr int kRound = kPass * 4;
 static_assert(kRound == kRound2, "the tile schedule orders chunks by rounds of the pass");
 constexpr int kGather = 2;                  // particles whose gathers are in flight together
 constexpr int kPPT = 8;                     // slots per thread of the helper kernels
-// The untiled pass runs one round a block.  Up to kSmallStore slots its blocks
-// are single wavefronts (256 slots): with 2048 slots a block 12 000 ions
-// kept 6 CUs busy and took 9.1 us, and 300 000 147 CUs.
-constexpr int64_t kSmallStore = 1 << 20;
+// The untiled pass runs one round of 256 slots a block, and its blocks are
+// single wavefronts: with 2048 slots a block 12 000 ions kept 6 CUs busy and
+// took 9.1 us (now 5.7); from a million slots on both take the same time.
+constexpr int kPassU = 64;
+constexpr int kRoundU = kPassU * 4;
 
 // component c of the state (x, z, vx, vy, vz, and the position remainders
 // xl, zl of long-time positions); c is a constant after unrolling, so the
@@ -264,25 +265,41 @@ __device__ __forceinline__ long long rec_node2(const unsigned long long *rec, si
 // wider arithmetic and those with long-time positions (two more state
 // components) keep four (128 VGPRs).  The untiled deposit, whose atomics hold
 // a wavefront's weights and addresses beside the state, keeps three, and two
-// in the generic forms with a gridded B or long-time positions.  Each is
+// in the generic forms with a gridded B or long-time positions; the scatter's
+// FP64 chain in the pass (SCAT) keeps three.  Each is
 // the most that builds without spilling to scratch memory, which costs far
 // more than the occupancy gains.
-template <bool DEPOSIT, bool TILED, bool FAST, bool BGRID, bool PHT, bool HIPOS>
+template <bool DEPOSIT, bool TILED, bool FAST, bool BGRID, bool PHT, bool HIPOS, bool SCAT>
 constexpr int pass_waves()
 {
+    if (SCAT) return 3;
     if (!TILED && DEPOSIT) return !FAST && (HIPOS || BGRID) ? 2 : 3;
     if (HIPOS) return 4;  // two more state components
     return TILED && FAST ? (PHT ? 6 : 5) : 4;
 }
 
 // HIPOS: long-time positions, the FP32 pairs (x, xl), (z, zl).
-template <bool DEPOSIT, bool MCC, bool TILED, bool FAST, bool BGRID = false, bool PHT = false, bool HIPOS = false>
-__global__ void __launch_bounds__(kPass)
-__attribute__((amdgpu_waves_per_eu(pass_waves<DEPOSIT, TILED, FAST, BGRID, PHT, HIPOS>())))
+// SCAT (a step without a deposit, so without a flush launch): the block, one
+// wavefront, scatters its own collisions after storing its slots, from a
+// queue in LDS.  Pass and scatter launch against this, per step: 12k slots
+// 12.2 and 7.4 us, 1M 22.4 and 20.6; with 1% of the slots colliding, whose
+// appends to the one queue in memory cost 8 ns each, 1M 124 and 60 us, 8M 926
+// and 365.
+template <bool DEPOSIT, bool MCC, bool TILED, bool FAST, bool BGRID = false, bool PHT = false, bool HIPOS = false,
+          bool SCAT = false>
+__global__ void __launch_bounds__(TILED ? kPass : kPassU)
+__attribute__((amdgpu_waves_per_eu(pass_waves<DEPOSIT, TILED, FAST, BGRID, PHT, HIPOS, SCAT>())))
 k_advance2d(PushArgs a)
 {
+    static_assert(!SCAT || (MCC && !TILED && !DEPOSIT), "a deposit's flush launch scatters too");
     __shared__ unsigned long long win[TILED ? kWin * kWin : 1];
+    __shared__ float4 hits[SCAT ? kRoundU : 1];  // velocity after the push and slot - lo
+    __shared__ int n_hits;
     const int tid = threadIdx.x;
+    if constexpr (SCAT) {
+        if (tid == 0) n_hits = 0;
+        __syncthreads();
+    }
     // slots [lo, hi) of this block; rounds start at lo rounded down to 64, so
     // a thread's 4 slots are one aligned float4 of each component and share
     // one trial Philox block
@@ -304,14 +321,14 @@ k_advance2d(PushArgs a)
         for (int k = tid; k < kWin * kWin; k += kPass) win[k] = 0ull;
         __syncthreads();
     } else {
-        lo = (int64_t)blockIdx.x * (4 * blockDim.x);  // one round
-        hi = min(lo + (int64_t)(4 * blockDim.x), a.n);
+        lo = (int64_t)blockIdx.x * kRoundU;
+        hi = min(lo + (int64_t)kRoundU, a.n);
         co0 = lo;
     }
     int n_removed = 0, n_coll = 0;
     bool nan_any = false, gbad = false;
 #pragma unroll 1
-    for (int64_t co = co0; co < hi; co += TILED ? kRound : 4 * kPass) {  // uniform over the block
+    for (int64_t co = co0; co < hi; co += TILED ? kRound : kRoundU) {  // uniform over the block
         // ---- this thread's slots pb..pb+3; slots outside [lo, hi) belong to
         // other blocks: they are neither computed nor written
         const int64_t pb = co + 4 * tid;
@@ -418,7 +435,11 @@ k_advance2d(PushArgs a)
                     // or the deposit below: the slot is queued and k_flush_scatter
                     // applies BaseSpecies::scatter afterwards.
                     if (MCC) {
-                        if ((uint64_t)tw[q] < a.trial_thr) {
+                        if (SCAT && (uint64_t)tw[q] < a.trial_thr) {
+                            hits[atomicAdd(&n_hits, 1)] =
+                                make_float4(vx, vy, vz, __int_as_float((int)(pb - lo) + q0 + q));
+                            n_coll++;
+                        } else if ((uint64_t)tw[q] < a.trial_thr) {
                             unsigned long long at = atomicAdd(a.cq_len, 1ull);
                             a.cq[at] = (uint32_t)(pb + q0 + q);
                             a.cqv[at] = make_float4(vx, vy, vz, 0.f);
@@ -563,6 +584,19 @@ k_advance2d(PushArgs a)
         for (int k = tid; k < kWin * kWin; k += kPass) {
             const unsigned long long v = win[k];
             if (v) atomicAdd(a.acc + (size_t)(wi0 + k / kWin) * a.nz + (wj0 + k % kWin), v);
+        }
+    }
+    if constexpr (SCAT) {
+        // (the wavefront's own stores above come before these)
+        __syncthreads();
+        for (int k = tid; k < n_hits; k += kPassU) {
+            const float4 w = hits[k];
+            const int64_t p = lo + __float_as_int(w.w);
+            float vx = w.x, vy = w.y, vz = w.z;
+            Rng rg;
+            rg.begin(a.seed, a.stream, (uint32_t)p, a.step, kPurposeMcc);
+            scatter_last(*a.mcc, rg, vx, vy, vz, a.counters);
+            a.vx[p] = vx; a.vy[p] = vy; a.vz[p] = vz;
         }
     }
     // ---- counters: one atomic per wavefront
@@ -1307,8 +1341,13 @@ static void fill_push_args(PushArgs &a, m2d_fields2d *f, const m2d_species2d *s,
 // the deposit and the MCC trial are on.  Long-time positions (HIPOS) have no
 // generic tiled form: the caller runs those untiled.
 template <bool HIPOS>
-static void (*pick_pass(bool tiled, bool fast, bool pht, bool bgrid, bool deposit, bool mcc))(PushArgs)
+static void (*pick_pass(bool tiled, bool fast, bool pht, bool bgrid, bool deposit, bool mcc, bool scat))(PushArgs)
 {
+    if (scat) {
+        if (fast) return k_advance2d<false, true, false, true, false, false, HIPOS, true>;
+        return bgrid ? k_advance2d<false, true, false, false, true, false, HIPOS, true>
+                     : k_advance2d<false, true, false, false, false, false, HIPOS, true>;
+    }
     if (tiled) {
         if (fast && pht)
             return mcc ? k_advance2d<true, true, true, true, false, true, HIPOS>
@@ -1368,10 +1407,24 @@ int m2d_advance_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s, const 
     // the MCC trial belongs to advance_boris; an empty store queues nothing
     // (and leaves the alternating queue counters as they are)
     bool use_mcc = p->n > 0 && a.push && mcc && std::isfinite(s->lifetime) && s->lifetime > 0;
+    // an interaction that turns its partner (COULOMB) scatters the queue
+    // in slot order after the flush, by one thread
+    const bool serial = use_mcc && mcc->h.partner_update;
+    // a target whose partner ensemble is this very store would read
+    // velocities that other collisions of the step are writing: the
+    // scatter then keeps its results in the queue, and k_scatter_apply
+    // stores them once every collision has read its partner
+    bool self_target = false;
+    if (use_mcc && !serial)
+        for (int t = 0; t < mcc->h.n_targets; t++) self_target |= mcc->h.t[t].px == p->x;
+    a.cq_defer = self_target ? 1 : 0;
+    const bool scat = use_mcc && !serial && !self_target && !deposit;
     unsigned long long *next_len = nullptr;
     if (use_mcc) {
         a.trial_thr = trial_threshold(1.0 - exp(-s->dt / s->lifetime));  // particles.cpp:937
         a.mcc = mcc->d;
+    }
+    if (use_mcc && !scat) {
         // slots (u32), then velocities (float4) from a 16-byte boundary
         const size_t qn = (size_t)p->n, vo = (qn * sizeof(uint32_t) + 15) & ~(size_t)15;
         M2D_TRY(ensure(ctx, ctx->cq, vo + qn * sizeof(float4)));
@@ -1412,19 +1465,18 @@ int m2d_advance_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s, const 
         const bool bgrid = f->bt != nullptr;  // B per particle (generic pass)
         // the flush after the previous pass left the tables for this phase
         const bool pht = T && fast && f->ph_valid && f->ph_phase == a.phase;
-        void (*kern)(PushArgs) = hipos ? pick_pass<true>(T != nullptr, fast, pht, bgrid, deposit, use_mcc)
-                                       : pick_pass<false>(T != nullptr, fast, pht, bgrid, deposit, use_mcc);
+        void (*kern)(PushArgs) = hipos ? pick_pass<true>(T != nullptr, fast, pht, bgrid, deposit, use_mcc, scat)
+                                       : pick_pass<false>(T != nullptr, fast, pht, bgrid, deposit, use_mcc, scat);
         M2D_CHECK(kern, M2D_ERR_UNSUPPORTED, "m2d_advance_2d: no compiled form of the pass for this configuration");
-        const int threads = T || p->n > kSmallStore ? kPass : 64;
-        const int g = T ? (int)xcd_run_grid((unsigned)T->max_chunks) : (int)((p->n + 4 * threads - 1) / (4 * threads));
+        const int g = T ? (int)xcd_run_grid((unsigned)T->max_chunks) : (int)((p->n + kRoundU - 1) / kRoundU);
         fast_tiled = T && fast;
-        launch_timed(ctx, kern, dim3(g), dim3(threads), a);
+        launch_timed(ctx, kern, dim3(g), dim3(T ? kPass : kPassU), a);
         M2D_HIP(hipGetLastError());
         ctx->last_pass = (deposit ? M2D_PASS_DEPOSIT : 0u) | (use_mcc ? M2D_PASS_MCC : 0u) |
                          (T ? M2D_PASS_TILED : 0u) | (fast ? M2D_PASS_FAST : bgrid ? M2D_PASS_BGRID : 0u) |
                          (pht ? M2D_PASS_PHT : 0u) | (hipos ? M2D_PASS_HIPOS : 0u);
     }
-    if (deposit || use_mcc) {
+    if (deposit || (use_mcc && !scat)) {
         // the grid flush, the next step's phase-applied tables (after a
         // specialised tiled pass, when they do not hold that phase yet) and
         // the collision queue in one launch.  The next phase is the one the
@@ -1443,17 +1495,6 @@ int m2d_advance_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s, const 
         const bool build_ph = fast_tiled && !f->p.selfconsistent && !(f->ph_valid && f->ph_phase == pb.ph);
         const unsigned ntab =
             build_ph ? (unsigned)((pb.nxe + pb.nze + kBlock * kPhPerThread - 1) / (kBlock * kPhPerThread)) : 0u;
-        // an interaction that turns its partner (COULOMB) scatters the queue
-        // in slot order after the flush, by one thread
-        const bool serial = use_mcc && mcc->h.partner_update;
-        // a target whose partner ensemble is this very store would read
-        // velocities that other collisions of the step are writing: the
-        // scatter then keeps its results in the queue, and k_scatter_apply
-        // stores them once every collision has read its partner
-        bool self_target = false;
-        if (use_mcc && !serial)
-            for (int t = 0; t < mcc->h.n_targets; t++) self_target |= mcc->h.t[t].px == p->x;
-        a.cq_defer = self_target ? 1 : 0;
         const unsigned g = nfl + ntab + (use_mcc && !serial ? kScatterBlocks : 0u);
         // without a deposit no flush block runs: n = 0 ends them at once
         const size_t nodes = deposit ? f->n : 0;
@@ -1484,7 +1525,7 @@ int m2d_advance_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s, const 
             M2D_HIP(hipGetLastError());
         }
     }
-    if (use_mcc) ctx->cq_dirty = false;
+    if (use_mcc && !scat) ctx->cq_dirty = false;
     if (stats) {
         M2D_TRY(read_counters(ctx));
         stats->removed = (int64_t)ctx->h_counters[CNT_REMOVED];
