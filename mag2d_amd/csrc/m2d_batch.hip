@@ -59,6 +59,8 @@ struct BatchArgs {
     uint64_t seed;
     const BatchRun *runs;
     const int64_t *offsets;  // n_runs + 1
+    const int64_t *threads;  // n_runs + 1: the first thread index of each run, counts rounded up to 4
+    int64_t n_threads;
     int n_runs;
     unsigned long long *counters;
 };
@@ -76,11 +78,35 @@ __device__ __forceinline__ int run_of(const int64_t *off, int n_runs, int64_t p)
 // one particle state carried across the steps of a segment
 struct BP {
     float x, z, vx, vy, vz;
-    float xl, zl;   // position remainders (HIPOS)
+    float xl, zl;       // position remainders (HIPOS)
     bool live;
+    bool free_;         // the cell of the last step's end is free (looked up, not yet acted on)
     int r;
-    uint32_t slot;  // slot within its run
+    uint32_t slot;      // slot within its run
+    double amp;         // of its run
+    uint64_t trial_thr;
+    uint32_t trial[4];  // the slot's trial words of four steps
 };
+
+// A quad's slots share each step's trial block, so lane j computes the block
+// of step s + j and the quad's words are exchanged: trial[j] of a lane is its
+// own slot's word at step s + j.  Called by whole quads.
+__device__ __forceinline__ void quad_trials(BP &q, uint64_t step, uint64_t seed, uint32_t stream)
+{
+    const int l = __lane_id() & 3;
+    const uint64_t mine = step + (uint64_t)l;
+    uint32_t c0 = q.slot >> 2, c1 = (uint32_t)mine, c2 = 0u;
+    uint32_t c3 = (kPurposeTrial << 24) | ((uint32_t)(mine >> 32) & 0xFFFFFFu);
+    philox4x32_10(c0, c1, c2, c3, (uint32_t)seed, (uint32_t)(seed >> 32) ^ stream);
+    auto own = [&](uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3) {
+        const uint32_t a = (l & 1) ? w1 : w0, b = (l & 1) ? w3 : w2;
+        return (l & 2) ? b : a;
+    };
+    q.trial[0] = own(quad_lane<0>(c0), quad_lane<0>(c1), quad_lane<0>(c2), quad_lane<0>(c3));
+    q.trial[1] = own(quad_lane<1>(c0), quad_lane<1>(c1), quad_lane<1>(c2), quad_lane<1>(c3));
+    q.trial[2] = own(quad_lane<2>(c0), quad_lane<2>(c1), quad_lane<2>(c2), quad_lane<2>(c3));
+    q.trial[3] = own(quad_lane<3>(c0), quad_lane<3>(c1), quad_lane<3>(c2), quad_lane<3>(c3));
+}
 
 // segment of `nsteps` steps from step niter0 for PPT particles per thread;
 // cosv[s] = cos of the RF phase at step niter0 + s.  FASTG: the fields and
@@ -88,8 +114,18 @@ struct BP {
 // 0, no wrap, no constant field, origin 0, free-cell test on), whose gather
 // is the FP32 origin-0 one; the same gather here keeps the runs bit for bit.
 // HIPOS: long-time positions (FP32 pairs), as in m2d_advance_2d.
+//
+// A step is a chain of two table lookups (the gather, then the free cell of
+// the new position), so it needs wavefronts: the scatter's FP64 chain, which
+// runs once in thousands of particle steps, took 203 VGPRs and left two a
+// SIMD.  Four (128 VGPRs) spill around the scatter.  The free-cell answer is
+// awaited in the next step, behind that step's gather, and a quad's four
+// lanes share the trial blocks of four steps (quad_trials).  256 runs of
+// 5000 ions, 400 steps: 9.6 ms before, 7.05 with four wavefronts alone, 6.26
+// now; three wavefronts 6.57, five 8.4.
 template <int PPT, bool FASTG, bool HIPOS>
-__global__ void __launch_bounds__(256) k_batch2d(BatchArgs a, uint64_t niter0, int nsteps, const double *cosv)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+k_batch2d(BatchArgs a, uint64_t niter0, int nsteps, const double *cosv)
 {
     const int64_t nthreads = (int64_t)gridDim.x * blockDim.x;
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -98,17 +134,29 @@ __global__ void __launch_bounds__(256) k_batch2d(BatchArgs a, uint64_t niter0, i
     bool nan_any = false;
 #pragma unroll
     for (int k = 0; k < PPT; k++) {
-        const int64_t p = gid + k * nthreads;
+        const int64_t t = gid + k * nthreads;
         q[k].live = false;
-        if (p < a.n) {
-            q[k].x = a.x[p];
-            q[k].live = !is_dead(q[k].x);
-            if (q[k].live) {
-                q[k].z = a.z[p]; q[k].vx = a.vx[p]; q[k].vy = a.vy[p]; q[k].vz = a.vz[p];
-                q[k].xl = HIPOS ? a.xl[p] : 0.f;
-                q[k].zl = HIPOS ? a.zl[p] : 0.f;
-                q[k].r = run_of(a.offsets, a.n_runs, p);
-                q[k].slot = (uint32_t)(p - a.runs[q[k].r].off);
+        q[k].free_ = true;
+        q[k].r = 0;
+        q[k].slot = 0;
+        q[k].amp = 0.0;
+        q[k].trial_thr = 0;
+        if (t < a.n_threads) {
+            const int r = run_of(a.threads, a.n_runs, t);
+            const BatchRun &R = a.runs[r];
+            q[k].r = r;
+            q[k].slot = (uint32_t)(t - a.threads[r]);
+            q[k].amp = R.amp;
+            q[k].trial_thr = R.trial_thr;
+            const int64_t p = R.off + q[k].slot;
+            if (p < a.offsets[r + 1]) {
+                q[k].x = a.x[p];
+                q[k].live = !is_dead(q[k].x);
+                if (q[k].live) {
+                    q[k].z = a.z[p]; q[k].vx = a.vx[p]; q[k].vy = a.vy[p]; q[k].vz = a.vz[p];
+                    q[k].xl = HIPOS ? a.xl[p] : 0.f;
+                    q[k].zl = HIPOS ? a.zl[p] : 0.f;
+                }
             }
         }
     }
@@ -117,18 +165,23 @@ __global__ void __launch_bounds__(256) k_batch2d(BatchArgs a, uint64_t niter0, i
         const double cs = cosv[s];
 #pragma unroll
         for (int k = 0; k < PPT; k++) {
+            if (__ballot(q[k].live) == 0ull) continue;  // uniform
+            if ((s & 3) == 0 && q[k].trial_thr) quad_trials(q[k], step, a.seed, a.runs[q[k].r].stream);
             if (!q[k].live) continue;
-            const BatchRun &R = a.runs[q[k].r];
             // the per-step phase of m2d_advance_2d, rounded the same way (no contraction)
-            const float ph = (float)__dadd_rn(__dmul_rn(R.amp, cs), a.U0);
+            const float ph = (float)__dadd_rn(__dmul_rn(q[k].amp, cs), a.U0);
             float x = q[k].x, z = q[k].z, vx = q[k].vx, vy = q[k].vy, vz = q[k].vz;
             float xl = q[k].xl, zl = q[k].zl;
             float ex, ez;
+            bool out = false;
             if constexpr (FASTG) {
-                if (gather_E_f(a, x, xl, z, zl, ph, ex, ez)) raise_flag(a.counters, M2D_FLAG_OUT_OF_RANGE);
+                out = gather_E_f(a, x, xl, z, zl, ph, ex, ez);
             } else {
                 gather_E(a, HIPOS ? pos64(x, xl) : (double)x, HIPOS ? pos64(z, zl) : (double)z, ph, ex, ez);
             }
+            // the last step's cell was not free: the particle ended there
+            if (!q[k].free_) { q[k].live = false; n_removed++; continue; }
+            if (FASTG && out) raise_flag(a.counters, M2D_FLAG_OUT_OF_RANGE);
             vx = fmaf(ex, a.qmdt2, vx);
             vz = fmaf(ez, a.qmdt2, vz);
             if (a.rotate) {
@@ -148,13 +201,11 @@ __global__ void __launch_bounds__(256) k_batch2d(BatchArgs a, uint64_t niter0, i
                 x = fmaf(vx, a.dt, x);
                 z = fmaf(vz, a.dt, z);
             }
-            if (R.trial_thr) {
-                // the trial word of slot s: word s%4 of the Philox block (s/4, step, 0, purpose 2)
-                uint32_t c0 = q[k].slot >> 2, c1 = (uint32_t)step, c2 = 0u;
-                uint32_t c3 = (kPurposeTrial << 24) | ((uint32_t)(step >> 32) & 0xFFFFFFu);
-                philox4x32_10(c0, c1, c2, c3, (uint32_t)a.seed, (uint32_t)(a.seed >> 32) ^ R.stream);
-                const uint32_t w = (q[k].slot & 3) == 0 ? c0 : (q[k].slot & 3) == 1 ? c1 : (q[k].slot & 3) == 2 ? c2 : c3;
-                if ((uint64_t)w < R.trial_thr) {
+            if (q[k].trial_thr) {
+                const uint32_t w = (s & 2) ? ((s & 1) ? q[k].trial[3] : q[k].trial[2])
+                                           : ((s & 1) ? q[k].trial[1] : q[k].trial[0]);
+                if ((uint64_t)w < q[k].trial_thr) {
+                    const BatchRun &R = a.runs[q[k].r];
                     Rng rg;
                     rg.begin(a.seed, R.stream, q[k].slot, step, kPurposeMcc);
                     scatter(*R.mcc, rg, vx, vy, vz, a.counters);
@@ -182,22 +233,24 @@ __global__ void __launch_bounds__(256) k_batch2d(BatchArgs a, uint64_t niter0, i
                 }
             }
             if (!dead && a.checkfree) {
-                bool fr = false;
+                bool in_grid;
+                int cell = 0;
                 if constexpr (FASTG) {
                     // the cell of the specialised single-run pass (the box test gave x, z >= 0)
                     int ci, cj;
                     float u, ou;
                     cell_f(x, xl, a.idxh, a.idxl, ci, u, ou);
                     cell_f(z, zl, a.idzh, a.idzl, cj, u, ou);
-                    if ((unsigned)ci <= (unsigned)(a.nx - 1) && (unsigned)cj <= (unsigned)(a.nz - 1))
-                        fr = a.cellfree[ci * a.nz + cj] != 0;
+                    in_grid = (unsigned)ci <= (unsigned)(a.nx - 1) && (unsigned)cj <= (unsigned)(a.nz - 1);
+                    if (in_grid) cell = ci * a.nz + cj;
                 } else {
                     const double X = ((HIPOS ? pos64(x, xl) : (double)x) - a.xmin) * a.idx;
                     const double Z = ((HIPOS ? pos64(z, zl) : (double)z) - a.zmin) * a.idz;
-                    if (X >= 0.0 && X < (double)a.nx && Z >= 0.0 && Z < (double)a.nz)
-                        fr = a.cellfree[(int)X * a.nz + (int)Z] != 0;
+                    in_grid = X >= 0.0 && X < (double)a.nx && Z >= 0.0 && Z < (double)a.nz;
+                    if (in_grid) cell = (int)X * a.nz + (int)Z;
                 }
-                dead = !fr;
+                dead = !in_grid;
+                if (in_grid) q[k].free_ = a.cellfree[cell] != 0;
             }
             if (dead) { q[k].live = false; n_removed++; }
             q[k].x = x; q[k].z = z; q[k].vx = vx; q[k].vy = vy; q[k].vz = vz;
@@ -206,8 +259,11 @@ __global__ void __launch_bounds__(256) k_batch2d(BatchArgs a, uint64_t niter0, i
     }
 #pragma unroll
     for (int k = 0; k < PPT; k++) {
-        const int64_t p = gid + k * nthreads;
-        if (p >= a.n || is_dead(a.x[p])) continue;
+        const int64_t t = gid + k * nthreads;
+        if (t >= a.n_threads) continue;
+        const int64_t p = a.runs[q[k].r].off + q[k].slot;
+        if (p >= a.offsets[q[k].r + 1] || is_dead(a.x[p])) continue;
+        if (q[k].live && !q[k].free_) { q[k].live = false; n_removed++; }
         if (!q[k].live) { a.x[p] = dead_value(); continue; }
         a.x[p] = q[k].x; a.z[p] = q[k].z; a.vx[p] = q[k].vx; a.vy[p] = q[k].vy; a.vz[p] = q[k].vz;
         if (HIPOS) { a.xl[p] = q[k].xl; a.zl[p] = q[k].zl; }
@@ -271,6 +327,7 @@ struct m2d_batch {
     m2d_species2d s{};
     m2d_particles2d p{};
     int n_runs = 0;
+    int64_t n_threads = 0;    // sum of the runs' counts rounded up to 4
     m2d::BatchRun *d_runs = nullptr;
     int64_t *d_off = nullptr;
     std::vector<int64_t> off;
@@ -331,6 +388,8 @@ static void batch_args(const m2d_batch *b, const m2d_particles2d &p, BatchArgs &
     a.seed = b->ctx->seed;
     a.runs = b->d_runs;
     a.offsets = b->d_off;
+    a.threads = b->d_off + b->n_runs + 1;
+    a.n_threads = b->n_threads;
     a.n_runs = b->n_runs;
     a.counters = b->ctx->counters;
 }
@@ -376,7 +435,7 @@ static int launch_segment(m2d_batch *b, const m2d_particles2d &p, const m2d_batc
 {
     BatchArgs a;
     batch_args(b, p, a);
-    const int64_t threads = (p.n + sh.ppt - 1) / sh.ppt;
+    const int64_t threads = (b->n_threads + sh.ppt - 1) / sh.ppt;
     const unsigned grid = (unsigned)std::max<int64_t>(1, (threads + sh.block - 1) / sh.block);
     hipStream_t st = b->ctx->stream;
     const bool fastg = a.checkfree && !a.rotate && !a.periodic && !a.econst && a.xmin == 0.0 && a.zmin == 0.0;
@@ -430,6 +489,12 @@ int m2d_batch_create(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s, cons
     b->p = *p;
     b->n_runs = d->n_runs;
     b->off.assign(d->offset, d->offset + d->n_runs + 1);
+    std::vector<int64_t> off(b->off);  // on the device: the offsets, then the threads' (see BatchArgs)
+    for (int r = 0; r < d->n_runs; r++) {
+        off.push_back(b->n_threads);
+        b->n_threads += (d->offset[r + 1] - d->offset[r] + 3) / 4 * 4;
+    }
+    off.push_back(b->n_threads);
     std::vector<BatchRun> runs((size_t)d->n_runs);
     for (int r = 0; r < d->n_runs; r++) {
         BatchRun &R = runs[(size_t)r];
@@ -457,12 +522,12 @@ int m2d_batch_create(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s, cons
     }
     auto fail = [&](int code) { m2d_batch_destroy(b); return code; };
     if (hipMalloc((void **)&b->d_runs, sizeof(BatchRun) * runs.size()) != hipSuccess ||
-        hipMalloc((void **)&b->d_off, sizeof(int64_t) * b->off.size()) != hipSuccess ||
+        hipMalloc((void **)&b->d_off, sizeof(int64_t) * off.size()) != hipSuccess ||
         hipMalloc((void **)&b->esum, sizeof(double) * (size_t)d->n_runs) != hipSuccess ||
         hipMalloc((void **)&b->ecount, sizeof(unsigned long long) * (size_t)d->n_runs) != hipSuccess)
         return fail(set_error(M2D_ERR_NO_MEMORY, "m2d_batch_create: device allocation"));
     if (hipMemcpy(b->d_runs, runs.data(), sizeof(BatchRun) * runs.size(), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(b->d_off, b->off.data(), sizeof(int64_t) * b->off.size(), hipMemcpyHostToDevice) != hipSuccess)
+        hipMemcpy(b->d_off, off.data(), sizeof(int64_t) * off.size(), hipMemcpyHostToDevice) != hipSuccess)
         return fail(set_error(M2D_ERR_HIP, "m2d_batch_create: upload"));
     ctx_retain(ctx);
     b->retained = true;
