@@ -65,14 +65,34 @@ struct AdjArgs {
 
 __device__ __forceinline__ double uat(const double *u, int nz, int i, int j) { return u[(size_t)i * nz + j]; }
 
-// lu contributions of one particle: 8 node updates of the x component and 8
-// of the z component of the gather transpose
+// lu contributions of one particle, the transpose of its gather: the x
+// component's nodes are rows xr - 1 .. xr + 1 of columns xc, xc + 1, the z
+// component's columns zc - 1 .. zc + 1 of rows zr, zr + 1.  (An edge e with
+// weight t adds t to its upper node and -t to its lower one; neighbouring
+// edges share the middle node, and two edges clamped onto one fall together.)
 struct LuAdd {
-    int row[16], col[16];
-    double val[16];
-    int n = 0;
-    __device__ void add(int r, int c, double v) { row[n] = r; col[n] = c; val[n] = v; n++; }
+    int xr, xc, zr, zc;
+    double x[3][2], z[2][3];
+    template <class F>
+    __device__ __forceinline__ void each(const F &f) const
+    {
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+#pragma unroll
+            for (int d = 0; d < 2; d++) {
+                if (x[r][d] != 0.0) f(xr - 1 + r, xc + d, x[r][d]);
+                if (z[d][r] != 0.0) f(zr + d, zc - 1 + r, z[d][r]);
+            }
+    }
 };
+
+// the smallest v of the wavefront, in every lane
+__device__ __forceinline__ int wave_min(int v)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
+    return v;
+}
 
 constexpr int kAdjWin = 2304;  // doubles of the block's LDS window (18 KiB)
 
@@ -148,7 +168,10 @@ __global__ void __launch_bounds__(256) k_adj_scatter2d(AdjArgs a)
 
 // one reverse step for every particle (see the header comment); the gather
 // transpose is summed in an LDS window over the block's node bounding box
-// when it fits, else added to lu directly
+// when it fits, else added to lu directly.  A particle's 16 updates meet at
+// 12 nodes, which stay in registers: as arrays of rows, columns and values
+// they lay in scratch memory, 256 bytes a thread (250k electrons 50.7 us a
+// step, now 15.6).
 __global__ void __launch_bounds__(256) k_adj_step2d(AdjArgs a)
 {
     __shared__ double win[kAdjWin];
@@ -211,45 +234,51 @@ __global__ void __launch_bounds__(256) k_adj_step2d(AdjArgs a)
             lx += lEx * dExdx + lEz * dEzdx;
             lz += lEx * dExdz + lEz * dEzdz;
             // transpose of the gather
-            for (int c = 0; c < 2; c++)
-                for (int d = 0; d < 2; d++) {
-                    const double tx = -lEx * wx[c][d] * a.idx;
-                    L.add(er[c], jx + d, tx);
-                    L.add(er[c] - 1, jx + d, -tx);
-                    const double tz = -lEz * wz[c][d] * a.idz;
-                    L.add(i0 + c, ec[d], tz);
-                    L.add(i0 + c, ec[d] - 1, -tz);
-                }
+            const bool xs = er[1] == er[0], zs = ec[1] == ec[0];  // both edges clamped onto one
+            L.xr = er[0]; L.xc = jx; L.zr = i0; L.zc = ec[0];
+#pragma unroll
+            for (int d = 0; d < 2; d++) {
+                const double t0 = -lEx * wx[0][d] * a.idx, t1 = -lEx * wx[1][d] * a.idx;
+                L.x[0][d] = xs ? -t0 - t1 : -t0;
+                L.x[1][d] = xs ? t0 + t1 : t0 - t1;
+                L.x[2][d] = xs ? 0.0 : t1;
+                const double s0 = -lEz * wz[d][0] * a.idz, s1 = -lEz * wz[d][1] * a.idz;
+                L.z[d][0] = zs ? -s0 - s1 : -s0;
+                L.z[d][1] = zs ? s0 + s1 : s0 - s1;
+                L.z[d][2] = zs ? 0.0 : s1;
+            }
             a.lx[p] = lx; a.lz[p] = lz;
             a.lvx[p] = lvx; a.lvy[p] = lvy; a.lvz[p] = lvz;
         }
     }
     __syncthreads();
-    if (active) {
-        int r0 = nx, r1 = -1, c0 = nz, c1 = -1;
-        for (int k = 0; k < L.n; k++) {
-            r0 = min(r0, L.row[k]); r1 = max(r1, L.row[k]);
-            c0 = min(c0, L.col[k]); c1 = max(c1, L.col[k]);
-        }
+    // the bounding box of nodes with a contribution
+    int r0 = nx, r1 = -1, c0 = nz, c1 = -1;
+    if (active)
+        L.each([&](int r, int c, double) {
+            r0 = min(r0, r); r1 = max(r1, r);
+            c0 = min(c0, c); c1 = max(c1, c);
+        });
+    r0 = wave_min(r0); r1 = -wave_min(-r1);
+    c0 = wave_min(c0); c1 = -wave_min(-c1);
+    if (__lane_id() == 0 && r1 >= 0) {
         atomicMin(&bb[0], r0); atomicMax(&bb[1], r1);
         atomicMin(&bb[2], c0); atomicMax(&bb[3], c1);
     }
     __syncthreads();
     const int R0 = bb[0], C0 = bb[2], W = bb[3] - bb[2] + 1, H = bb[1] - bb[0] + 1;
-    if (H <= 0) return;  // uniform: no active particle in the block
+    if (H <= 0) return;  // uniform: no contribution in the block
     if (H * W <= kAdjWin) {
         for (int k = threadIdx.x; k < H * W; k += blockDim.x) win[k] = 0.0;
         __syncthreads();
-        for (int k = 0; k < L.n; k++)
-            if (L.val[k] != 0.0) atomicAdd(&win[(L.row[k] - R0) * W + (L.col[k] - C0)], L.val[k]);
+        if (active) L.each([&](int r, int c, double v) { atomicAdd(&win[(r - R0) * W + (c - C0)], v); });
         __syncthreads();
         for (int k = threadIdx.x; k < H * W; k += blockDim.x) {
             const double v = win[k];
             if (v != 0.0) atomicAdd(a.lu + (size_t)(R0 + k / W) * nz + (C0 + k % W), v);
         }
-    } else {
-        for (int k = 0; k < L.n; k++)
-            if (L.val[k] != 0.0) atomicAdd(a.lu + (size_t)L.row[k] * nz + L.col[k], L.val[k]);
+    } else if (active) {
+        L.each([&](int r, int c, double v) { atomicAdd(a.lu + (size_t)r * nz + c, v); });
     }
 }
 
