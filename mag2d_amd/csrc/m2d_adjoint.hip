@@ -447,7 +447,10 @@ int m2d_adjoint_energy_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s,
             for (int c = 0; c < 5; c++)
                 M2D_HIP(hipMemcpyAsync(ckpt.as<float>() + ((size_t)(n / K) * 5 + c) * np, parr[c],
                                        sizeof(float) * np, hipMemcpyDeviceToDevice, st));
-        M2D_TRY(m2d_fields2d_solve(f, M2D_SOLVE_STATIC, 1e-10, &si));
+        // the differentiated run and its reverse sweep keep the multigrid
+        // solve: a gradient carries its solves' 1e-10 in full (the direct
+        // solve moved one of a small run by 3e-9)
+        M2D_TRY(fields_solve_multigrid(f, M2D_SOLVE_STATIC, 1e-10, &si));
         if (grad)
             M2D_HIP(hipMemcpyAsync(U.as<double>() + (size_t)n * nc, f->u, sizeof(double) * nc,
                                    hipMemcpyDeviceToDevice, st));
@@ -574,7 +577,7 @@ int m2d_adjoint_energy_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s,
             // A_FF y = lu_F
             k_adj_rhs<<<gb, 256, 0, st>>>(f->mask, lu.as<double>(), af->rho, nc);
             M2D_HIP(hipGetLastError());
-            M2D_TRY(m2d_fields2d_solve(af, M2D_SOLVE_RAW, adj_tol, &si));
+            M2D_TRY(fields_solve_multigrid(af, M2D_SOLVE_RAW, adj_tol, &si));
             k_adj_groups<<<gb, 256, 0, st>>>(f->mask, dgroup.as<int>(), lu.as<double>(), af->u, f->nx, f->nz,
                                              cfg->n_groups, gpart.as<double>());
             k_adj_groups_sum<<<cfg->n_groups, 256, 0, st>>>(gpart.as<double>(), (int)gb, cfg->n_groups,

@@ -1418,8 +1418,9 @@ static int refine_direct(m2d_fields2d *f, double *u, double tol)
 }
 
 // FP64 iterative refinement of u over FP32 multigrid-preconditioned CG
-// passes, queued whole (queue_refinement)
-static int solve(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info)
+// passes, queued whole (queue_refinement); direct: where the field has the
+// direct solve
+static int solve(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info, bool direct)
 {
     hipStream_t s = f->ctx->stream;
     Mg &mg = f->mg;
@@ -1431,7 +1432,7 @@ static int solve(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info)
     SolveCtl *ctl = solve_ctl(mg);
     SolveCtl *h = (SolveCtl *)(mg.h_dots + 16);
     queue_first_residual(f, u, mode, scale, tol, kMaxOuter);
-    if (f->direct.on)
+    if (direct)
         M2D_TRY(refine_direct(f, u, tol));
     else
         M2D_TRY(queue_refinement(
@@ -1446,6 +1447,17 @@ static int solve(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info)
         return set_error(M2D_ERR_NOT_CONVERGED, "Fields solve: relative residual %.3e > %.3e after %d steps",
                          h->rel, tol, h->outer);
     return M2D_OK;
+}
+
+int fields_solve_multigrid(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info)
+{
+    if (f->direct.on && f->mg_late != 1) {
+        M2D_CHECK(f->mg_late == 0, M2D_ERR_NO_MEMORY, "Fields solve: the multigrid set-up failed before");
+        f->mg_late = -1;
+        M2D_TRY(mg_setup(f));
+        f->mg_late = 1;
+    }
+    return solve(f, mode, tol, info, false);
 }
 
 }  // namespace m2d
@@ -1694,7 +1706,7 @@ int m2d_fields2d_solve(m2d_fields2d *f, int mode, double tol, m2d_solve_info *in
     M2D_CHECK(f, M2D_ERR_BAD_ARG, "m2d_fields2d_solve: NULL argument");
     M2D_CHECK(mode == M2D_SOLVE_STATIC || mode == M2D_SOLVE_RF || mode == M2D_SOLVE_RAW, M2D_ERR_BAD_ARG,
               "m2d_fields2d_solve: unknown mode %d", mode);
-    return solve(f, mode, tol, info);
+    return solve(f, mode, tol, info, f->direct.on);
 }
 
 }  // extern "C"

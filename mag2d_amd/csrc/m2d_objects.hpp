@@ -112,7 +112,8 @@ struct m2d_fields2d {
     m2d_grid2d bgrid{};
     double *smooth_tmp = nullptr;  // nx*nz copy of the field u_smooth filters
     m2d::Mg mg;
-    m2d::Direct2 direct;          // on: the solve is direct, and mg holds no levels
+    m2d::Direct2 direct;          // on: the solve is direct, and mg holds no levels (but see mg_late)
+    int mg_late = 0;              // levels of a direct field (fields_solve_multigrid): 1 there, -1 failed
     std::vector<uint8_t> h_mask;
 };
 
@@ -126,6 +127,9 @@ struct m2d_mcc {
 
 namespace m2d {
 int fields_build_tables(m2d_fields2d *f);
+// m2d_fields2d_solve by multigrid-PCG, also where the field has the direct
+// solve: a field's first such call sets the levels up, which it then keeps
+int fields_solve_multigrid(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info);
 bool direct2d_fits(const std::vector<uint8_t> &mask, int nx, int nz, Direct2 &d);
 int direct2d_setup(m2d_fields2d *f);
 int direct2d_pass(m2d_fields2d *f, double *u, SolveCtl *ctl);
