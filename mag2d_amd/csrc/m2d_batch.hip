@@ -173,15 +173,17 @@ k_batch2d(BatchArgs a, uint64_t niter0, int nsteps, const double *cosv)
             float x = q[k].x, z = q[k].z, vx = q[k].vx, vy = q[k].vy, vz = q[k].vz;
             float xl = q[k].xl, zl = q[k].zl;
             float ex, ez;
-            bool out = false;
+            bool out;
             if constexpr (FASTG) {
                 out = gather_E_f(a, x, xl, z, zl, ph, ex, ez);
             } else {
-                gather_E(a, HIPOS ? pos64(x, xl) : (double)x, HIPOS ? pos64(z, zl) : (double)z, ph, ex, ez);
+                out = gather_E_clamped(a, HIPOS ? pos64(x, xl) : (double)x, HIPOS ? pos64(z, zl) : (double)z, ph, ex,
+                                       ez);
             }
-            // the last step's cell was not free: the particle ended there
+            // the last step's cell was not free: the particle ended there, and
+            // its gather does not count
             if (!q[k].free_) { q[k].live = false; n_removed++; continue; }
-            if (FASTG && out) raise_flag(a.counters, M2D_FLAG_OUT_OF_RANGE);
+            if (out) raise_flag(a.counters, M2D_FLAG_OUT_OF_RANGE);
             vx = fmaf(ex, a.qmdt2, vx);
             vz = fmaf(ez, a.qmdt2, vz);
             if (a.rotate) {
