@@ -142,4 +142,19 @@ inline bool mcc_partners_alias(const m2d_mcc *m, const void *x)
         if ((const void *)m->h.t[t].px == x) return true;
     return false;
 }
+// some target draws its partners from memory that a step of the store p
+// writes: p itself, or a part of it, or a store that shares some of its arrays
+inline bool mcc_partners_overlap(const m2d_mcc *m, const m2d_particles2d *p)
+{
+    const float *const own[7] = {p->x, p->z, p->vx, p->vy, p->vz, p->xl, p->zl};
+    for (int t = 0; t < m->h.n_targets; t++) {
+        const McTarget &T = m->h.t[t];
+        if (!T.px || T.pn <= 0) continue;
+        for (const float *q : {T.px, (const float *)T.pvx, (const float *)T.pvy, (const float *)T.pvz})
+            for (const float *o : own)
+                if (q && o && (uintptr_t)q < (uintptr_t)(o + p->n) && (uintptr_t)o < (uintptr_t)(q + T.pn))
+                    return true;
+    }
+    return false;
+}
 }  // namespace m2d

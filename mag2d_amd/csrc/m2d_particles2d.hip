@@ -1410,13 +1410,12 @@ int m2d_advance_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s, const 
     // an interaction that turns its partner (COULOMB) scatters the queue
     // in slot order after the flush, by one thread
     const bool serial = use_mcc && mcc->h.partner_update;
-    // a target whose partner ensemble is this very store would read
-    // velocities that other collisions of the step are writing: the
-    // scatter then keeps its results in the queue, and k_scatter_apply
-    // stores them once every collision has read its partner
-    bool self_target = false;
-    if (use_mcc && !serial)
-        for (int t = 0; t < mcc->h.n_targets; t++) self_target |= mcc->h.t[t].px == p->x;
+    // a target whose partner ensemble is this very store, or shares memory
+    // with it, would read velocities that other collisions of the step are
+    // writing (and, scattered in the pass, that the push has not written
+    // yet): the scatter then keeps its results in the queue, and
+    // k_scatter_apply stores them once every collision has read its partner
+    const bool self_target = use_mcc && !serial && mcc_partners_overlap(mcc, p);
     a.cq_defer = self_target ? 1 : 0;
     const bool scat = use_mcc && !serial && !self_target && !deposit;
     unsigned long long *next_len = nullptr;

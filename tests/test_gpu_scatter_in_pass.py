@@ -1,6 +1,8 @@
 """Collisions scattered inside the pass (a step without a deposit) against
 those that a launch after the pass takes from the queue (a step with one):
-the same draws from the same velocities, so the same bits."""
+the same draws from the same velocities, so the same bits.  And partners that
+are part of the colliding store, which every collision reads as the push left
+them."""
 import numpy as np
 import pytest
 
@@ -37,3 +39,33 @@ def test_pass_and_queue_agree(ctx, n, density, field, hipos):
     assert n < 255 or sum(c for c, _ in out[0][1]) > 0
     for k in out[0][0]:
         assert np.array_equal(out[0][0][k], out[1][0][k]), k
+
+
+@pytest.mark.parametrize("deposit", [False, True])
+@pytest.mark.parametrize("part", [slice(0, None), slice(1, None), slice(500_000, None), slice(0, 300_001)])
+def test_partners_from_a_part_of_the_store(ctx, part, deposit):
+    """Charge exchange of ions that move alike with partners from their own
+    store: whichever partner is drawn, the velocity it hands over is the one
+    after the push, so all ions end with that velocity."""
+    n, g = 1_000_000, abi.grid2d(64, 64, 1e-3, 1e-3)
+    L = 63e-3
+    mask, volt = abi.grid_build(g, abi.GEO_EMPTY, L, L)
+    prm = abi.FieldsParams(g, L, L, 1, 0, 0, abi.BC_FREE, 2e3, 0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 1e-12)
+    fields = abi.Fields2D(ctx, prm, mask, volt)
+    rng = np.random.default_rng(3)
+    x, z = ((20e-3 + 20e-3 * rng.uniform(size=n)).astype(np.float32) for _ in range(2))
+    v = [np.full(n, c, np.float32) for c in (100.0, -50.0, 70.0)]
+    P = abi.ParticlesSoA.from_host(ctx, x, z, *v)
+    at = range(n)[part]
+    partner = abi.Particles2D(*(P.arr[k].ptr + 4 * at.start for k in P.NAMES), len(at))
+    mcc = abi.Mcc(ctx, M_ION, [abi.Target(M_ION, 1e24, 300.0, 0.0, partner)],
+                  [abi.Interaction(abi.CX, 0, 0.0, 1e-15, 0.0, 0, 0)], 1.0)
+    rho = ctx.to_device(np.zeros(64 * 64))
+    flags = abi.STEP_PUSH | abi.STEP_BOUNDARY | (abi.STEP_DEPOSIT if deposit else 0)
+    st = abi.advance(ctx, fields, species(QE, M_ION, 1e-9, mcc.lifetime), P, mcc=mcc,
+                     rho_ptr=rho.ptr if deposit else None, flags=flags, want_stats=True)
+    assert st.collisions > n // 2 and st.removed == 0
+    d = P.download()
+    for k, old in zip(("vx", "vy", "vz"), v):
+        assert len(np.unique(d[k])) == 1, k
+    assert any(d[k][0] != c[0] for k, c in zip(("vx", "vy", "vz"), v))
