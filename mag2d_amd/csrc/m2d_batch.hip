@@ -121,154 +121,171 @@ __device__ __forceinline__ void quad_trials(BP &q, uint64_t step, uint64_t seed,
 // SIMD.  Four (128 VGPRs) spill around the scatter.  The free-cell answer is
 // awaited in the next step, behind that step's gather, and a quad's four
 // lanes share the trial blocks of four steps (quad_trials).  256 runs of
-// 5000 ions, 400 steps: 9.6 ms before, 7.05 with four wavefronts alone, 6.26
-// now; three wavefronts 6.57, five 8.4.
+// 5000 ions, 400 steps, one particle a thread: 9.6 ms before, 7.05 with four
+// wavefronts alone, 6.26 now; three wavefronts 6.57, five 8.4.
+// Two particles a thread need 168 VGPRs: at four wavefronts their state
+// spills in the step itself.  256 runs of 6000 ions, 200 steps, at two, three
+// and four wavefronts: 3.03, 2.46 and 2.60 ms (with B 3.29, 2.67 and 3.20);
+// 16 runs of 1500: 459, 474 and 503 us (491, 501 and 660).
+// Four particles a thread run as two pairs, one after the other: as one array
+// their state lay in scratch memory (4.7 ms, and 6.9 with the trial words in
+// it too; the pairs 2.62).
+template <int PPT>
+constexpr int batch_waves()
+{
+    return PPT == 1 ? 4 : 3;
+}
+
 template <int PPT, bool FASTG, bool HIPOS>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(batch_waves<PPT>())))
 k_batch2d(BatchArgs a, uint64_t niter0, int nsteps, const double *cosv)
 {
     const int64_t nthreads = (int64_t)gridDim.x * blockDim.x;
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    BP q[PPT];
     int n_removed = 0, n_coll = 0;
     bool nan_any = false;
+    constexpr int G = PPT < 4 ? PPT : 2;
+#pragma unroll 1
+    for (int64_t first = gid; first < gid + PPT * nthreads; first += G * nthreads) {
+        BP q[G];
 #pragma unroll
-    for (int k = 0; k < PPT; k++) {
-        const int64_t t = gid + k * nthreads;
-        q[k].live = false;
-        q[k].free_ = true;
-        q[k].r = 0;
-        q[k].slot = 0;
-        q[k].amp = 0.0;
-        q[k].trial_thr = 0;
-        if (t < a.n_threads) {
-            const int r = run_of(a.threads, a.n_runs, t);
-            const BatchRun &R = a.runs[r];
-            q[k].r = r;
-            q[k].slot = (uint32_t)(t - a.threads[r]);
-            q[k].amp = R.amp;
-            q[k].trial_thr = R.trial_thr;
-            const int64_t p = R.off + q[k].slot;
-            if (p < a.offsets[r + 1]) {
-                q[k].x = a.x[p];
-                q[k].live = !is_dead(q[k].x);
-                if (q[k].live) {
-                    q[k].z = a.z[p]; q[k].vx = a.vx[p]; q[k].vy = a.vy[p]; q[k].vz = a.vz[p];
-                    q[k].xl = HIPOS ? a.xl[p] : 0.f;
-                    q[k].zl = HIPOS ? a.zl[p] : 0.f;
-                }
-            }
-        }
-    }
-    for (int s = 0; s < nsteps; s++) {
-        const uint64_t step = niter0 + (uint64_t)s;
-        const double cs = cosv[s];
-#pragma unroll
-        for (int k = 0; k < PPT; k++) {
-            if (__ballot(q[k].live) == 0ull) continue;  // uniform
-            if ((s & 3) == 0 && q[k].trial_thr) quad_trials(q[k], step, a.seed, a.runs[q[k].r].stream);
-            if (!q[k].live) continue;
-            // the per-step phase of m2d_advance_2d, rounded the same way (no contraction)
-            const float ph = (float)__dadd_rn(__dmul_rn(q[k].amp, cs), a.U0);
-            float x = q[k].x, z = q[k].z, vx = q[k].vx, vy = q[k].vy, vz = q[k].vz;
-            float xl = q[k].xl, zl = q[k].zl;
-            float ex, ez;
-            bool out;
-            if constexpr (FASTG) {
-                out = gather_E_f(a, x, xl, z, zl, ph, ex, ez);
-            } else {
-                out = gather_E_clamped(a, HIPOS ? pos64(x, xl) : (double)x, HIPOS ? pos64(z, zl) : (double)z, ph, ex,
-                                       ez);
-            }
-            // the last step's cell was not free: the particle ended there, and
-            // its gather does not count
-            if (!q[k].free_) { q[k].live = false; n_removed++; continue; }
-            if (out) raise_flag(a.counters, M2D_FLAG_OUT_OF_RANGE);
-            vx = fmaf(ex, a.qmdt2, vx);
-            vz = fmaf(ez, a.qmdt2, vz);
-            if (a.rotate) {
-                float vpr = vx - vy * a.tz + vz * a.ty;
-                float vpz = vz - vx * a.ty + vy * a.tx;
-                float vpt = vy - vz * a.tx + vx * a.tz;
-                vx = vx - vpt * a.sz + vpz * a.sy;
-                vy = vy - vpz * a.sx + vpr * a.sz;
-                vz = vz - vpr * a.sy + vpt * a.sx;
-            }
-            vx = fmaf(ex, a.qmdt2, vx);
-            vz = fmaf(ez, a.qmdt2, vz);
-            if constexpr (HIPOS) {
-                drift_pair(x, xl, vx, a.dt, a.dtl);
-                drift_pair(z, zl, vz, a.dt, a.dtl);
-            } else {
-                x = fmaf(vx, a.dt, x);
-                z = fmaf(vz, a.dt, z);
-            }
-            if (q[k].trial_thr) {
-                const uint32_t w = (s & 2) ? ((s & 1) ? q[k].trial[3] : q[k].trial[2])
-                                           : ((s & 1) ? q[k].trial[1] : q[k].trial[0]);
-                if ((uint64_t)w < q[k].trial_thr) {
-                    const BatchRun &R = a.runs[q[k].r];
-                    Rng rg;
-                    rg.begin(a.seed, R.stream, q[k].slot, step, kPurposeMcc);
-                    scatter(*R.mcc, rg, vx, vy, vz, a.counters);
-                    n_coll++;
-                }
-            }
-            // advance_boundary (particles.hpp:376-406), no deposit
-            bool dead = false;
-            const double xd = HIPOS ? pos64(x, xl) : (double)x, zd = HIPOS ? pos64(z, zl) : (double)z;
-            const bool inside = HIPOS ? xd >= a.xmin && xd <= a.xper && zd >= a.zmin && zd <= a.zper
-                                      : x >= a.fx0 && x <= a.fx1 && z >= a.fz0 && z <= a.fz1;
-            if (!inside) {
-                if (x != x || z != z) { dead = true; nan_any = true; }
-                else if (!a.periodic) dead = true;
-                else {
-                    double xm = fmod(xd, a.xper), zm = fmod(zd, a.zper);
-                    if (xm < 0) xm += a.xper;
-                    if (zm < 0) zm += a.zper;
-                    if constexpr (HIPOS) {
-                        pos_split(xm, x, xl);
-                        pos_split(zm, z, zl);
-                    } else {
-                        x = (float)xm; z = (float)zm;
+        for (int k = 0; k < G; k++) {
+            const int64_t t = first + k * nthreads;
+            q[k].live = false;
+            q[k].free_ = true;
+            q[k].r = 0;
+            q[k].slot = 0;
+            q[k].amp = 0.0;
+            q[k].trial_thr = 0;
+            if (t < a.n_threads) {
+                const int r = run_of(a.threads, a.n_runs, t);
+                const BatchRun &R = a.runs[r];
+                q[k].r = r;
+                q[k].slot = (uint32_t)(t - a.threads[r]);
+                q[k].amp = R.amp;
+                q[k].trial_thr = R.trial_thr;
+                const int64_t p = R.off + q[k].slot;
+                if (p < a.offsets[r + 1]) {
+                    q[k].x = a.x[p];
+                    q[k].live = !is_dead(q[k].x);
+                    if (q[k].live) {
+                        q[k].z = a.z[p]; q[k].vx = a.vx[p]; q[k].vy = a.vy[p]; q[k].vz = a.vz[p];
+                        q[k].xl = HIPOS ? a.xl[p] : 0.f;
+                        q[k].zl = HIPOS ? a.zl[p] : 0.f;
                     }
                 }
             }
-            if (!dead && a.checkfree) {
-                bool in_grid;
-                int cell = 0;
-                if constexpr (FASTG) {
-                    // the cell of the specialised single-run pass (the box test gave x, z >= 0)
-                    int ci, cj;
-                    float u, ou;
-                    cell_f(x, xl, a.idxh, a.idxl, ci, u, ou);
-                    cell_f(z, zl, a.idzh, a.idzl, cj, u, ou);
-                    in_grid = (unsigned)ci <= (unsigned)(a.nx - 1) && (unsigned)cj <= (unsigned)(a.nz - 1);
-                    if (in_grid) cell = ci * a.nz + cj;
-                } else {
-                    const double X = ((HIPOS ? pos64(x, xl) : (double)x) - a.xmin) * a.idx;
-                    const double Z = ((HIPOS ? pos64(z, zl) : (double)z) - a.zmin) * a.idz;
-                    in_grid = X >= 0.0 && X < (double)a.nx && Z >= 0.0 && Z < (double)a.nz;
-                    if (in_grid) cell = (int)X * a.nz + (int)Z;
-                }
-                dead = !in_grid;
-                if (in_grid) q[k].free_ = a.cellfree[cell] != 0;
-            }
-            if (dead) { q[k].live = false; n_removed++; }
-            q[k].x = x; q[k].z = z; q[k].vx = vx; q[k].vy = vy; q[k].vz = vz;
-            q[k].xl = xl; q[k].zl = zl;
         }
-    }
+        for (int s = 0; s < nsteps; s++) {
+            const uint64_t step = niter0 + (uint64_t)s;
+            const double cs = cosv[s];
 #pragma unroll
-    for (int k = 0; k < PPT; k++) {
-        const int64_t t = gid + k * nthreads;
-        if (t >= a.n_threads) continue;
-        const int64_t p = a.runs[q[k].r].off + q[k].slot;
-        if (p >= a.offsets[q[k].r + 1] || is_dead(a.x[p])) continue;
-        if (q[k].live && !q[k].free_) { q[k].live = false; n_removed++; }
-        if (!q[k].live) { a.x[p] = dead_value(); continue; }
-        a.x[p] = q[k].x; a.z[p] = q[k].z; a.vx[p] = q[k].vx; a.vy[p] = q[k].vy; a.vz[p] = q[k].vz;
-        if (HIPOS) { a.xl[p] = q[k].xl; a.zl[p] = q[k].zl; }
+            for (int k = 0; k < G; k++) {
+                if (__ballot(q[k].live) == 0ull) continue;  // uniform
+                if ((s & 3) == 0 && q[k].trial_thr) quad_trials(q[k], step, a.seed, a.runs[q[k].r].stream);
+                if (!q[k].live) continue;
+                // the per-step phase of m2d_advance_2d, rounded the same way (no contraction)
+                const float ph = (float)__dadd_rn(__dmul_rn(q[k].amp, cs), a.U0);
+                float x = q[k].x, z = q[k].z, vx = q[k].vx, vy = q[k].vy, vz = q[k].vz;
+                float xl = q[k].xl, zl = q[k].zl;
+                float ex, ez;
+                bool out;
+                if constexpr (FASTG) {
+                    out = gather_E_f(a, x, xl, z, zl, ph, ex, ez);
+                } else {
+                    out = gather_E_clamped(a, HIPOS ? pos64(x, xl) : (double)x, HIPOS ? pos64(z, zl) : (double)z, ph, ex,
+                                           ez);
+                }
+                // the last step's cell was not free: the particle ended there, and
+                // its gather does not count
+                if (!q[k].free_) { q[k].live = false; n_removed++; continue; }
+                if (out) raise_flag(a.counters, M2D_FLAG_OUT_OF_RANGE);
+                vx = fmaf(ex, a.qmdt2, vx);
+                vz = fmaf(ez, a.qmdt2, vz);
+                if (a.rotate) {
+                    float vpr = vx - vy * a.tz + vz * a.ty;
+                    float vpz = vz - vx * a.ty + vy * a.tx;
+                    float vpt = vy - vz * a.tx + vx * a.tz;
+                    vx = vx - vpt * a.sz + vpz * a.sy;
+                    vy = vy - vpz * a.sx + vpr * a.sz;
+                    vz = vz - vpr * a.sy + vpt * a.sx;
+                }
+                vx = fmaf(ex, a.qmdt2, vx);
+                vz = fmaf(ez, a.qmdt2, vz);
+                if constexpr (HIPOS) {
+                    drift_pair(x, xl, vx, a.dt, a.dtl);
+                    drift_pair(z, zl, vz, a.dt, a.dtl);
+                } else {
+                    x = fmaf(vx, a.dt, x);
+                    z = fmaf(vz, a.dt, z);
+                }
+                if (q[k].trial_thr) {
+                    const uint32_t w = (s & 2) ? ((s & 1) ? q[k].trial[3] : q[k].trial[2])
+                                               : ((s & 1) ? q[k].trial[1] : q[k].trial[0]);
+                    if ((uint64_t)w < q[k].trial_thr) {
+                        const BatchRun &R = a.runs[q[k].r];
+                        Rng rg;
+                        rg.begin(a.seed, R.stream, q[k].slot, step, kPurposeMcc);
+                        scatter(*R.mcc, rg, vx, vy, vz, a.counters);
+                        n_coll++;
+                    }
+                }
+                // advance_boundary (particles.hpp:376-406), no deposit
+                bool dead = false;
+                const double xd = HIPOS ? pos64(x, xl) : (double)x, zd = HIPOS ? pos64(z, zl) : (double)z;
+                const bool inside = HIPOS ? xd >= a.xmin && xd <= a.xper && zd >= a.zmin && zd <= a.zper
+                                          : x >= a.fx0 && x <= a.fx1 && z >= a.fz0 && z <= a.fz1;
+                if (!inside) {
+                    if (x != x || z != z) { dead = true; nan_any = true; }
+                    else if (!a.periodic) dead = true;
+                    else {
+                        double xm = fmod(xd, a.xper), zm = fmod(zd, a.zper);
+                        if (xm < 0) xm += a.xper;
+                        if (zm < 0) zm += a.zper;
+                        if constexpr (HIPOS) {
+                            pos_split(xm, x, xl);
+                            pos_split(zm, z, zl);
+                        } else {
+                            x = (float)xm; z = (float)zm;
+                        }
+                    }
+                }
+                if (!dead && a.checkfree) {
+                    bool in_grid;
+                    int cell = 0;
+                    if constexpr (FASTG) {
+                        // the cell of the specialised single-run pass (the box test gave x, z >= 0)
+                        int ci, cj;
+                        float u, ou;
+                        cell_f(x, xl, a.idxh, a.idxl, ci, u, ou);
+                        cell_f(z, zl, a.idzh, a.idzl, cj, u, ou);
+                        in_grid = (unsigned)ci <= (unsigned)(a.nx - 1) && (unsigned)cj <= (unsigned)(a.nz - 1);
+                        if (in_grid) cell = ci * a.nz + cj;
+                    } else {
+                        const double X = ((HIPOS ? pos64(x, xl) : (double)x) - a.xmin) * a.idx;
+                        const double Z = ((HIPOS ? pos64(z, zl) : (double)z) - a.zmin) * a.idz;
+                        in_grid = X >= 0.0 && X < (double)a.nx && Z >= 0.0 && Z < (double)a.nz;
+                        if (in_grid) cell = (int)X * a.nz + (int)Z;
+                    }
+                    dead = !in_grid;
+                    if (in_grid) q[k].free_ = a.cellfree[cell] != 0;
+                }
+                if (dead) { q[k].live = false; n_removed++; }
+                q[k].x = x; q[k].z = z; q[k].vx = vx; q[k].vy = vy; q[k].vz = vz;
+                q[k].xl = xl; q[k].zl = zl;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < G; k++) {
+            const int64_t t = first + k * nthreads;
+            if (t >= a.n_threads) continue;
+            const int64_t p = a.runs[q[k].r].off + q[k].slot;
+            if (p >= a.offsets[q[k].r + 1] || is_dead(a.x[p])) continue;
+            if (q[k].live && !q[k].free_) { q[k].live = false; n_removed++; }
+            if (!q[k].live) { a.x[p] = dead_value(); continue; }
+            a.x[p] = q[k].x; a.z[p] = q[k].z; a.vx[p] = q[k].vx; a.vy[p] = q[k].vy; a.vz[p] = q[k].vz;
+            if (HIPOS) { a.xl[p] = q[k].xl; a.zl[p] = q[k].zl; }
+        }
     }
     int sum = n_removed;
     for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
