@@ -495,7 +495,7 @@ int m2d_adjoint_energy_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s,
     m2d_fields2d *af = nullptr;
     {
         std::vector<double> zero(nc, 0.0);
-        M2D_TRY(m2d_fields2d_create(ctx, &f->p, f->h_mask.data(), zero.data(), &af));
+        M2D_TRY(fields_create(ctx, &f->p, f->h_mask.data(), zero.data(), false, &af));
     }
     struct Closer { m2d_fields2d *f; ~Closer() { m2d_fields2d_destroy(f); } } closer{af};
     AdjArgs a{};

@@ -1100,6 +1100,9 @@ static int mg_setup(m2d_fields2d *f)
         dirs.push_back(std::move(dc));
         dims.push_back({nxc, nzc});
     }
+    mg.coarse_n = dims.back().first * dims.back().second;
+    M2D_CHECK(ops.size() <= (size_t)kMaxLevels && mg.coarse_n <= 3200, M2D_ERR_BAD_ARG,
+              "Fields: multigrid hierarchy of %d levels, coarsest %d nodes", (int)ops.size(), mg.coarse_n);
     mg.lv.resize(ops.size());
     for (size_t l = 0; l < ops.size(); l++) {
         MgLevel &L = mg.lv[l];
@@ -1127,7 +1130,6 @@ static int mg_setup(m2d_fields2d *f)
     const MgLevel &C = mg.lv.back();
     M2D_CHECK(dense_inverse(ops.back(), dirs.back(), C.nx, C.nz, inv), M2D_ERR_BAD_ARG,
               "Fields: coarsest multigrid operator is singular");
-    mg.coarse_n = (int)C.n;
     M2D_TRY(dmalloc((void **)&mg.coarse_inv, sizeof(float) * inv.size()));
     M2D_HIP(hipMemcpy(mg.coarse_inv, inv.data(), sizeof(float) * inv.size(), hipMemcpyHostToDevice));
     {
@@ -1149,20 +1151,27 @@ static int mg_setup(m2d_fields2d *f)
     mg.lc = (int)mg.lv.size() - 1;
     for (int l = 1; l < (int)mg.lv.size(); l++)
         if (mg.lv[l].n <= kBlockLevelNodes) { mg.lc = l; break; }
-    M2D_CHECK(mg.lv.size() <= (size_t)kMaxLevels && mg.coarse_n <= 3200, M2D_ERR_BAD_ARG,
-              "Fields: multigrid hierarchy of %d levels, coarsest %d nodes", (int)mg.lv.size(), mg.coarse_n);
     return M2D_OK;
 }
 
-static void mg_free(Mg &mg)
+// what mg_setup allocates, whole or in part
+static void mg_free_levels(Mg &mg)
 {
     for (MgLevel &L : mg.lv)
         for (void *p : {(void *)L.st, (void *)L.dinv, (void *)L.dir, (void *)L.x, (void *)L.x2,
                         (void *)L.r, (void *)L.b})
             if (p) (void)hipFree(p);
     mg.lv.clear();
-    for (void *p : {(void *)mg.coarse_inv, (void *)mg.pr, (void *)mg.pz, (void *)mg.pp, (void *)mg.pp2, (void *)mg.pq,
-                    (void *)mg.pe, (void *)mg.r64, (void *)mg.dots, (void *)mg.partial, (void *)mg.ticket, (void *)mg.coarse_invT})
+    for (float **p : {&mg.coarse_inv, &mg.coarse_invT, &mg.pz, &mg.pp, &mg.pp2, &mg.pq, &mg.pe}) {
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+    }
+}
+
+static void mg_free(Mg &mg)
+{
+    mg_free_levels(mg);
+    for (void *p : {(void *)mg.pr, (void *)mg.r64, (void *)mg.dots, (void *)mg.partial, (void *)mg.ticket})
         if (p) (void)hipFree(p);
     if (mg.h_dots) (void)hipHostFree(mg.h_dots);
     mg = Mg();
@@ -1451,11 +1460,12 @@ static int solve(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info, bo
 
 int fields_solve_multigrid(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info)
 {
-    if (f->direct.on && f->mg_late != 1) {
-        M2D_CHECK(f->mg_late == 0, M2D_ERR_NO_MEMORY, "Fields solve: the multigrid set-up failed before");
-        f->mg_late = -1;
-        M2D_TRY(mg_setup(f));
-        f->mg_late = 1;
+    if (f->mg.lv.empty()) {
+        const int r = mg_setup(f);
+        if (r != M2D_OK) {
+            mg_free_levels(f->mg);
+            return r;
+        }
     }
     return solve(f, mode, tol, info, false);
 }
@@ -1468,6 +1478,14 @@ extern "C" {
 
 int m2d_fields2d_create(m2d_ctx *ctx, const m2d_fields2d_params *p, const uint8_t *mask,
                         const double *voltage, m2d_fields2d **out)
+{
+    return fields_create(ctx, p, mask, voltage, true, out);
+}
+
+}  // extern "C"
+
+int m2d::fields_create(m2d_ctx *ctx, const m2d_fields2d_params *p, const uint8_t *mask, const double *voltage,
+                       bool direct, m2d_fields2d **out)
 {
     M2D_CHECK(ctx && p && mask && voltage && out, M2D_ERR_BAD_ARG, "m2d_fields2d_create: NULL argument");
     *out = nullptr;
@@ -1541,7 +1559,7 @@ int m2d_fields2d_create(m2d_ctx *ctx, const m2d_fields2d_params *p, const uint8_
         (r = fill_bytes(ctx, f->rho, 0, 8 * n)))
         return fail(r);
     // a rectangle of free nodes is solved directly, anything else by multigrid-PCG
-    f->direct.on = direct2d_fits(f->h_mask, f->nx, f->nz, f->direct);
+    f->direct.on = direct && direct2d_fits(f->h_mask, f->nx, f->nz, f->direct);
     if ((r = solve_setup(f)) || (r = f->direct.on ? direct2d_setup(f) : mg_setup(f))) return fail(r);
     if ((r = fields_build_tables(f))) return fail(r);
     if (hipStreamSynchronize(ctx->stream) != hipSuccess)
@@ -1549,6 +1567,8 @@ int m2d_fields2d_create(m2d_ctx *ctx, const m2d_fields2d_params *p, const uint8_
     *out = f;
     return M2D_OK;
 }
+
+extern "C" {
 
 int m2d_fields2d_destroy(m2d_fields2d *f)
 {

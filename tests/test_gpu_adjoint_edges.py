@@ -1,6 +1,7 @@
 """The adjoint of the gather in the outer half cells of the grid, where its
 two edges are clamped onto one: the gradient of a run that starts there
-against central differences of the FP64 oracle."""
+against central differences of the FP64 oracle.  And a field that is
+solved, differentiated and solved again."""
 import numpy as np
 import pytest
 
@@ -44,3 +45,70 @@ def test_gradient_of_a_run_along_an_edge(ctx, axis, low):
     assert scale > 0
     # the bound of the run in the middle of the trap
     assert np.abs(grad - fd).max() <= 1e-4 * scale, (grad, fd)
+
+
+def small_run(ctx, n=32, L=2e-2, electrode=False):
+    g, mask, volt, group, dx = trap(n, L)
+    volt = volt + np.where(group >= 0, np.random.default_rng(1).uniform(-5, 5, 8)[np.maximum(group, 0)], 0.0)
+    if electrode:
+        mask.reshape(n, n)[3:5, 3:5] = abi.FIXED
+    dV = 400 / 1e12 / (n - 1) ** 2
+    params = abi.FieldsParams(g, L, L, 1, 1, 0, abi.BC_FREE, 0.0, 0, 0.0, 0.0, 0.0, 0.0, 0.1, 0.0, dV)
+    return abi.Fields2D(ctx, params, mask, volt), group
+
+
+def gradient(ctx, fields, group, cols):
+    P = abi.ParticlesSoA.from_host(ctx, *cols)
+    fields.upload(abi.FIELD_U, np.zeros(group.size))
+    J, grad, info = abi.adjoint_energy(ctx, fields, abi.Species2D(-QE, M_E, 1e-11, float("inf"), 0, 0, 0), P, 8,
+                                       group=group, n_groups=8, checkpoint_every=3)
+    return J, grad, info.n_live, {k: a[P.alive()] for k, a in P.download().items()}
+
+
+@pytest.mark.parametrize("electrode", [False, True])
+def test_solves_around_a_gradient_are_the_same(ctx, electrode):
+    """A field keeps what its gradients set up and queue apart from its own
+    solves: the same charge gives the same bits and counts before and after."""
+    fields, group = small_run(ctx, electrode=electrode)
+    rng = np.random.default_rng(5)
+    rho = rng.normal(size=group.size) * 1e-18
+    x, z, v = electrons(400, 2e-2, rng)
+
+    def solve(tol):
+        fields.upload(abi.FIELD_U, np.zeros(group.size))
+        fields.upload(abi.FIELD_RHO, rho)
+        info = fields.solve(abi.SOLVE_STATIC, tol)
+        return info.outer_iters, info.inner_iters, info.rel_residual, fields.download(abi.FIELD_U).tobytes()
+
+    first = solve(1e-10)
+    a = gradient(ctx, fields, group, [x, z, *v])
+    assert solve(1e-10) == first
+    tight = solve(1e-13)
+    assert solve(1e-10) == first and solve(1e-13) == tight
+    b = gradient(ctx, fields, group, [x, z, *v])
+    assert abs(a[0] - b[0]) <= 1e-12 * a[0] and np.abs(a[1] - b[1]).max() <= 1e-8 * np.abs(a[1]).max()
+
+
+def test_a_refused_hierarchy_is_refused_alike_each_time(ctx):
+    """A 4 x 850 box is solved directly, but its gradient's multigrid has no
+    coarse level small enough: a bad argument, in the first call and in later
+    ones, which leaves the field's own solves as they were."""
+    nx, nz, h = 4, 850, 1e-4
+    mask = np.full((nx, nz), abi.FIXED, np.uint8)
+    mask[1:-1, 1:-1] = abi.FREE
+    g = abi.grid2d(nx, nz, h, h)
+    prm = abi.FieldsParams(g, h * (nx - 1), h * (nz - 1), 1, 1, 0, abi.BC_FREE, 0.0, 0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0,
+                           1e-12)
+    fields = abi.Fields2D(ctx, prm, mask.ravel(), np.zeros(nx * nz))
+    rho = np.where(mask.ravel() == abi.FREE, np.random.default_rng(1).normal(size=nx * nz) * 1e-18, 0.0)
+    P = abi.ParticlesSoA.from_host(ctx, *(np.full(4, c, np.float32) for c in (1.5e-4, 4e-2, 0.0, 0.0, 0.0)))
+    us = []
+    for _ in range(3):
+        fields.upload(abi.FIELD_U, np.zeros(nx * nz))
+        fields.upload(abi.FIELD_RHO, rho)
+        assert fields.solve(abi.SOLVE_STATIC, 1e-10).rel_residual <= 1e-10
+        us.append(fields.download(abi.FIELD_U).tobytes())
+        with pytest.raises(abi.M2DError) as e:
+            abi.adjoint_energy(ctx, fields, abi.Species2D(-QE, M_E, 1e-11, float("inf"), 0, 0, 0), P, 2)
+        assert abi.STATUS[e.value.code] == "BAD_ARG", e.value
+    assert us[0] == us[1] == us[2]
