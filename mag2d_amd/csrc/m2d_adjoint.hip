@@ -479,7 +479,9 @@ int m2d_adjoint_energy_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s,
     // per replayed step: x, z, and with MCC the velocities vx, vy, vz
     const int SC = mcc ? 5 : 2;
     M2D_TRY(seg.alloc(sizeof(float) * SC * np * (size_t)(K + 1)));
-    M2D_TRY(rep.alloc(sizeof(float) * 5 * np));
+    // the replayed store: m2d_advance_2d takes arrays of 16-byte alignment
+    const size_t pitch = (np + 3) / 4 * 4;
+    M2D_TRY(rep.alloc(sizeof(float) * 5 * pitch));
     const unsigned gb = nblk(nc);
     M2D_TRY(gpart.alloc(sizeof(double) * (size_t)gb * cfg->n_groups));
     M2D_TRY(dgrad.alloc(sizeof(double) * cfg->n_groups));
@@ -532,8 +534,8 @@ int m2d_adjoint_energy_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s,
         a.stream = s->stream;
     }
     const double rscale = -(f->p.grid.dx * f->p.grid.dx) / kEps0 / f->p.dV;  // b_F = rscale * rho
-    float *const rarr[5] = {rep.as<float>(), rep.as<float>() + np, rep.as<float>() + 2 * np,
-                            rep.as<float>() + 3 * np, rep.as<float>() + 4 * np};
+    float *rarr[5];
+    for (int c = 0; c < 5; c++) rarr[c] = rep.as<float>() + c * pitch;
     const m2d_particles2d rp{rarr[0], rarr[1], rarr[2], rarr[3], rarr[4], p->n};
     float *segx = seg.as<float>();
     for (int s0 = ((N - 1) / K) * K; s0 >= 0; s0 -= K) {

@@ -1,7 +1,7 @@
 """The adjoint of the gather in the outer half cells of the grid, where its
 two edges are clamped onto one: the gradient of a run that starts there
-against central differences of the FP64 oracle.  And a field that is
-solved, differentiated and solved again."""
+against central differences of the FP64 oracle.  Stores of any slot count, and
+a field that is solved, differentiated and solved again."""
 import numpy as np
 import pytest
 
@@ -63,6 +63,25 @@ def gradient(ctx, fields, group, cols):
     J, grad, info = abi.adjoint_energy(ctx, fields, abi.Species2D(-QE, M_E, 1e-11, float("inf"), 0, 0, 0), P, 8,
                                        group=group, n_groups=8, checkpoint_every=3)
     return J, grad, info.n_live, {k: a[P.alive()] for k, a in P.download().items()}
+
+
+@pytest.mark.parametrize("count", [1, 401, 402, 403])
+def test_slot_counts_of_any_remainder(ctx, count):
+    """Against the same store with empty slots up to a multiple of four.  The
+    gradient's atomic sums have no order; 1e-8 of it holds what that and the
+    solves' 1e-10 leave."""
+    fields, group = small_run(ctx)
+    x, z, v = electrons(count, 2e-2, np.random.default_rng(count))
+    cols = [x, z, *v]
+    J, grad, live, out = gradient(ctx, fields, group, cols)
+    dead = np.array([abi.DEAD_BITS], np.uint32).view(np.float32)
+    pad = -count % 4
+    want = gradient(ctx, fields, group, [np.concatenate([c, np.repeat(dead, pad)]) for c in cols])
+    assert live == want[2] and abs(J - want[0]) <= 1e-12 * want[0]
+    for k in out:
+        assert np.array_equal(out[k], want[3][k]), k
+    scale = np.abs(want[1]).max()
+    assert scale > 0 and np.abs(grad - want[1]).max() <= 1e-8 * scale
 
 
 @pytest.mark.parametrize("electrode", [False, True])
