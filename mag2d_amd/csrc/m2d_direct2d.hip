@@ -65,6 +65,7 @@ struct DstStage {
     int ldC;
     const double *lrow, *lcol;  // stage 2
     int rvalid;            // stage 4: rows inside the rectangle
+    const int *ahead;      // a pass that may well be needless: its stop flag, waited for before any operand is read
     SolveCtl *ctl;
 };
 
@@ -74,6 +75,7 @@ __global__ void __launch_bounds__(kDstThreads) k_dst_stage(DstStage a)
     constexpr int T = 16 * NT;
     __shared__ double part[4][T][T + 1];
     const int stop = a.ctl->stop_outer;
+    if (stopped(a.ahead)) return;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 15, kk = lane >> 4;
     const int row0 = blockIdx.y * T, col0 = blockIdx.x * T;
     const int len = a.K / 4, k0 = wave * len;
@@ -98,7 +100,7 @@ __global__ void __launch_bounds__(kDstThreads) k_dst_stage(DstStage a)
 #pragma unroll
             for (int t = 0; t < NT; t++) acc[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[s], B[t], acc[s][t], 0, 0, 0);
     }
-    if (stop) return;  // uniform; read beside the operands, not before them
+    if (stop) return;  // uniform; a first pass reads it beside its operands, not before them
     // accumulator r of lane l: row l / 16 + 4 r, column l % 16 of its 16 x 16 tile
 #pragma unroll
     for (int s = 0; s < NT; s++)
@@ -137,14 +139,18 @@ static void launch_stage(const DstStage &a, int rows, int cols, hipStream_t s)
 }
 
 // u -= A'^-1 r on the rectangle (r: FP64 residual on the grid), unless the
-// solve has stopped; counts one pass of one iteration
-int direct2d_pass(m2d_fields2d *f, double *u, SolveCtl *ctl)
+// solve has stopped; counts one pass of one iteration.  surplus: the pass is
+// one of several queued together, which the first may have made needless: its
+// products then wait for the stop flag before they read their operands (at
+// 1024^2 a needless pass took 226 us, now 8)
+int direct2d_pass(m2d_fields2d *f, double *u, SolveCtl *ctl, bool surplus)
 {
     const Direct2 &d = f->direct;
     hipStream_t s = f->ctx->stream;
     const size_t corner = (size_t)d.i0 * f->nz + d.j0;
     DstStage a{};
     a.ctl = ctl;
+    a.ahead = surplus ? &ctl->stop_outer : nullptr;
     a.S = d.sm; a.ldS = d.M; a.B = f->mg.r64 + corner; a.ldB = f->nz;
     a.K = d.M; a.kvalid = d.m; a.cvalid = d.n; a.C = d.t0; a.ldC = d.M;
     launch_stage<1>(a, d.M, d.N, s);

@@ -1405,16 +1405,17 @@ static void queue_first_residual(m2d_fields2d *f, double *u, int mode, double sc
 
 // FP64 refinement whose every pass is the direct solve of its residual: one
 // pass meets any tolerance FP64 can hold on most grids, and as many as the
-// last solve took are queued before the host reads the control block
+// last direct solve took are queued before the host reads the control block
+// (the field's multigrid solves keep their own estimate)
 static int refine_direct(m2d_fields2d *f, double *u, double tol)
 {
     Mg &mg = f->mg;
     hipStream_t s = f->ctx->stream;
     SolveCtl *ctl = solve_ctl(mg), *h = (SolveCtl *)(mg.h_dots + 16);
-    int J = mg.est.passes < 1 ? 1 : (mg.est.passes > kMaxOuter ? kMaxOuter : mg.est.passes);
+    int J = f->direct.passes;
     for (int round = 0; round <= kMaxOuter; round++, J = 1) {
         for (int j = 0; j < J; j++) {
-            M2D_TRY(direct2d_pass(f, u, ctl));
+            M2D_TRY(direct2d_pass(f, u, ctl, j > 0));
             queue_residual(f, u, tol, kMaxOuter);
         }
         M2D_HIP(hipGetLastError());
@@ -1422,7 +1423,7 @@ static int refine_direct(m2d_fields2d *f, double *u, double tol)
         M2D_HIP(hipStreamSynchronize(s));
         if (h->nan || h->stop_outer) break;
     }
-    mg.est.passes = h->outer > 1 ? h->outer : 1;
+    f->direct.passes = std::min(std::max(h->outer, 1), kMaxOuter);
     return M2D_OK;
 }
 

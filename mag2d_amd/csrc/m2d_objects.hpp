@@ -80,6 +80,7 @@ constexpr int kDstPad = 32;
 struct Direct2 {
     bool on = false;
     int i0 = 0, j0 = 0, m = 0, n = 0, M = 0, N = 0;
+    int passes = 1;               // the last direct solve's passes: what the next queues
     double *buf = nullptr;        // one allocation behind the pointers below
     double *sm = nullptr, *sn = nullptr, *lm = nullptr, *ln = nullptr, *t0 = nullptr, *t1 = nullptr;
 };
@@ -136,7 +137,7 @@ int fields_create(m2d_ctx *ctx, const m2d_fields2d_params *p, const uint8_t *mas
 int fields_solve_multigrid(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info);
 bool direct2d_fits(const std::vector<uint8_t> &mask, int nx, int nz, Direct2 &d);
 int direct2d_setup(m2d_fields2d *f);
-int direct2d_pass(m2d_fields2d *f, double *u, SolveCtl *ctl);
+int direct2d_pass(m2d_fields2d *f, double *u, SolveCtl *ctl, bool surplus);
 int mcc_sync(m2d_mcc *m);
 // some target draws its partners from the store whose first position array
 // is x (the colliding species itself)
