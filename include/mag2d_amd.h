@@ -97,6 +97,10 @@ int m2d_ctx_profile_read(m2d_ctx *ctx, double *ms, int64_t *launches);
 #define M2D_PASS_HIPOS  64u   /* long-time positions (FP32 pairs) */
 int m2d_ctx_last_pass(m2d_ctx *ctx, uint32_t *variant);
 
+/* Device memory.  A context keeps records of deposits (32 bytes a node, in 3D
+ * 64 bytes a node up to 1 GiB) and of sorts (32 bytes a slot, at most a quarter
+ * of the memory that was free) from one call to the next; a request of this or
+ * any other call that does not fit frees them before it is refused. */
 int m2d_malloc(m2d_ctx *ctx, size_t bytes, void **out);
 int m2d_free(m2d_ctx *ctx, void *p);
 int m2d_memcpy_h2d(m2d_ctx *ctx, void *dst, const void *src, size_t bytes);   /* synchronous */

@@ -1077,13 +1077,11 @@ struct Key3 {
 };
 
 // ------------------------------------------------------------------ host helpers
-static int dmalloc3(void **p, size_t bytes)
+static int dmalloc3(m2d_ctx *ctx, void **p, size_t bytes)
 {
-    hipError_t e = hipMalloc(p, bytes < 16 ? 16 : bytes);
-    if (e != hipSuccess) {
-        *p = nullptr;
+    hipError_t e = dev_malloc(ctx, p, bytes < 16 ? 16 : bytes);
+    if (e != hipSuccess)
         return set_error(M2D_ERR_NO_MEMORY, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
-    }
     return M2D_OK;
 }
 
@@ -1270,14 +1268,14 @@ static int mg3_setup(m2d_fields3d *f, const std::vector<uint8_t> &mask)
         const Host3 &H = lv[l];
         V.nx = H.n[0]; V.ny = H.n[1]; V.nz = H.n[2];
         V.n = H.size();
-        M2D_TRY(dmalloc3((void **)&V.nbm, V.n));
+        M2D_TRY(dmalloc3(f->ctx, (void **)&V.nbm, V.n));
         M2D_HIP(hipMemcpy(V.nbm, H.nbm.data(), V.n, hipMemcpyHostToDevice));
         if (l == 0) continue;
         di.resize(V.n);
         for (size_t m = 0; m < V.n; m++) di[m] = 1.f / H.diag(m);
-        M2D_TRY(dmalloc3((void **)&V.di, sizeof(float) * V.n));
-        M2D_TRY(dmalloc3((void **)&V.x, sizeof(float) * V.n));
-        M2D_TRY(dmalloc3((void **)&V.b, sizeof(float) * V.n));
+        M2D_TRY(dmalloc3(f->ctx, (void **)&V.di, sizeof(float) * V.n));
+        M2D_TRY(dmalloc3(f->ctx, (void **)&V.x, sizeof(float) * V.n));
+        M2D_TRY(dmalloc3(f->ctx, (void **)&V.b, sizeof(float) * V.n));
         M2D_HIP(hipMemcpy(V.di, di.data(), sizeof(float) * V.n, hipMemcpyHostToDevice));
         // the descent's tiles need not cover the last, pinned nodes
         M2D_HIP(hipMemset(V.b, 0, sizeof(float) * V.n));
@@ -1286,18 +1284,18 @@ static int mg3_setup(m2d_fields3d *f, const std::vector<uint8_t> &mask)
     if (f->coarse_dense) {
         std::vector<float> inv;
         M2D_CHECK(dense_inverse7(lv.back(), inv), M2D_ERR_BAD_ARG, "Fields3D: coarsest multigrid operator is singular");
-        M2D_TRY(dmalloc3((void **)&f->coarse_inv, sizeof(float) * inv.size()));
+        M2D_TRY(dmalloc3(f->ctx, (void **)&f->coarse_inv, sizeof(float) * inv.size()));
         M2D_HIP(hipMemcpy(f->coarse_inv, inv.data(), sizeof(float) * inv.size(), hipMemcpyHostToDevice));
     }
     const size_t n = f->n;
-    for (float **q : {&f->pr, &f->pz, &f->pp, &f->pp2, &f->pq, &f->pe}) M2D_TRY(dmalloc3((void **)q, sizeof(float) * n));
+    for (float **q : {&f->pr, &f->pz, &f->pp, &f->pp2, &f->pq, &f->pe}) M2D_TRY(dmalloc3(f->ctx, (void **)q, sizeof(float) * n));
     // 16 scalars, then the solve's control block
-    M2D_TRY(dmalloc3((void **)&f->dots, sizeof(double) * 32));
+    M2D_TRY(dmalloc3(f->ctx, (void **)&f->dots, sizeof(double) * 32));
     M2D_HIP(hipHostMalloc((void **)&f->h_dots, sizeof(double) * 32));
     // up to three sums per block of the fused reductions, one per tile of the ascent
     f->npartial = (int)std::max({red_blocks3(n), up_blocks3(f), 3 * Cols3{f->nx, f->ny, f->nz}.blocks()});
-    M2D_TRY(dmalloc3((void **)&f->partial, sizeof(double) * f->npartial));
-    M2D_TRY(dmalloc3((void **)&f->ticket, sizeof(unsigned int) * kTicketWords));
+    M2D_TRY(dmalloc3(f->ctx, (void **)&f->partial, sizeof(double) * f->npartial));
+    M2D_TRY(dmalloc3(f->ctx, (void **)&f->ticket, sizeof(unsigned int) * kTicketWords));
     M2D_HIP(hipMemset(f->ticket, 0, sizeof(unsigned int) * kTicketWords));
     return M2D_OK;
 }
@@ -1582,10 +1580,10 @@ int m2d_fields3d_create(m2d_ctx *ctx, const m2d_fields3d_params *p, const uint8_
     f->idx = 1.0 / g.dx; f->idy = 1.0 / g.dy; f->idz = 1.0 / g.dz;
     int r = M2D_OK;
     auto fail = [&](int code) { m2d_fields3d_destroy(f); return code; };
-    if ((r = dmalloc3((void **)&f->mask, n)) || (r = dmalloc3((void **)&f->cellfree, n)) ||
-        (r = dmalloc3((void **)&f->voltage, 8 * n)) || (r = dmalloc3((void **)&f->u, 8 * n)) ||
-        (r = dmalloc3((void **)&f->rho, 8 * n)) || (r = dmalloc3((void **)&f->tx, 4 * n)) ||
-        (r = dmalloc3((void **)&f->ty, 4 * n)) || (r = dmalloc3((void **)&f->tz, 4 * n)))
+    if ((r = dmalloc3(f->ctx, (void **)&f->mask, n)) || (r = dmalloc3(f->ctx, (void **)&f->cellfree, n)) ||
+        (r = dmalloc3(f->ctx, (void **)&f->voltage, 8 * n)) || (r = dmalloc3(f->ctx, (void **)&f->u, 8 * n)) ||
+        (r = dmalloc3(f->ctx, (void **)&f->rho, 8 * n)) || (r = dmalloc3(f->ctx, (void **)&f->tx, 4 * n)) ||
+        (r = dmalloc3(f->ctx, (void **)&f->ty, 4 * n)) || (r = dmalloc3(f->ctx, (void **)&f->tz, 4 * n)))
         return fail(r);
     std::vector<uint8_t> hm(mask, mask + n), cf(n, 0);
     for (int i = 0; i + 1 < g.nx; i++)

@@ -367,13 +367,11 @@ struct DBuf {
             (void)hipFree(p);
         }
     }
-    int alloc(size_t bytes)
+    int alloc(m2d_ctx *ctx, size_t bytes)
     {
-        hipError_t e = hipMalloc(&p, bytes < 16 ? 16 : bytes);
-        if (e != hipSuccess) {
-            p = nullptr;
+        hipError_t e = dev_malloc(ctx, &p, bytes < 16 ? 16 : bytes);
+        if (e != hipSuccess)
             return set_error(M2D_ERR_NO_MEMORY, "adjoint: hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
-        }
         return M2D_OK;
     }
     template <typename T> T *as() const { return (T *)p; }
@@ -435,8 +433,8 @@ int m2d_adjoint_energy_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s,
     DBuf U, ckpt;
     const int nck = (N + K - 1) / K;
     if (grad) {
-        M2D_TRY(U.alloc(sizeof(double) * nc * (size_t)N));
-        M2D_TRY(ckpt.alloc(sizeof(float) * 5 * np * (size_t)nck));
+        M2D_TRY(U.alloc(ctx, sizeof(double) * nc * (size_t)N));
+        M2D_TRY(ckpt.alloc(ctx, sizeof(float) * 5 * np * (size_t)nck));
     }
     float *const parr[5] = {p->x, p->z, p->vx, p->vy, p->vz};
     M2D_TRY(m2d_fields2d_reset(f));
@@ -473,19 +471,19 @@ int m2d_adjoint_energy_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s,
 
     // ---- reverse sweep
     DBuf lam, lu, lrho, seg, rep, gpart, dgrad, dgroup;
-    M2D_TRY(lam.alloc(sizeof(double) * 5 * np));
-    M2D_TRY(lu.alloc(sizeof(double) * nc));
-    M2D_TRY(lrho.alloc(sizeof(double) * nc));
+    M2D_TRY(lam.alloc(ctx, sizeof(double) * 5 * np));
+    M2D_TRY(lu.alloc(ctx, sizeof(double) * nc));
+    M2D_TRY(lrho.alloc(ctx, sizeof(double) * nc));
     // per replayed step: x, z, and with MCC the velocities vx, vy, vz
     const int SC = mcc ? 5 : 2;
-    M2D_TRY(seg.alloc(sizeof(float) * SC * np * (size_t)(K + 1)));
+    M2D_TRY(seg.alloc(ctx, sizeof(float) * SC * np * (size_t)(K + 1)));
     // the replayed store: m2d_advance_2d takes arrays of 16-byte alignment
     const size_t pitch = (np + 3) / 4 * 4;
-    M2D_TRY(rep.alloc(sizeof(float) * 5 * pitch));
+    M2D_TRY(rep.alloc(ctx, sizeof(float) * 5 * pitch));
     const unsigned gb = nblk(nc);
-    M2D_TRY(gpart.alloc(sizeof(double) * (size_t)gb * cfg->n_groups));
-    M2D_TRY(dgrad.alloc(sizeof(double) * cfg->n_groups));
-    M2D_TRY(dgroup.alloc(sizeof(int) * nc));
+    M2D_TRY(gpart.alloc(ctx, sizeof(double) * (size_t)gb * cfg->n_groups));
+    M2D_TRY(dgrad.alloc(ctx, sizeof(double) * cfg->n_groups));
+    M2D_TRY(dgroup.alloc(ctx, sizeof(int) * nc));
     M2D_HIP(hipMemcpy(dgroup.p, cfg->group, sizeof(int) * nc, hipMemcpyHostToDevice));
     M2D_TRY(fill_bytes(ctx, dgrad.p, 0, sizeof(double) * cfg->n_groups));
     M2D_TRY(fill_bytes(ctx, lrho.p, 0, sizeof(double) * nc));

@@ -419,7 +419,7 @@ static int ensure_cos(m2d_batch *b, uint64_t niter0, int steps)
         if (b->cosv) (void)hipFree(b->cosv);
         b->cosv = nullptr;
         b->cosv_n = 0;
-        M2D_HIP(hipMalloc((void **)&b->cosv, sizeof(double) * (size_t)steps));
+        M2D_HIP(dev_malloc(b->ctx, (void **)&b->cosv, sizeof(double) * (size_t)steps));
         b->cosv_n = (size_t)steps;
     }
     std::vector<double> c((size_t)steps);
@@ -540,10 +540,10 @@ int m2d_batch_create(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s, cons
         R.pad = 0;
     }
     auto fail = [&](int code) { m2d_batch_destroy(b); return code; };
-    if (hipMalloc((void **)&b->d_runs, sizeof(BatchRun) * runs.size()) != hipSuccess ||
-        hipMalloc((void **)&b->d_off, sizeof(int64_t) * off.size()) != hipSuccess ||
-        hipMalloc((void **)&b->esum, sizeof(double) * (size_t)d->n_runs) != hipSuccess ||
-        hipMalloc((void **)&b->ecount, sizeof(unsigned long long) * (size_t)d->n_runs) != hipSuccess)
+    if (dev_malloc(ctx, (void **)&b->d_runs, sizeof(BatchRun) * runs.size()) != hipSuccess ||
+        dev_malloc(ctx, (void **)&b->d_off, sizeof(int64_t) * off.size()) != hipSuccess ||
+        dev_malloc(ctx, (void **)&b->esum, sizeof(double) * (size_t)d->n_runs) != hipSuccess ||
+        dev_malloc(ctx, (void **)&b->ecount, sizeof(unsigned long long) * (size_t)d->n_runs) != hipSuccess)
         return fail(set_error(M2D_ERR_NO_MEMORY, "m2d_batch_create: device allocation"));
     if (hipMemcpy(b->d_runs, runs.data(), sizeof(BatchRun) * runs.size(), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(b->d_off, off.data(), sizeof(int64_t) * off.size(), hipMemcpyHostToDevice) != hipSuccess)

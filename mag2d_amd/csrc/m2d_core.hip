@@ -21,7 +21,33 @@ int set_error(int code, const char *fmt, ...)
     return code;
 }
 
-int ensure(m2d_ctx *ctx, Scratch &s, size_t bytes)
+bool capturing(m2d_ctx *ctx)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone) return false;
+    (void)hipGetLastError();
+    return true;
+}
+
+hipError_t dev_malloc(m2d_ctx *ctx, void **p, size_t bytes, bool optional)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && !optional && (ctx->rec.ptr || ctx->pack.ptr) && !capturing(ctx)) {
+        (void)hipStreamSynchronize(ctx->stream);
+        for (Scratch *s : {&ctx->rec, &ctx->pack}) {
+            if (s->ptr) (void)hipFree(s->ptr);
+            *s = Scratch();
+        }
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+        *p = nullptr;
+        (void)hipGetLastError();  // reported by the caller, not by the next launch
+    }
+    return e;
+}
+
+int ensure(m2d_ctx *ctx, Scratch &s, size_t bytes, bool optional)
 {
     if (s.bytes >= bytes) return M2D_OK;
     if (s.ptr) {
@@ -31,11 +57,9 @@ int ensure(m2d_ctx *ctx, Scratch &s, size_t bytes)
         s.bytes = 0;
     }
     size_t want = bytes < 4096 ? 4096 : bytes;
-    hipError_t e = hipMalloc(&s.ptr, want);
-    if (e != hipSuccess) {
-        s.ptr = nullptr;
+    hipError_t e = dev_malloc(ctx, &s.ptr, want, optional);
+    if (e != hipSuccess)
         return set_error(M2D_ERR_NO_MEMORY, "hipMalloc(%zu): %s", want, hipGetErrorString(e));
-    }
     s.bytes = want;
     return M2D_OK;
 }
@@ -224,7 +248,7 @@ void ctx_release(m2d_ctx *c)
     if (--c->refs > 0) return;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
-    for (Scratch *s : {&c->acc, &c->rec, &c->red, &c->tmp, &c->sortbuf, &c->cq})
+    for (Scratch *s : {&c->acc, &c->rec, &c->red, &c->tmp, &c->sortbuf, &c->pack, &c->cq})
         if (s->ptr) (void)hipFree(s->ptr);
     free_tilings(c);
     for (auto &pr : c->ev_pending) c->ev_pool.insert(c->ev_pool.end(), {pr.first, pr.second});
@@ -274,11 +298,9 @@ int m2d_malloc(m2d_ctx *c, size_t bytes, void **out)
     M2D_CHECK(c && out, M2D_ERR_BAD_ARG, "m2d_malloc: NULL argument");
     *out = nullptr;
     if (bytes == 0) bytes = 1;
-    hipError_t e = hipMalloc(out, bytes);
-    if (e != hipSuccess) {
-        *out = nullptr;
+    hipError_t e = dev_malloc(c, out, bytes);
+    if (e != hipSuccess)
         return set_error(M2D_ERR_NO_MEMORY, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
-    }
     return M2D_OK;
 }
 

@@ -202,11 +202,9 @@ int direct2d_setup(m2d_fields2d *f)
     Direct2 &d = f->direct;
     const size_t M = d.M, N = d.N;
     const size_t words = M * M + M + N * N + N + 2 * M * N;
-    hipError_t e = hipMalloc((void **)&d.buf, words * sizeof(double));
-    if (e != hipSuccess) {
-        d.buf = nullptr;
+    hipError_t e = dev_malloc(f->ctx, (void **)&d.buf, words * sizeof(double));
+    if (e != hipSuccess)
         return set_error(M2D_ERR_NO_MEMORY, "Fields: hipMalloc(%zu): %s", words * sizeof(double), hipGetErrorString(e));
-    }
     d.sm = d.buf;
     d.sn = d.sm + M * M;
     d.t0 = d.sn + N * N;

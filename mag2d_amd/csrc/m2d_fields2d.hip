@@ -1039,13 +1039,11 @@ static bool dense_inverse(const std::vector<double> &A9, const std::vector<uint8
     return true;
 }
 
-static int dmalloc(void **p, size_t bytes)
+static int dmalloc(m2d_ctx *ctx, void **p, size_t bytes)
 {
-    hipError_t e = hipMalloc(p, bytes < 16 ? 16 : bytes);
-    if (e != hipSuccess) {
-        *p = nullptr;
+    hipError_t e = dev_malloc(ctx, p, bytes < 16 ? 16 : bytes);
+    if (e != hipSuccess)
         return set_error(M2D_ERR_NO_MEMORY, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
-    }
     return M2D_OK;
 }
 
@@ -1054,16 +1052,16 @@ static int solve_setup(m2d_fields2d *f)
 {
     Mg &mg = f->mg;
     const size_t n = f->n;
-    M2D_TRY(dmalloc((void **)&mg.pr, sizeof(float) * n));
-    M2D_TRY(dmalloc((void **)&mg.r64, sizeof(double) * n));
+    M2D_TRY(dmalloc(f->ctx, (void **)&mg.pr, sizeof(float) * n));
+    M2D_TRY(dmalloc(f->ctx, (void **)&mg.r64, sizeof(double) * n));
     // 16 device scalars, then the solve's control block (SolveCtl)
-    M2D_TRY(dmalloc((void **)&mg.dots, sizeof(double) * 32));
-    M2D_TRY(dmalloc((void **)&mg.ticket, sizeof(unsigned int) * kTicketWords));
+    M2D_TRY(dmalloc(f->ctx, (void **)&mg.dots, sizeof(double) * 32));
+    M2D_TRY(dmalloc(f->ctx, (void **)&mg.ticket, sizeof(unsigned int) * kTicketWords));
     M2D_HIP(hipMemset(mg.ticket, 0, sizeof(unsigned int) * kTicketWords));
     M2D_HIP(hipHostMalloc((void **)&mg.h_dots, sizeof(double) * 32));
     mg.npartial = (int)std::min<size_t>((n + 255) / 256, 65536);
     // up to three sums per block of the fused reductions
-    M2D_TRY(dmalloc((void **)&mg.partial, sizeof(double) * 3 * std::max<size_t>(mg.npartial, (n + 255) / 256)));
+    M2D_TRY(dmalloc(f->ctx, (void **)&mg.partial, sizeof(double) * 3 * std::max<size_t>(mg.npartial, (n + 255) / 256)));
     return M2D_OK;
 }
 
@@ -1115,13 +1113,13 @@ static int mg_setup(m2d_fields2d *f)
             double d = ops[l][9 * k + 4];
             dinv[k] = dirs[l][k] || !(d > 0) ? 0.f : (float)(1.0 / d);
         }
-        M2D_TRY(dmalloc((void **)&L.st, sizeof(float) * 9 * L.n));
-        M2D_TRY(dmalloc((void **)&L.dinv, sizeof(float) * L.n));
-        M2D_TRY(dmalloc((void **)&L.dir, L.n));
-        M2D_TRY(dmalloc((void **)&L.x, sizeof(float) * L.n));
-        M2D_TRY(dmalloc((void **)&L.x2, sizeof(float) * L.n));
-        M2D_TRY(dmalloc((void **)&L.r, sizeof(float) * L.n));
-        M2D_TRY(dmalloc((void **)&L.b, sizeof(float) * L.n));
+        M2D_TRY(dmalloc(f->ctx, (void **)&L.st, sizeof(float) * 9 * L.n));
+        M2D_TRY(dmalloc(f->ctx, (void **)&L.dinv, sizeof(float) * L.n));
+        M2D_TRY(dmalloc(f->ctx, (void **)&L.dir, L.n));
+        M2D_TRY(dmalloc(f->ctx, (void **)&L.x, sizeof(float) * L.n));
+        M2D_TRY(dmalloc(f->ctx, (void **)&L.x2, sizeof(float) * L.n));
+        M2D_TRY(dmalloc(f->ctx, (void **)&L.r, sizeof(float) * L.n));
+        M2D_TRY(dmalloc(f->ctx, (void **)&L.b, sizeof(float) * L.n));
         M2D_HIP(hipMemcpy(L.st, st.data(), sizeof(float) * 9 * L.n, hipMemcpyHostToDevice));
         M2D_HIP(hipMemcpy(L.dinv, dinv.data(), sizeof(float) * L.n, hipMemcpyHostToDevice));
         M2D_HIP(hipMemcpy(L.dir, dirs[l].data(), L.n, hipMemcpyHostToDevice));
@@ -1130,22 +1128,22 @@ static int mg_setup(m2d_fields2d *f)
     const MgLevel &C = mg.lv.back();
     M2D_CHECK(dense_inverse(ops.back(), dirs.back(), C.nx, C.nz, inv), M2D_ERR_BAD_ARG,
               "Fields: coarsest multigrid operator is singular");
-    M2D_TRY(dmalloc((void **)&mg.coarse_inv, sizeof(float) * inv.size()));
+    M2D_TRY(dmalloc(f->ctx, (void **)&mg.coarse_inv, sizeof(float) * inv.size()));
     M2D_HIP(hipMemcpy(mg.coarse_inv, inv.data(), sizeof(float) * inv.size(), hipMemcpyHostToDevice));
     {
         const size_t cn = C.n;
         std::vector<float> invT(cn * cn);
         for (size_t r = 0; r < cn; r++)
             for (size_t c = 0; c < cn; c++) invT[c * cn + r] = inv[r * cn + c];
-        M2D_TRY(dmalloc((void **)&mg.coarse_invT, sizeof(float) * invT.size()));
+        M2D_TRY(dmalloc(f->ctx, (void **)&mg.coarse_invT, sizeof(float) * invT.size()));
         M2D_HIP(hipMemcpy(mg.coarse_invT, invT.data(), sizeof(float) * invT.size(), hipMemcpyHostToDevice));
     }
     const size_t n = f->n;
-    M2D_TRY(dmalloc((void **)&mg.pz, sizeof(float) * n));
-    M2D_TRY(dmalloc((void **)&mg.pp, sizeof(float) * n));
-    M2D_TRY(dmalloc((void **)&mg.pp2, sizeof(float) * n));
-    M2D_TRY(dmalloc((void **)&mg.pq, sizeof(float) * n));
-    M2D_TRY(dmalloc((void **)&mg.pe, sizeof(float) * n));
+    M2D_TRY(dmalloc(f->ctx, (void **)&mg.pz, sizeof(float) * n));
+    M2D_TRY(dmalloc(f->ctx, (void **)&mg.pp, sizeof(float) * n));
+    M2D_TRY(dmalloc(f->ctx, (void **)&mg.pp2, sizeof(float) * n));
+    M2D_TRY(dmalloc(f->ctx, (void **)&mg.pq, sizeof(float) * n));
+    M2D_TRY(dmalloc(f->ctx, (void **)&mg.pe, sizeof(float) * n));
     // the coarse part of the V-cycle runs in one workgroup from the first
     // level of at most kBlockLevelNodes nodes (the dense level at the latest)
     mg.lc = (int)mg.lv.size() - 1;
@@ -1523,18 +1521,18 @@ int m2d::fields_create(m2d_ctx *ctx, const m2d_fields2d_params *p, const uint8_t
     f->h_mask.assign(mask, mask + n);
     int r = M2D_OK;
     auto fail = [&](int code) { m2d_fields2d_destroy(f); return code; };
-    if ((r = dmalloc((void **)&f->mask, n)) || (r = dmalloc((void **)&f->cellfree, n)) ||
-        (r = dmalloc((void **)&f->voltage, 8 * n)) || (r = dmalloc((void **)&f->u, 8 * n)) ||
-        (r = dmalloc((void **)&f->urf, 8 * n)) || (r = dmalloc((void **)&f->rho, 8 * n)) ||
-        (r = dmalloc((void **)&f->gx, sizeof(float2) * (size_t)(g.nx + 1) * g.nz)) ||
-        (r = dmalloc((void **)&f->gz, sizeof(float2) * (size_t)g.nx * (g.nz + 1))) ||
-        (r = dmalloc((void **)&f->phx, sizeof(float) * (size_t)(g.nx + 1) * g.nz)) ||
-        (r = dmalloc((void **)&f->phz, sizeof(float) * (size_t)g.nx * (g.nz + 1))))
+    if ((r = dmalloc(f->ctx, (void **)&f->mask, n)) || (r = dmalloc(f->ctx, (void **)&f->cellfree, n)) ||
+        (r = dmalloc(f->ctx, (void **)&f->voltage, 8 * n)) || (r = dmalloc(f->ctx, (void **)&f->u, 8 * n)) ||
+        (r = dmalloc(f->ctx, (void **)&f->urf, 8 * n)) || (r = dmalloc(f->ctx, (void **)&f->rho, 8 * n)) ||
+        (r = dmalloc(f->ctx, (void **)&f->gx, sizeof(float2) * (size_t)(g.nx + 1) * g.nz)) ||
+        (r = dmalloc(f->ctx, (void **)&f->gz, sizeof(float2) * (size_t)g.nx * (g.nz + 1))) ||
+        (r = dmalloc(f->ctx, (void **)&f->phx, sizeof(float) * (size_t)(g.nx + 1) * g.nz)) ||
+        (r = dmalloc(f->ctx, (void **)&f->phz, sizeof(float) * (size_t)g.nx * (g.nz + 1))))
         return fail(r);
     // sort tiles of 8 x 8 cells; the deposit window of tile (ti, tj) spans
     // cells [8 ti - 8, 8 ti + 16) x [8 tj - 8, 8 tj + 16)
     const int ntx = (g.nx - 2) / kTile + 1, ntz = (g.nz - 2) / kTile + 1;
-    if ((r = dmalloc((void **)&f->winfree, (size_t)ntx * ntz))) return fail(r);
+    if ((r = dmalloc(f->ctx, (void **)&f->winfree, (size_t)ntx * ntz))) return fail(r);
     std::vector<uint8_t> cf(n, 0);
     for (int i = 0; i + 1 < g.nx; i++)
         for (int j = 0; j + 1 < g.nz; j++) {
@@ -1605,7 +1603,7 @@ int m2d_fields2d_set_magnetic_field(m2d_fields2d *f, const m2d_grid2d *g, const 
                   "Fields::load_magnetic_field() garbage loaded");
         h[k] = make_float2((float)Br[k], (float)Bz[k]);
     }
-    M2D_TRY(dmalloc((void **)&f->bt, n * sizeof(float2)));
+    M2D_TRY(dmalloc(f->ctx, (void **)&f->bt, n * sizeof(float2)));
     M2D_HIP(hipMemcpy(f->bt, h.data(), n * sizeof(float2), hipMemcpyHostToDevice));
     f->bgrid = *g;
     return M2D_OK;
@@ -1705,7 +1703,7 @@ int m2d_fields2d_u_smooth(m2d_fields2d *f, int which, int symmetry, double radiu
         k_smooth_sym<<<dim3((unsigned)((h + 127) / 128), (unsigned)h), 128, 0, st>>>(u, lmax, ic, jc);
         M2D_HIP(hipGetLastError());
     }
-    if (!f->smooth_tmp) M2D_TRY(dmalloc((void **)&f->smooth_tmp, 8 * f->n));
+    if (!f->smooth_tmp) M2D_TRY(dmalloc(f->ctx, (void **)&f->smooth_tmp, 8 * f->n));
     M2D_HIP(hipMemcpyAsync(f->smooth_tmp, u, 8 * f->n, hipMemcpyDeviceToDevice, st));
     const double r2 = radius > 0 ? (radius / f->p.grid.dx) * (radius / f->p.grid.dx) : radius;
     if (jmax > 2 && lmax > 2) {

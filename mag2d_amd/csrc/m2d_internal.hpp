@@ -133,7 +133,8 @@ struct m2d_ctx {
     bool rec_dirty = false; // a call failed between writing records and clearing them
     m2d::Scratch red;       // reduction partials
     m2d::Scratch tmp;       // general temporaries (compaction offsets)
-    m2d::Scratch sortbuf;   // keys, slots, packed particles and radix-sort temporaries
+    m2d::Scratch sortbuf;   // keys, slots and radix-sort temporaries
+    m2d::Scratch pack;      // packed particles of scattered stores (see sort_records)
     m2d::Scratch cq;        // MCC collision queue (slot indices)
     uint64_t launch_seq = 0;  // selects the collision-queue counter of a launch
     bool cq_dirty = false;    // a call failed between appending to a queue counter and its scatter
@@ -173,7 +174,14 @@ inline void launch_timed(m2d_ctx *ctx, F kernel, dim3 grid, dim3 block, Args... 
 
 namespace m2d {
 
-int ensure(m2d_ctx *ctx, Scratch &s, size_t bytes);
+// the context's stream is being captured in a graph (or cannot say)
+bool capturing(m2d_ctx *ctx);
+// hipMalloc; where that fails, the context's optional buffers (the records of
+// deposits and sorts, which only make calls faster and which no captured graph
+// holds) are given back and it is tried once more.  optional: a request for
+// one of those, which takes nothing from the other.
+hipError_t dev_malloc(m2d_ctx *ctx, void **p, size_t bytes, bool optional = false);
+int ensure(m2d_ctx *ctx, Scratch &s, size_t bytes, bool optional = false);
 
 // vector kernels shared by the 2D and 3D solvers (m2d_fields2d.hip) and the
 // fixed-point flush (m2d_particles2d.hip)

@@ -136,8 +136,8 @@ int m2d_mcc_create(m2d_ctx *ctx, const m2d_mcc_desc *d, m2d_mcc **out)
         rate += D.rate;
     }
     h.lifetime = rate > 0.0 ? 1.0 / rate : INFINITY;
-    hipError_t e = hipMalloc((void **)&m->d, sizeof(McDev));
-    if (e == hipSuccess && !tab.empty()) e = hipMalloc((void **)&m->tab, sizeof(double) * tab.size());
+    hipError_t e = dev_malloc(ctx, (void **)&m->d, sizeof(McDev));
+    if (e == hipSuccess && !tab.empty()) e = dev_malloc(ctx, (void **)&m->tab, sizeof(double) * tab.size());
     if (e != hipSuccess) {
         m2d_mcc_destroy(m);
         return set_error(M2D_ERR_NO_MEMORY, "m2d_mcc_create: %s", hipGetErrorString(e));

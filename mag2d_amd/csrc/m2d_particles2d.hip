@@ -1208,18 +1208,15 @@ int deposit_buffer(m2d_ctx *ctx, size_t nodes, int corners, int &rec, unsigned l
     M2D_TRY(ensure_acc(ctx, nodes));
     acc = (unsigned long long *)ctx->acc.ptr;
     if (!rec) return M2D_OK;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
+    if (capturing(ctx)) {
         rec = 0;
         return M2D_OK;
     }
     const size_t need = nodes * corners * sizeof(unsigned long long);
     const bool grown = ctx->rec.bytes < need;
     if (grown) {
-        const int r = ensure(ctx, ctx->rec, need);
+        const int r = ensure(ctx, ctx->rec, need, true);
         if (r == M2D_ERR_NO_MEMORY) {  // the node grid does
-            (void)hipGetLastError();
             rec = 0;
             return M2D_OK;
         }

@@ -179,17 +179,8 @@ void free_tilings(m2d_ctx *ctx)
 int sort_scratch(m2d_ctx *ctx, size_t n, size_t radix_bytes, SortScratch &s)
 {
     auto up = [](size_t v) { return (v + 255) / 256 * 256; };
-    const size_t arr = up(n * 4), least = 4 * arr + up(radix_bytes) + 256, all = least + n * 32;
-    bool pack = ctx->sortbuf.bytes >= all;
-    if (!pack) {
-        size_t avail = 0, total = 0;
-        pack = hipMemGetInfo(&avail, &total) == hipSuccess && all <= avail / 4 &&
-               ensure(ctx, ctx->sortbuf, all) == M2D_OK;
-        if (!pack) {
-            (void)hipGetLastError();
-            M2D_TRY(ensure(ctx, ctx->sortbuf, least));
-        }
-    }
+    const size_t arr = up(n * 4);
+    M2D_TRY(ensure(ctx, ctx->sortbuf, 4 * arr + up(radix_bytes) + 256));
     uint8_t *b = (uint8_t *)ctx->sortbuf.ptr;
     s.k0 = (uint32_t *)b;
     s.k1 = (uint32_t *)(b + arr);
@@ -197,8 +188,22 @@ int sort_scratch(m2d_ctx *ctx, size_t n, size_t radix_bytes, SortScratch &s)
     s.v1 = (uint32_t *)(b + 3 * arr);
     s.scattered = (uint32_t *)(b + 4 * arr);
     s.radix = b + 4 * arr + 256;
-    s.rec = pack ? (float4 *)(b + least) : nullptr;
     return M2D_OK;
+}
+
+float4 *sort_records(m2d_ctx *ctx, size_t n)
+{
+    const size_t need = n * 2 * sizeof(float4);
+    if (capturing(ctx)) return nullptr;
+    if (ctx->pack.bytes < need) {
+        size_t avail = 0, total = 0;
+        if (hipMemGetInfo(&avail, &total) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (need > avail / 4 || ensure(ctx, ctx->pack, need, true) != M2D_OK) return nullptr;
+    }
+    return (float4 *)ctx->pack.ptr;
 }
 
 // the schedule record of the store at x (n slots, tiles ntx * nty * ntz, nty

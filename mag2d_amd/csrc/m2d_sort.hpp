@@ -130,14 +130,17 @@ inline int sort_key_bits(uint64_t tiles)
 inline uint32_t sort_dead_key(int bits) { return bits == 32 ? 0xFFFFFFFFu : (uint32_t)((1ull << bits) - 1); }
 
 // The sort's scratch: keys and slots, the sorted ones, the radix sort's
-// temporaries, the sample's answer and, where a quarter of the free memory
-// holds them, the records (rec: null without).  n > 0.
+// temporaries and the sample's answer.  n > 0.
 struct SortScratch {
     uint32_t *k0, *k1, *v0, *v1, *scattered;
     void *radix;
-    float4 *rec;
 };
 int sort_scratch(m2d_ctx *ctx, size_t n, size_t radix_bytes, SortScratch &s);
+// The records' memory, 32 bytes a slot, where a quarter of what is free holds
+// it; null otherwise, and in a call that is being captured in a graph (whose
+// replays would keep the address).  After the call's other allocations, which
+// may give it back (dev_malloc).
+float4 *sort_records(m2d_ctx *ctx, size_t n);
 // Queue the schedule of a tile-sorted store: tiling_begin before the gather,
 // which fills T->tile_start and T->tile_end (adjacent, zeroed before it) and
 // tiling_finish after it
@@ -167,15 +170,16 @@ int sort_store(m2d_ctx *ctx, const Key &key, const Columns<NC> &src, const Colum
     M2D_TRY(sort_scratch(ctx, n, temp, w));
     m2d_tiling *T;
     M2D_TRY(tiling_begin(ctx, dst.c[0], (int64_t)n, ntx, nty, ntz, cap, T));
+    float4 *const rec = sort_records(ctx, n);
     unsigned long long *live = ctx->counters + CNT_LIVE;
     const unsigned blocks = (unsigned)((n + 255) / 256);
     k_sort_sample<<<1, 1024, 0, ctx->stream>>>(key, (int64_t)n, dead_key, live, w.scattered);
-    k_sort_keys<<<blocks, 256, 0, ctx->stream>>>(key, src, (int64_t)n, w.k0, w.v0, w.rec, w.scattered, T->tile_start,
+    k_sort_keys<<<blocks, 256, 0, ctx->stream>>>(key, src, (int64_t)n, w.k0, w.v0, rec, w.scattered, T->tile_start,
                                                  2 * (int64_t)ntx * nty * ntz);
     M2D_HIP(hipGetLastError());
     e = rocprim::radix_sort_pairs<SortConfig>(w.radix, temp, w.k0, w.k1, w.v0, w.v1, n, lo, bits, ctx->stream);
     M2D_CHECK(e == hipSuccess, M2D_ERR_HIP, "radix_sort_pairs: %s", hipGetErrorString(e));
-    k_sort_gather<<<xcd_grid(blocks), 256, 0, ctx->stream>>>(src, dst, (int64_t)n, w.k1, w.v1, dead_key, live, w.rec,
+    k_sort_gather<<<xcd_grid(blocks), 256, 0, ctx->stream>>>(src, dst, (int64_t)n, w.k1, w.v1, dead_key, live, rec,
                                                              w.scattered, T->tile_start, T->tile_end);
     M2D_HIP(hipGetLastError());
     M2D_TRY(tiling_finish(ctx, T, dst.c[0], (int64_t)n, cap, round));

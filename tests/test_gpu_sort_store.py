@@ -1,5 +1,8 @@
 """The sort's two gathers (packed records of a scattered store, components of
-a nearly ordered one) and the schedule built from several blocks."""
+a nearly ordered one), the schedule built from several blocks, and the memory
+of the records."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -98,3 +101,44 @@ def test_schedule_covers_every_particle_once(ctx, n, r):
     assert np.array_equal(out[0][0], out[1][0])
     for k in abi.ParticlesSoA.NAMES:
         assert np.array_equal(out[0][1][k].view(np.uint32), out[1][1][k].view(np.uint32)), k
+
+
+def test_records_are_given_back_when_an_allocation_fails(ctx):
+    """The records of sorts and deposits only make calls faster: an allocation
+    that does not fit frees them before it is refused, and the next calls make
+    them again."""
+    hip = C.CDLL(abi.lib()._name)  # the HIP runtime that the library itself is linked to
+
+    def free():
+        ctx.sync()
+        a, b = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    sc = Scene(ctx, n=1100, solve_oracle=False, geometry=abi.GEO_EMPTY, rf=False)
+    rng = np.random.default_rng(5)
+    n = 2_000_000
+    pos = [rng.uniform(1e-4, sc.L * 0.999, n).astype(np.float32) for _ in range(2)]
+    src = abi.ParticlesSoA.from_host(ctx, *pos, *(rng.normal(size=n).astype(np.float32) for _ in range(3)))
+    dst = abi.ParticlesSoA(ctx, n)
+    rho = ctx.to_device(np.zeros(1100 * 1100))
+
+    def calls():
+        rho.zero()
+        abi.accumulate(ctx, sc.g, src, QE, rho.ptr)
+        abi.sort(ctx, sc.fields, src, dst)
+        return {**dst.download(), "rho": rho.get()}
+
+    want = calls()
+    held = 32 * n + 32 * 1100 * 1100
+    before = free()
+    with pytest.raises(abi.M2DError) as e:
+        ctx.malloc(1 << 46)
+    assert abi.STATUS[e.value.code] == "NO_MEMORY"
+    after = free()
+    assert after - before >= held
+    for _ in range(2):
+        got = calls()
+        for k in want:
+            assert np.array_equal(got[k], want[k]), k
+    assert after - free() >= held
