@@ -542,13 +542,15 @@ __global__ void __launch_bounds__(256) k3_dense(const float *inv, const float *b
     if (lane == 0 && !stopped_) x[row] = s;
 }
 
-// Half sweep of colour on a grid that has one level only and is too large
-// for a dense solve (a side below 5 nodes): its preconditioner is symmetric
-// sweeps from zero.  Threads cover only the nodes of the colour: thread
-// (kk, j, i) updates k = 2 kk + parity, blocks of 64 x 4 (kk, j).
+// Half sweep of colour on a coarsest level that is too large for a dense
+// solve (a side below 5 nodes) and for k3_sweeps: the finest level of a thin
+// grid (di null: its diagonal is 6) or a coarse one.  Threads cover only the
+// nodes of the colour: thread (kk, j, i) updates k = 2 kk + parity, blocks of
+// 64 x 4 (kk, j).
 constexpr int kRbgsX = 64, kRbgsY = 4;
-__global__ void __launch_bounds__(kRbgsX * kRbgsY) k3_rbgs(const uint8_t *nbm, float *x, const float *b, int nx,
-                                                           int ny, int nz, int colour, const int *stop)
+__global__ void __launch_bounds__(kRbgsX * kRbgsY) k3_rbgs(const uint8_t *nbm, const float *di, float *x,
+                                                           const float *b, int nx, int ny, int nz, int colour,
+                                                           const int *stop)
 {
     if (stopped(stop)) return;
     const int i = blockIdx.z, j = blockIdx.y * kRbgsY + threadIdx.y;
@@ -556,7 +558,7 @@ __global__ void __launch_bounds__(kRbgsX * kRbgsY) k3_rbgs(const uint8_t *nbm, f
     if (i >= nx || j >= ny || k >= nz) return;
     const int m = (i * ny + j) * nz + k;
     const uint8_t nb = nbm[m];
-    if (!(nb & kNbSelf)) x[m] = (b[m] + links7(nb, x, m, ny * nz, nz)) * (1.f / 6.f);
+    if (!(nb & kNbSelf)) x[m] = (b[m] + links7(nb, x, m, ny * nz, nz)) * (di ? di[m] : 1.f / 6.f);
 }
 
 __global__ void k3_zero(float *x, size_t n, const int *stop)
@@ -568,22 +570,46 @@ __global__ void k3_zero(float *x, size_t n, const int *stop)
 
 // A coarsest level too large for a dense solve (a thin grid's): kCoarseSweeps
 // symmetric red-black sweeps from zero, half of them in reverse order, by one
-// workgroup with barriers between the half sweeps
+// workgroup with barriers between the half sweeps.  A thread keeps its nodes'
+// right-hand sides, diagonals and links in registers and x is in LDS: with
+// all of them in memory a solve of 90 x 90 x 5 nodes took 6.0 ms, of 5 x 90 x
+// 90 3.0 (now 2.0 and 1.1).  Larger levels take a launch a half sweep
+// (k3_rbgs), 80 of about 2.5 us: a solve of 90 x 90 x 6 nodes, whose 8464
+// coarse nodes one workgroup swept in memory, 8.5 ms, now 4.0; of 200 x 200 x
+// 5 27.2 and 5.4.
 constexpr int kMaxLevels3 = 16;
+constexpr int kSweepsPer = 8;
+constexpr size_t kSweepsNodes = (size_t)kSweepsPer * kCoarseThreads;
 __global__ void __launch_bounds__(kCoarseThreads) k3_sweeps(const uint8_t *nbm, const float *di, const float *b,
                                                             float *x, int ny, int nz, int n, int sweeps,
                                                             const int *stop)
 {
     if (stopped(stop)) return;
-    for (int m = threadIdx.x; m < n; m += kCoarseThreads) x[m] = 0.f;
+    __shared__ float sx[kSweepsNodes];
+    uint8_t nb[kSweepsPer];
+    float bv[kSweepsPer], d[kSweepsPer];
+#pragma unroll
+    for (int q = 0; q < kSweepsPer; q++) {
+        const int m = threadIdx.x + q * kCoarseThreads, at = min(m, n - 1);
+        nb[q] = m < n ? nbm[at] : kNbSelf;
+        bv[q] = b[at];
+        d[q] = di[at];
+        sx[m] = 0.f;
+    }
     __syncthreads();
     for (int h = 0; h < 2 * sweeps; h++) {
         const uint8_t colour = (h & 1) == (h < sweeps ? 0 : 1) ? 0 : kNbBlack;
-        for (int m = threadIdx.x; m < n; m += kCoarseThreads) {
-            const uint8_t nb = nbm[m];
-            if ((nb & (kNbSelf | kNbBlack)) == colour) x[m] = (b[m] + links7(nb, x, m, ny * nz, nz)) * di[m];
+#pragma unroll
+        for (int q = 0; q < kSweepsPer; q++) {
+            const int m = threadIdx.x + q * kCoarseThreads;
+            if ((nb[q] & (kNbSelf | kNbBlack)) == colour) sx[m] = (bv[q] + links7(nb[q], sx, m, ny * nz, nz)) * d[q];
         }
         __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < kSweepsPer; q++) {
+        const int m = threadIdx.x + q * kCoarseThreads;
+        if (m < n) x[m] = sx[m];
     }
 }
 
@@ -1230,7 +1256,10 @@ static Host3 coarsen3(const Host3 &F)
 }
 
 constexpr size_t kCoarsest3 = 800;      // coarsening stops at this many nodes (9^3 = 729 and fewer)
-constexpr int kCoarseDenseMax = 1024;   // nodes for the dense coarsest solve
+// nodes for the dense coarsest solve: below kCoarsest3, or of a level with a
+// side that cannot be halved, of whose nodes few are free then (10 MB to read
+// at most: a solve of 36 x 36 x 6 nodes 455 us, by sweeps 2.0 ms)
+constexpr int kCoarseDenseMax = 1600;
 constexpr int kCoarseSweeps = 40;       // symmetric RB-GS sweeps otherwise
 
 // tiles of the finest and of the other levels (see k3_down)
@@ -1356,14 +1385,14 @@ static int vcycle3(m2d_fields3d *f, const float *rhs, float *out, double *dot, c
     float *zx = L == 1 ? out : Z.x;
     if (f->coarse_dense) {
         k3_dense<<<(unsigned)((Z.n + 3) / 4), 256, 0, s>>>(f->coarse_inv, zb, zx, (int)Z.n, stop);
-    } else if (L > 1) {
+    } else if (L > 1 && Z.n <= kSweepsNodes) {
         k3_sweeps<<<1, kCoarseThreads, 0, s>>>(Z.nbm, Z.di, zb, zx, Z.ny, Z.nz, (int)Z.n, kCoarseSweeps, stop);
     } else {
         const dim3 g((unsigned)(((Z.nz + 1) / 2 + kRbgsX - 1) / kRbgsX), (unsigned)((Z.ny + kRbgsY - 1) / kRbgsY),
                      (unsigned)Z.nx);
-        k3_zero<<<blocks_for(Z.n), 256, 0, s>>>(out, Z.n, stop);
+        k3_zero<<<blocks_for(Z.n), 256, 0, s>>>(zx, Z.n, stop);
         for (int h = 0; h < 2 * kCoarseSweeps; h++)
-            k3_rbgs<<<g, dim3(kRbgsX, kRbgsY), 0, s>>>(Z.nbm, out, rhs, Z.nx, Z.ny, Z.nz,
+            k3_rbgs<<<g, dim3(kRbgsX, kRbgsY), 0, s>>>(Z.nbm, Z.di, zx, zb, Z.nx, Z.ny, Z.nz,
                                                        h < kCoarseSweeps ? h & 1 : ~h & 1, stop);
     }
     for (int l = L - 2; l >= 1; l--) launch_up3<false>(f->lv[l], f->lv[l + 1], f->lv[l].b, f->lv[l].x, s, stop);

@@ -2,7 +2,8 @@
 nodes on), levels whose last tile is cut or whose last node lies past the fine
 grid (even sides), links cut by an electrode thinner than a coarse cell, a
 single dense level, a single level too large for that, a coarsest level too
-large for it, and the column kernels of 4 and 8 planes.
+large for it, swept by one workgroup or by launches (at, and one row past, the
+8192 nodes a workgroup holds), and the column kernels of 4 and 8 planes.
 
 Every solve is held to its own tolerance by the FP64 rows (1% for the
 rounding of the norms), repeats bit for bit, and needs few CG iterations (a
@@ -43,9 +44,10 @@ def solve(ctx, shape, mask, volt, rho, most):
 
 
 # large tiles with cut last ones; small tiles one short of, at and past their
-# sizes; even sides; a single dense level; a coarsest level swept
+# sizes; even sides; a single dense level; a coarsest level swept, or thin and dense
 @pytest.mark.parametrize("shape,most", [((128, 96, 90), 30), ((131, 83, 97), 30), ((101, 102, 103), 30),
-                                        ((16, 33, 64), 30), ((9, 9, 9), 30), ((10, 9, 9), 30), ((5, 60, 60), 200)])
+                                        ((16, 33, 64), 30), ((9, 9, 9), 30), ((10, 9, 9), 30), ((5, 60, 60), 200),
+                                        ((36, 36, 6), 30), ((90, 90, 6), 30), ((6, 63, 127), 30), ((6, 63, 129), 30)])
 def test_levels_and_tiles(ctx, shape, most):
     mask, volt, rho = scene3(*shape, seed=sum(shape))
     solve(ctx, shape, mask, volt, rho, most)
