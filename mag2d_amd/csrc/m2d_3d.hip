@@ -63,17 +63,27 @@ __device__ __forceinline__ void node3(size_t m, int ny, int nz, int &i, int &j, 
 }
 
 // ------------------------------------------------------------------ tables and solve kernels
-// blocks of 64 x 4 nodes (k, j) and a grid of (nz / 64, ny / 4, nx)
+// Kernels of a thread a node run in blocks of 64 x 4 nodes (k, j) and a grid
+// of (nz / 64, ny / 4, nx), which stops at the 65535 blocks that a launch takes
+// along y and z: their threads step on to the nodes past it.
+static dim3 planes3(int nx, int ny, int nz)
+{
+    return dim3((unsigned)((nz + 63) / 64), (unsigned)std::min((ny + 3) / 4, 65535), (unsigned)std::min(nx, 65535));
+}
+
 __global__ void __launch_bounds__(256) k3_tables(const double *u, int nx, int ny, int nz, double idx, double idy,
                                                  double idz, float *tx, float *ty, float *tz)
 {
-    const int i = blockIdx.z, j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.x * 64 + threadIdx.x;
-    if (j >= ny || k >= nz) return;
-    const size_t m = ((size_t)i * ny + j) * nz + k, sx = (size_t)ny * nz;
-    const double c = u[m], ux = u[i >= 1 ? m - sx : m], uy = u[j >= 1 ? m - nz : m], uz = u[k >= 1 ? m - 1 : m];
-    tx[m] = (float)((c - ux) * idx);
-    ty[m] = (float)((c - uy) * idy);
-    tz[m] = (float)((c - uz) * idz);
+    const int k = blockIdx.x * 64 + threadIdx.x;
+    if (k >= nz) return;
+    for (int i = blockIdx.z; i < nx; i += gridDim.z)
+        for (int j = blockIdx.y * 4 + threadIdx.y; j < ny; j += gridDim.y * 4) {
+            const size_t m = ((size_t)i * ny + j) * nz + k, sx = (size_t)ny * nz;
+            const double c = u[m], ux = u[i >= 1 ? m - sx : m], uy = u[j >= 1 ? m - nz : m], uz = u[k >= 1 ? m - 1 : m];
+            tx[m] = (float)((c - ux) * idx);
+            ty[m] = (float)((c - uy) * idy);
+            tz[m] = (float)((c - uz) * idz);
+        }
 }
 
 // u += e on free nodes
@@ -800,20 +810,24 @@ __device__ __forceinline__ void wave_deposit3(int cell, const uint32_t w8[8], co
 }
 
 // rho += charge * (sum of the records of the 8 cells around the node) *
-// 2^-31; blocks of 64 x 4 nodes (k, j) and a grid of (nz / 64, ny / 4, nx)
+// 2^-31 (launched on planes3)
 __global__ void __launch_bounds__(256) k3_flush_rec(const unsigned long long *rec, double *rho, double charge, int nx,
                                                     int ny, int nz)
 {
-    const int i = blockIdx.z, j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.x * 64 + threadIdx.x;
-    if (j >= ny || k >= nz) return;
-    const size_t sx = (size_t)ny * nz, m = (size_t)i * sx + (size_t)j * nz + k;
-    unsigned long long v = 0;
+    const int k = blockIdx.x * 64 + threadIdx.x;
+    if (k >= nz) return;
+    const size_t sx = (size_t)ny * nz;
+    for (int i = blockIdx.z; i < nx; i += gridDim.z)
+        for (int j = blockIdx.y * 4 + threadIdx.y; j < ny; j += gridDim.y * 4) {
+            const size_t m = (size_t)i * sx + (size_t)j * nz + k;
+            unsigned long long v = 0;
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-        const int a = q & 1, b = (q >> 1) & 1, c = q >> 2;
-        if (i >= a && j >= b && k >= c) v += rec[8 * (m - a * sx - (size_t)b * nz - c) + q];
-    }
-    if (v) rho[m] += charge * ((double)(long long)v * kInvFix);
+            for (int q = 0; q < 8; q++) {
+                const int a = q & 1, b = (q >> 1) & 1, c = q >> 2;
+                if (i >= a && j >= b && k >= c) v += rec[8 * (m - a * sx - (size_t)b * nz - c) + q];
+            }
+            if (v) rho[m] += charge * ((double)(long long)v * kInvFix);
+        }
 }
 
 // mod (mymath.cpp:62-67)
@@ -1483,8 +1497,8 @@ static void queue_residual3(m2d_fields3d *f, double tol, bool first)
 
 static int build_tables3(m2d_fields3d *f)
 {
-    k3_tables<<<dim3((unsigned)((f->nz + 63) / 64), (unsigned)((f->ny + 3) / 4), (unsigned)f->nx), dim3(64, 4), 0,
-                f->ctx->stream>>>(f->u, f->nx, f->ny, f->nz, f->idx, f->idy, f->idz, f->tx, f->ty, f->tz);
+    k3_tables<<<planes3(f->nx, f->ny, f->nz), dim3(64, 4), 0, f->ctx->stream>>>(
+        f->u, f->nx, f->ny, f->nz, f->idx, f->idy, f->idz, f->tx, f->ty, f->tz);
     M2D_HIP(hipGetLastError());
     return M2D_OK;
 }
@@ -1555,8 +1569,8 @@ static bool use_rec3(int64_t particles, size_t nodes)
 
 static int flush_rec3(m2d_ctx *ctx, double *rho, double charge, int nx, int ny, int nz)
 {
-    k3_flush_rec<<<dim3((unsigned)((nz + 63) / 64), (unsigned)((ny + 3) / 4), (unsigned)nx), dim3(64, 4), 0,
-                   ctx->stream>>>((const unsigned long long *)ctx->rec.ptr, rho, charge, nx, ny, nz);
+    k3_flush_rec<<<planes3(nx, ny, nz), dim3(64, 4), 0, ctx->stream>>>((const unsigned long long *)ctx->rec.ptr, rho,
+                                                                       charge, nx, ny, nz);
     M2D_HIP(hipGetLastError());
     return rec_done(ctx, (size_t)nx * ny * nz, 8);
 }

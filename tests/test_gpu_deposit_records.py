@@ -139,6 +139,42 @@ def test_advance_3d(ctx):
         assert np.array_equal(step(slice(0, n)), want)
 
 
+@pytest.mark.parametrize("axis", [0, 1])
+def test_grids_longer_than_a_launch(ctx, axis):
+    """Sides past the 65535 blocks (of one and of four nodes) a launch takes:
+    the field's tables and the record flush on the long axis against the same
+    grid with that axis along z, where a launch has room.  The weights' products
+    round in another order: each within a few of their 2^31 units, and the
+    step's FP32 arithmetic to 1e-5 of the kick."""
+    rng = np.random.default_rng(axis)
+    long, n, h = (70_000, 262_153)[axis], 300_000, 1e-4
+    u = rng.normal(size=(3, 3, long))
+    cells = [rng.uniform(0, 1.999, n), rng.uniform(0, 1.999, n), rng.uniform(0, long - 1.001, n)]
+    out = []
+    for order in ((0, 1, 2), (2, 0, 1) if axis == 0 else (0, 2, 1)):  # grid axis -> axis of u
+        shape = [u.shape[a] for a in order]
+        g = abi.grid3d(*shape, h, h, h)
+        mask = np.full(shape, abi.FIXED, np.uint8)
+        mask[1:-1, 1:-1, 1:-1] = abi.FREE
+        prm = abi.Fields3DParams(g, *(h * (s - 1) for s in shape), abi.BC_FREE, 0.0, 0.0, 0.0, 1.0)
+        fields = abi.Fields3D(ctx, prm, mask, np.zeros(mask.size))
+        fields.upload(abi.FIELD_U, np.ascontiguousarray(u.transpose(order)))
+        zero = np.zeros(n, np.float32)
+        P = abi.ParticlesSoA3D.from_host(ctx, *((cells[a] * h).astype(np.float32) for a in order), zero, zero, zero)
+        rho = ctx.to_device(np.zeros(mask.size))
+        abi.accumulate_3d(ctx, g, P, UNIT, rho.ptr)
+        sp = abi.Species2D(1.0, 1.0, 1e-9, float("inf"), 0, 0, 0)
+        abi.advance_3d(ctx, fields, sp, P, flags=abi.STEP_PUSH)
+        d = P.download()
+        back = np.argsort(order)
+        out.append((rho.get().reshape(shape).transpose(back), [d["v" + "xyz"[a]] for a in back]))
+    (r0, v0), (r1, v1) = out
+    assert r0.sum() == r1.sum() == UNIT * n
+    assert np.abs(r0 - r1).max() <= 8 * 200  # at most 200 particles around a node, 8 units each
+    for a, b in zip(v0, v1):
+        assert np.abs(a - b).max() <= 1e-5 * np.abs(a).max()
+
+
 def test_captured_deposit_outlives_larger_records(ctx):
     """A captured deposit replays right after a call that outgrew the records
     (it runs on the node grid)."""
