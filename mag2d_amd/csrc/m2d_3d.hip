@@ -54,14 +54,6 @@ namespace m2d {
 
 __device__ __forceinline__ bool dir3(uint8_t m) { return m == M2D_FIXED || m == M2D_FIXED_RF; }
 
-__device__ __forceinline__ void node3(size_t m, int ny, int nz, int &i, int &j, int &k)
-{
-    k = (int)(m % nz);
-    size_t t = m / nz;
-    j = (int)(t % ny);
-    i = (int)(t / ny);
-}
-
 // ------------------------------------------------------------------ tables and solve kernels
 // Kernels of a thread a node run in blocks of 64 x 4 nodes (k, j) and a grid
 // of (nz / 64, ny / 4, nx), which stops at the 65535 blocks that a launch takes
@@ -980,7 +972,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
               wk0 = (t % ntz3) * kTile3 - kHalo3;
     for (int k = threadIdx.x; k < kWinN3; k += 256) win[k] = 0ull;
     __syncthreads();
-    bool removed_any = false, coll_any = false, nan_any = false, bad_any = false;
+    bool nan_any = false, bad_any = false;
     int n_removed = 0, n_coll = 0, n_spill = 0;
     for (int64_t p = s.y + threadIdx.x; p < s.z; p += 256) {
         Step3 o;
@@ -1005,7 +997,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
             }
         }
     }
-    (void)removed_any; (void)coll_any;
     __syncthreads();
     for (int k = threadIdx.x; k < kWinN3; k += 256) {
         const unsigned long long v = win[k];
@@ -1154,13 +1145,12 @@ static int check_parts3(const m2d_particles3d *p)
     return M2D_OK;
 }
 
-// blocks of the fused reductions over the finest level: one node a thread up
-// to kRed3Blocks blocks (524288 nodes), then that many, whose threads stride
-// over several nodes (each block's reduction and partial sum then serve more
-// nodes; the FP64 sums' order changes with the count, and with it their last
-// bits, which the FP32 CG coefficients round away in practice).  At 128^3,
-// 2048 blocks made the step 3% faster than one node a thread, 1024 and 4096
-// less so.
+// Blocks of the linear reductions over the finest level: a block per 256 nodes
+// up to kRed3Blocks, then that many, whose threads stride over several nodes
+// (four at a time).  kRed3Blocks = kFinBlocks, so that the sums are finished
+// in the launch itself.  A solve of 128^3 nodes: 256, 512 and 1024 blocks
+// 1.46, 1.45 and 1.46 ms, 2048 1.48, as many as 256 nodes each give 1.58
+// (96 x 112 x 128: 1.34, 1.34, 1.34, 1.37 and 1.42).
 constexpr size_t kRed3Blocks = 1024;
 static unsigned red_blocks3(size_t n)
 {

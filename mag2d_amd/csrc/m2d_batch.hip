@@ -40,7 +40,6 @@ struct BatchRun {
 // argument block: field / grid members named as gather_E expects them
 struct BatchArgs {
     float *x, *z, *vx, *vy, *vz;
-    int64_t n;
     float *xl, *zl;          // position remainders (long-time positions), or null
     const float2 *gx, *gz;
     const uint8_t *cellfree;
@@ -379,7 +378,7 @@ static void batch_args(const m2d_batch *b, const m2d_particles2d &p, BatchArgs &
     const m2d_fields2d *f = b->f;
     const m2d_fields2d_params &P = f->p;
     const m2d_species2d *s = &b->s;
-    a.x = p.x; a.z = p.z; a.vx = p.vx; a.vy = p.vy; a.vz = p.vz; a.n = p.n;
+    a.x = p.x; a.z = p.z; a.vx = p.vx; a.vy = p.vy; a.vz = p.vz;
     a.xl = p.xl; a.zl = p.zl;
     a.gx = f->gx; a.gz = f->gz; a.cellfree = f->cellfree;
     a.nx = f->nx; a.nz = f->nz; a.idx = f->idx; a.idz = f->idz;

@@ -122,44 +122,6 @@ __device__ __forceinline__ float apply9(const float *st, const float *x, int i, 
     return s;
 }
 
-// finest level: 5-point operator from the mask, A' = 4I - adjacency(free)
-__device__ __forceinline__ float apply5(const uint8_t *dir, const float *x, size_t k, int nz)
-{
-    float s = 4.f * x[k];
-    if (!dir[k - nz]) s -= x[k - nz];
-    if (!dir[k - 1]) s -= x[k - 1];
-    if (!dir[k + 1]) s -= x[k + 1];
-    if (!dir[k + nz]) s -= x[k + nz];
-    return s;
-}
-
-// red-black Gauss-Seidel update of node (i, j) of colour (i+j)&1 on the
-// finest level
-__device__ __forceinline__ void node_rbgs5(const uint8_t *dir, float *x, const float *b, int nz, size_t k)
-{
-    if (dir[k]) return;
-    float s = b[k];
-    if (!dir[k - nz]) s += x[k - nz];
-    if (!dir[k - 1]) s += x[k - 1];
-    if (!dir[k + 1]) s += x[k + 1];
-    if (!dir[k + nz]) s += x[k + nz];
-    x[k] = 0.25f * s;
-}
-
-// half sweep (colour = (i+j)&1)
-__global__ void k_rbgs5(const uint8_t *dir, float *x, const float *b, int nx, int nz, int colour)
-{
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    int i = blockIdx.y;
-    if (j >= nz || ((i + j) & 1) != colour) return;
-    node_rbgs5(dir, x, b, nz, (size_t)i * nz + j);
-}
-
-__device__ __forceinline__ float node_resid5(const uint8_t *dir, const float *x, const float *b, int nz, size_t k)
-{
-    return dir[k] ? 0.f : b[k] - apply5(dir, x, k, nz);
-}
-
 // weighted Jacobi on a 9-point level: xo = xi + w D^-1 (b - A xi)
 __device__ __forceinline__ float node_jacobi9(const float *st, const float *dinv, const float *xi, const float *b,
                                               int nx, int nz, float w, int i, int j)
@@ -169,29 +131,11 @@ __device__ __forceinline__ float node_jacobi9(const float *st, const float *dinv
     return dv == 0.f ? 0.f : xi[k] + w * dv * (b[k] - apply9(st, xi, i, j, nx, nz));
 }
 
-__global__ void k_jacobi9(const float *st, const float *dinv, const float *xi, float *xo,
-                          const float *b, int nx, int nz, float w)
-{
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    int i = blockIdx.y;
-    if (j >= nz) return;
-    xo[(size_t)i * nz + j] = node_jacobi9(st, dinv, xi, b, nx, nz, w, i, j);
-}
-
 __device__ __forceinline__ float node_resid9(const float *st, const float *dinv, const float *x, const float *b,
                                              int nx, int nz, int i, int j)
 {
     size_t k = (size_t)i * nz + j;
     return dinv[k] == 0.f ? 0.f : b[k] - apply9(st, x, i, j, nx, nz);
-}
-
-__global__ void k_resid9(const float *st, const float *dinv, const float *x, const float *b, float *r,
-                         int nx, int nz)
-{
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    int i = blockIdx.y;
-    if (j >= nz) return;
-    r[(size_t)i * nz + j] = node_resid9(st, dinv, x, b, nx, nz, i, j);
 }
 
 // b_c = P^T r_f with P the bilinear interpolation masked on fine Dirichlet nodes
@@ -213,15 +157,6 @@ __device__ __forceinline__ float node_restrict(const float *rf, int nxf, int nzf
         }
     }
     return s;
-}
-
-__global__ void k_restrict(const float *rf, int nxf, int nzf, float *bc, const float *dinvc, int nxc,
-                           int nzc)
-{
-    int J = blockIdx.x * blockDim.x + threadIdx.x;
-    int I = blockIdx.y;
-    if (J >= nzc) return;
-    bc[(size_t)I * nzc + J] = node_restrict(rf, nxf, nzf, dinvc, nzc, I, J);
 }
 
 // x_f += P x_c on free fine nodes
@@ -254,15 +189,6 @@ __device__ __forceinline__ void node_prolong(float *xf, const uint8_t *dirf, int
         s = 0.5f * (a + b);
     }
     xf[k] += s;
-}
-
-__global__ void k_prolong(float *xf, const uint8_t *dirf, int nxf, int nzf, const float *xc, int nxc,
-                          int nzc)
-{
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    int i = blockIdx.y;
-    if (j >= nzf) return;
-    node_prolong(xf, dirf, nzf, xc, nxc, nzc, i, j);
 }
 
 // dense coarsest solve x = A^-1 b, one block
@@ -300,7 +226,6 @@ __global__ void __launch_bounds__(kRedBlock) k_dot_fin(const float *a, const flo
     finish_sums<1>(v, partial, ticket, out, fin);
 }
 
-// q = A' p on the finest level, out = p.q
 // The CG direction and the operator in one launch: p' = z + beta p (first:
 // p' = z), q = A' p' and out = p'.q.  Each node's p' is recomputed at its
 // stencil neighbours from z and p -- the same operations as at the node
@@ -321,7 +246,6 @@ __global__ void __launch_bounds__(kRedBlock) k_dir_apply5_dot(const uint8_t *dir
         pn[k] = pk;
         float y = 0.f;
         if (!dir[k]) {
-            // apply5's order
             float t = 4.f * pk;
             if (!dir[k - nz]) t -= cg_dir_at(z, p, k - nz, beta, first);
             if (!dir[k - 1]) t -= cg_dir_at(z, p, k - 1, beta, first);
@@ -456,9 +380,8 @@ __device__ __forceinline__ float prolong_at(const float *xc, int nxc, int nzc, i
 // nodes (16, 8 or 4 by the grid's size, see l0_tile) plus a halo and runs several red-black half sweeps on it with
 // workgroup barriers in between.  A node at distance d from the halo's edge
 // keeps the exact global value for d half sweeps after the first, so the
-// halo is as wide as the sweeps (and the residual stencil) need.  Updates
-// use the node_rbgs5 order of additions, so the result is the same as the
-// half sweeps run one launch each.
+// halo is as wide as the sweeps (and the residual stencil) need.  The
+// result is that of half sweeps run one launch each.
 constexpr int kH0d = 2 * kPre + 1;   // descent: 2 kPre - 1 sweeps, residual, restriction
 constexpr int kH0u = 2 * kPost;      // ascent: 2 kPost sweeps
 constexpr int kT0Threads = 256;
@@ -510,7 +433,7 @@ __global__ void __launch_bounds__(kT0Threads) k_l0_down(const uint8_t *dir, cons
         tile_rbgs<S>(sx, sb, sd, i0, j0, h & 1);
         __syncthreads();
     }
-    // residual (node_resid5) where it reads only exact x: the 2 kPre - 1
+    // residual where it reads only exact x: the 2 kPre - 1
     // sweeps after the first left the outer 2 kPre - 1 rings inexact
     constexpr int R = 2 * kPre;
     for (int t = threadIdx.x; t < S * S; t += kT0Threads) {
