@@ -445,10 +445,7 @@ int m2d_adjoint_energy_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s,
             for (int c = 0; c < 5; c++)
                 M2D_HIP(hipMemcpyAsync(ckpt.as<float>() + ((size_t)(n / K) * 5 + c) * np, parr[c],
                                        sizeof(float) * np, hipMemcpyDeviceToDevice, st));
-        // the differentiated run and its reverse sweep keep the multigrid
-        // solve: a gradient carries its solves' 1e-10 in full (the direct
-        // solve moved one of a small run by 3e-9)
-        M2D_TRY(fields_solve_multigrid(f, M2D_SOLVE_STATIC, 1e-10, &si));
+        M2D_TRY(m2d_fields2d_solve(f, M2D_SOLVE_STATIC, 1e-10, &si));
         if (grad)
             M2D_HIP(hipMemcpyAsync(U.as<double>() + (size_t)n * nc, f->u, sizeof(double) * nc,
                                    hipMemcpyDeviceToDevice, st));
@@ -491,7 +488,12 @@ int m2d_adjoint_energy_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s,
     k_adj_init2d<<<nblk(np), 256, 0, st>>>(p->x, p->vx, p->vy, p->vz, p->n,
                                            s->mass / (kQE * (double)live), lx, lz, lvx, lvy, lvz);
     M2D_HIP(hipGetLastError());
-    // the adjoint solver: same mask and operator, zero Dirichlet values
+    // The adjoint solver: same mask and operator, zero Dirichlet values.  It
+    // is the multigrid on rectangles too.  A gradient there lies as far from
+    // the one of solves to 1e-13 as its reverse solves' 1e-10 leave it (2e-12
+    // to 1.5e-9 of it on 60 runs; with direct reverse solves 1e-14 to 7e-12,
+    // on 8 others), but direct ones would move the gradients of existing runs
+    // by up to 3e-9.
     m2d_fields2d *af = nullptr;
     {
         std::vector<double> zero(nc, 0.0);
@@ -577,7 +579,7 @@ int m2d_adjoint_energy_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s,
             // A_FF y = lu_F
             k_adj_rhs<<<gb, 256, 0, st>>>(f->mask, lu.as<double>(), af->rho, nc);
             M2D_HIP(hipGetLastError());
-            M2D_TRY(fields_solve_multigrid(af, M2D_SOLVE_RAW, adj_tol, &si));
+            M2D_TRY(m2d_fields2d_solve(af, M2D_SOLVE_RAW, adj_tol, &si));
             k_adj_groups<<<gb, 256, 0, st>>>(f->mask, dgroup.as<int>(), lu.as<double>(), af->u, f->nx, f->nz,
                                              cfg->n_groups, gpart.as<double>());
             k_adj_groups_sum<<<cfg->n_groups, 256, 0, st>>>(gpart.as<double>(), (int)gb, cfg->n_groups,

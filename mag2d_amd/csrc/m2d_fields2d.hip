@@ -1075,24 +1075,15 @@ static int mg_setup(m2d_fields2d *f)
     return M2D_OK;
 }
 
-// what mg_setup allocates, whole or in part
-static void mg_free_levels(Mg &mg)
+static void mg_free(Mg &mg)
 {
     for (MgLevel &L : mg.lv)
         for (void *p : {(void *)L.st, (void *)L.dinv, (void *)L.dir, (void *)L.x, (void *)L.x2,
                         (void *)L.r, (void *)L.b})
             if (p) (void)hipFree(p);
     mg.lv.clear();
-    for (float **p : {&mg.coarse_inv, &mg.coarse_invT, &mg.pz, &mg.pp, &mg.pp2, &mg.pq, &mg.pe}) {
-        if (*p) (void)hipFree(*p);
-        *p = nullptr;
-    }
-}
-
-static void mg_free(Mg &mg)
-{
-    mg_free_levels(mg);
-    for (void *p : {(void *)mg.pr, (void *)mg.r64, (void *)mg.dots, (void *)mg.partial, (void *)mg.ticket})
+    for (void *p : {(void *)mg.coarse_inv, (void *)mg.pr, (void *)mg.pz, (void *)mg.pp, (void *)mg.pp2, (void *)mg.pq,
+                    (void *)mg.pe, (void *)mg.r64, (void *)mg.dots, (void *)mg.partial, (void *)mg.ticket, (void *)mg.coarse_invT})
         if (p) (void)hipFree(p);
     if (mg.h_dots) (void)hipHostFree(mg.h_dots);
     mg = Mg();
@@ -1326,8 +1317,7 @@ static void queue_first_residual(m2d_fields2d *f, double *u, int mode, double sc
 
 // FP64 refinement whose every pass is the direct solve of its residual: one
 // pass meets any tolerance FP64 can hold on most grids, and as many as the
-// last direct solve took are queued before the host reads the control block
-// (the field's multigrid solves keep their own estimate)
+// last solve took are queued before the host reads the control block
 static int refine_direct(m2d_fields2d *f, double *u, double tol)
 {
     Mg &mg = f->mg;
@@ -1351,7 +1341,7 @@ static int refine_direct(m2d_fields2d *f, double *u, double tol)
 // FP64 iterative refinement of u over FP32 multigrid-preconditioned CG
 // passes, queued whole (queue_refinement); direct: where the field has the
 // direct solve
-static int solve(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info, bool direct)
+static int solve(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info)
 {
     hipStream_t s = f->ctx->stream;
     Mg &mg = f->mg;
@@ -1363,7 +1353,7 @@ static int solve(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info, bo
     SolveCtl *ctl = solve_ctl(mg);
     SolveCtl *h = (SolveCtl *)(mg.h_dots + 16);
     queue_first_residual(f, u, mode, scale, tol, kMaxOuter);
-    if (direct)
+    if (f->direct.on)
         M2D_TRY(refine_direct(f, u, tol));
     else
         M2D_TRY(queue_refinement(
@@ -1378,18 +1368,6 @@ static int solve(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info, bo
         return set_error(M2D_ERR_NOT_CONVERGED, "Fields solve: relative residual %.3e > %.3e after %d steps",
                          h->rel, tol, h->outer);
     return M2D_OK;
-}
-
-int fields_solve_multigrid(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info)
-{
-    if (f->mg.lv.empty()) {
-        const int r = mg_setup(f);
-        if (r != M2D_OK) {
-            mg_free_levels(f->mg);
-            return r;
-        }
-    }
-    return solve(f, mode, tol, info, false);
 }
 
 }  // namespace m2d
@@ -1648,7 +1626,7 @@ int m2d_fields2d_solve(m2d_fields2d *f, int mode, double tol, m2d_solve_info *in
     M2D_CHECK(f, M2D_ERR_BAD_ARG, "m2d_fields2d_solve: NULL argument");
     M2D_CHECK(mode == M2D_SOLVE_STATIC || mode == M2D_SOLVE_RF || mode == M2D_SOLVE_RAW, M2D_ERR_BAD_ARG,
               "m2d_fields2d_solve: unknown mode %d", mode);
-    return solve(f, mode, tol, info, f->direct.on);
+    return solve(f, mode, tol, info);
 }
 
 }  // extern "C"

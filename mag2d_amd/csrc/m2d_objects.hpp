@@ -113,8 +113,7 @@ struct m2d_fields2d {
     m2d_grid2d bgrid{};
     double *smooth_tmp = nullptr;  // nx*nz copy of the field u_smooth filters
     m2d::Mg mg;
-    m2d::Direct2 direct;          // on: the solve is direct, and mg holds levels only from the first
-                                  // fields_solve_multigrid on
+    m2d::Direct2 direct;          // on: the solve is direct, and mg holds no levels
     std::vector<uint8_t> h_mask;
 };
 
@@ -131,10 +130,6 @@ int fields_build_tables(m2d_fields2d *f);
 // m2d_fields2d_create; direct: with the direct solve where the mask allows it
 int fields_create(m2d_ctx *ctx, const m2d_fields2d_params *p, const uint8_t *mask, const double *voltage, bool direct,
                   m2d_fields2d **out);
-// m2d_fields2d_solve by multigrid-PCG, also where the field has the direct
-// solve: a field's first such call sets the levels up, which it then keeps
-// (a set-up that fails leaves none, so the next call tries again)
-int fields_solve_multigrid(m2d_fields2d *f, int mode, double tol, m2d_solve_info *info);
 bool direct2d_fits(const std::vector<uint8_t> &mask, int nx, int nz, Direct2 &d);
 int direct2d_setup(m2d_fields2d *f);
 int direct2d_pass(m2d_fields2d *f, double *u, SolveCtl *ctl, bool surplus);

@@ -1,7 +1,8 @@
 """The adjoint of the gather in the outer half cells of the grid, where its
 two edges are clamped onto one: the gradient of a run that starts there
-against central differences of the FP64 oracle.  Stores of any slot count, and
-a field that is solved, differentiated and solved again."""
+against central differences of the FP64 oracle.  Stores of any slot count, the
+differentiated run against the plain one, and a field that is solved,
+differentiated and solved again."""
 import numpy as np
 import pytest
 
@@ -85,6 +86,33 @@ def test_slot_counts_of_any_remainder(ctx, count):
 
 
 @pytest.mark.parametrize("electrode", [False, True])
+def test_the_differentiated_run_is_the_plain_run(ctx, electrode):
+    """The store, u and rho end as the same steps leave them, bit for bit."""
+    fields, group = small_run(ctx, electrode=electrode)
+    x, z, v = electrons(1200, 2e-2, np.random.default_rng(2))
+    steps, ends = 9, []
+    for grad in (None, False, True):
+        P = abi.ParticlesSoA.from_host(ctx, x, z, *v)
+        fields.upload(abi.FIELD_U, np.zeros(group.size))
+        if grad is None:
+            fields.reset()
+            rho = fields.ptr(abi.FIELD_RHO)
+            abi.accumulate(ctx, fields.params.grid, P, -QE, rho)
+            for k in range(steps):
+                fields.solve(abi.SOLVE_STATIC, 1e-10)
+                fields.reset()
+                abi.advance(ctx, fields, abi.Species2D(-QE, M_E, 1e-11, float("inf"), k, 0, 0), P, rho_ptr=rho,
+                            flags=abi.STEP_PUSH | abi.STEP_BOUNDARY | abi.STEP_DEPOSIT)
+        else:
+            abi.adjoint_energy(ctx, fields, abi.Species2D(-QE, M_E, 1e-11, float("inf"), 0, 0, 0), P, steps,
+                               group=group if grad else None, n_groups=8, checkpoint_every=4)
+        ends.append({**P.download(), "u": fields.download(abi.FIELD_U), "rho": fields.download(abi.FIELD_RHO)})
+    for e in ends[1:]:
+        for k in ends[0]:
+            assert np.array_equal(e[k].view(np.uint8), ends[0][k].view(np.uint8)), k
+
+
+@pytest.mark.parametrize("electrode", [False, True])
 def test_solves_around_a_gradient_are_the_same(ctx, electrode):
     """A field keeps what its gradients set up and queue apart from its own
     solves: the same charge gives the same bits and counts before and after."""
@@ -109,9 +137,9 @@ def test_solves_around_a_gradient_are_the_same(ctx, electrode):
 
 
 def test_a_refused_hierarchy_is_refused_alike_each_time(ctx):
-    """A 4 x 850 box is solved directly, but its gradient's multigrid has no
-    coarse level small enough: a bad argument, in the first call and in later
-    ones, which leaves the field's own solves as they were."""
+    """A 4 x 850 box is solved directly, but its gradient's reverse solves, by
+    multigrid, have no coarse level small enough: a bad argument, in the first
+    call and in later ones, which leaves the field's own solves as they were."""
     nx, nz, h = 4, 850, 1e-4
     mask = np.full((nx, nz), abi.FIXED, np.uint8)
     mask[1:-1, 1:-1] = abi.FREE
@@ -128,6 +156,7 @@ def test_a_refused_hierarchy_is_refused_alike_each_time(ctx):
         assert fields.solve(abi.SOLVE_STATIC, 1e-10).rel_residual <= 1e-10
         us.append(fields.download(abi.FIELD_U).tobytes())
         with pytest.raises(abi.M2DError) as e:
-            abi.adjoint_energy(ctx, fields, abi.Species2D(-QE, M_E, 1e-11, float("inf"), 0, 0, 0), P, 2)
+            abi.adjoint_energy(ctx, fields, abi.Species2D(-QE, M_E, 1e-11, float("inf"), 0, 0, 0), P, 2,
+                               group=np.full(nx * nz, -1), n_groups=1)
         assert abi.STATUS[e.value.code] == "BAD_ARG", e.value
     assert us[0] == us[1] == us[2]
