@@ -488,16 +488,18 @@ int m2d_adjoint_energy_2d(m2d_ctx *ctx, m2d_fields2d *f, const m2d_species2d *s,
     k_adj_init2d<<<nblk(np), 256, 0, st>>>(p->x, p->vx, p->vy, p->vz, p->n,
                                            s->mass / (kQE * (double)live), lx, lz, lvx, lvy, lvz);
     M2D_HIP(hipGetLastError());
-    // The adjoint solver: same mask and operator, zero Dirichlet values.  It
-    // is the multigrid on rectangles too.  A gradient there lies as far from
-    // the one of solves to 1e-13 as its reverse solves' 1e-10 leave it (2e-12
-    // to 1.5e-9 of it on 60 runs; with direct reverse solves 1e-14 to 7e-12,
-    // on 8 others), but direct ones would move the gradients of existing runs
-    // by up to 3e-9.
+    // The adjoint solver: same mask and operator, zero Dirichlet values.  On
+    // rectangles it is the direct solve where the caller asks for less than the
+    // default residual (500k ions on 256^2 at 1e-8: a gradient takes 3.4 forward
+    // runs, 0.87 s for 2000 steps; by multigrid 6.2, 1.58 s).  At the default it is the multigrid: a gradient
+    // then lies as far from the one of solves to 1e-13 as the reverse solves'
+    // 1e-10 leave it (2e-12 to 1.5e-9 of it on 60 runs; with direct ones 1e-14
+    // to 7e-12, on 8 others), but direct ones would move the gradients that
+    // existing runs give by up to 3e-9.
     m2d_fields2d *af = nullptr;
     {
         std::vector<double> zero(nc, 0.0);
-        M2D_TRY(fields_create(ctx, &f->p, f->h_mask.data(), zero.data(), false, &af));
+        M2D_TRY(fields_create(ctx, &f->p, f->h_mask.data(), zero.data(), adj_tol > 1e-10, &af));
     }
     struct Closer { m2d_fields2d *f; ~Closer() { m2d_fields2d_destroy(f); } } closer{af};
     AdjArgs a{};
