@@ -439,7 +439,8 @@ typedef struct {
     int32_t n_groups;            /* electrode voltages differentiated, <= 64 */
     const int32_t *group;        /* host, nx*nz: group of each FIXED node, -1 for none */
     double adjoint_tol;          /* FP64 relative residual of the adjoint solves; 0: 1e-10, the
-                                    forward solves' (the forward run always solves to 1e-10) */
+                                    forward solves' (the forward run always solves to 1e-10);
+                                    looser than that, fields with the direct solve use it */
     m2d_mcc *mcc;                /* NULL: no collisions; else the species' MCC (continuum targets
                                     only), stepped with the species' lifetime */
 } m2d_adjoint_cfg;

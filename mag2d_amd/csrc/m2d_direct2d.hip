@@ -1,6 +1,8 @@
 // m2d_direct2d.hip -- the direct form of the 2D Poisson solve, for fields
-// whose free nodes fill a rectangle (EMPTY, PENNING_SIMPLE and every other
-// grid whose electrodes leave a box: a frame, end caps, grounded walls).
+// whose free nodes fill a rectangle: EMPTY and any grid whose electrodes leave
+// a box (a frame, thick walls, end caps along whole walls).  Electrodes with
+// gaps between them or inside the box (the named traps, a probe) leave no
+// rectangle.
 //
 // On a full m x n rectangle between Dirichlet nodes the 5-point operator
 // A' = 4 - (sum of neighbours) is diagonal in the discrete sine basis:

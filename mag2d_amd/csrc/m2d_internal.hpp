@@ -187,8 +187,12 @@ int ensure(m2d_ctx *ctx, Scratch &s, size_t bytes, bool optional = false);
 // fixed-point flush (m2d_particles2d.hip)
 // The solver kernels take `stop`, a device flag that the solve's own control
 // kernels set once an iteration is not to run: a launch whose flag is set
-// returns at once (the flag is set before the launch starts and read the same
+// changes nothing (the flag is set before the launch starts and read the same
 // by every thread, so a whole launch runs or none of it).  Null: always run.
+// Most test it first (stopped()) and return at once.  Where waiting for the
+// flag would delay the operands' loads, it is read beside them and tested
+// after (the 3D V-cycle and column kernels; k_dst_stage in a solve's first
+// pass, which runs unless the first guess was good enough).
 __device__ __forceinline__ bool stopped(const int *stop) { return stop && *stop; }
 // the CG direction at node k: p' = z + beta p (first: p' = z), beta = rz_new / rz_old
 __device__ __forceinline__ float cg_beta(const double *rz_new, const double *rz_old)
@@ -242,7 +246,7 @@ int read_counters(m2d_ctx *ctx);
 // FP32 copy).  Small kernels of one thread keep it between the launches, so
 // the refinement and its CG passes are queued whole and read on the host
 // once: a pass that has converged turns the launches queued after it into
-// launches that return at once (see stopped()).
+// launches that change nothing (see stopped()).
 constexpr int kMaxOuter = 12;            // refinement passes at most
 constexpr int kMaxPasses = kMaxOuter + 1;
 struct SolveCtl {

@@ -268,7 +268,13 @@ __device__ __forceinline__ long long rec_node2(const unsigned long long *rec, si
 // in the generic forms with a gridded B or long-time positions; the scatter's
 // FP64 chain in the pass (SCAT) keeps three.  Each is
 // the most that builds without spilling to scratch memory, which costs far
-// more than the occupancy gains.
+// more than the occupancy gains; but the specialised tiled form with
+// collisions and the two-component tables spills 2 VGPRs at five (20 steps of
+// 4.2M slots 994 us; at four, where it does not, 999).  The untiled deposits
+// with a wavefront or two fewer than the rest are no slower for it where they
+// add at the nodes (10 steps against the forms of four wavefronts that summed
+// runs of equal cells first: 12k slots on 128^2 299 -> 233 us, 200k on 512^2
+// 508 -> 341, with a gridded B 558 -> 374).
 template <bool DEPOSIT, bool TILED, bool FAST, bool BGRID, bool PHT, bool HIPOS, bool SCAT>
 constexpr int pass_waves()
 {
