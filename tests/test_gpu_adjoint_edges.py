@@ -126,8 +126,9 @@ def test_reverse_solves_of_either_kind(ctx, electrode):
 
 @pytest.mark.parametrize("electrode", [False, True])
 def test_solves_around_a_gradient_are_the_same(ctx, electrode):
-    """A field keeps what its gradients set up and queue apart from its own
-    solves: the same charge gives the same bits and counts before and after."""
+    """What a gradient or a tighter solve leaves behind may change how many
+    passes the next solve queues, not what it gives: the same charge gives the
+    same bits and counts before and after."""
     fields, group = small_run(ctx, electrode=electrode)
     rng = np.random.default_rng(5)
     rho = rng.normal(size=group.size) * 1e-18
